@@ -4,6 +4,8 @@
 //   predictor_kernel  : spaceTimePredictorNonlinear.cpph (Picard loop :39-433,
 //                       time averaging :441-515, extrapolation :517-687) fused with
 //                       volumeIntegralNonlinear.cpph (time-averaged branch :133-223)
+//                       for a PDE with source / non-conservative terms; the
+//                       conservative PDEs run predictor_columns.h
 //   riemann_kernel    : riemannSolverNonlinear.cpph:37-128 + RiemannSolverUtils.h:152-177
 //   corrector_kernel  : faceIntegralNonlinear.cpph:21-103 (faces 0..2D-1 in order,
 //                       ADERDGSolver.cpp:1207-1221) + solutionUpdate.cpph:28-67 +
@@ -16,8 +18,8 @@
 //     Per time slice the node's flux is evaluated in registers and published
 //     to a double-buffered LDS slab; each thread then reads the B-point lines
 //     through its node along x/y/z (stiffness contraction), so the only LDS
-//     traffic is the flux slab.  lQi/rhs/lFi never touch HBM: per cell-step
-//     the kernel reads luh once and writes lduh, lQhbnd, lFhbnd once.
+//     traffic is the flux and state slab.  lQi/rhs/lFi never touch HBM: per
+//     cell-step the kernel reads luh once and writes lduh, lQhbnd, lFhbnd once.
 //   * Riemann: one wavefront per face, lanes over face nodes; the face
 //     averages are wave reductions (DPP shuffles).
 //   * corrector: thread per (cell, node); the per-cell CFL minimum is reduced
@@ -25,9 +27,6 @@
 //     bit pattern (exact and order independent for positive doubles), into
 //     the instance's dt_next or, on the uniform mesh, into one of 1024 slots
 //     on separate cache lines that dt_reduce_kernel merges afterwards.
-//   * CERK initial guess (optimised-kernel dialect, or chosen per context):
-//     two flux divergences through the flux slab before the Picard loop
-//     (predictor_tile<..., CG = true>).
 #include <hip/hip_runtime.h>
 
 #include <cfloat>
@@ -57,24 +56,9 @@ struct Shape {
 };
 
 template <typename R>
-__device__ __forceinline__ R tabK(const DevTables* T, int i);
-template <>
-__device__ __forceinline__ double tabK<double>(const DevTables* T, int i) { return T->Kxi[i]; }
-template <>
-__device__ __forceinline__ float tabK<float>(const DevTables* T, int i) { return T->Kxif[i]; }
+__device__ __forceinline__ R tabI(const DevTables* T, int i) { return T->iK1[i]; }
 template <typename R>
-__device__ __forceinline__ R tabI(const DevTables* T, int i);
-template <>
-__device__ __forceinline__ double tabI<double>(const DevTables* T, int i) { return T->iK1[i]; }
-template <>
-__device__ __forceinline__ float tabI<float>(const DevTables* T, int i) { return T->iK1f[i]; }
-
-template <typename R>
-__device__ __forceinline__ R tabD(const DevTables* T, int i);
-template <>
-__device__ __forceinline__ double tabD<double>(const DevTables* T, int i) { return T->dudx[i]; }
-template <>
-__device__ __forceinline__ float tabD<float>(const DevTables* T, int i) { return T->dudxf[i]; }
+__device__ __forceinline__ R tabD(const DevTables* T, int i) { return T->dudx[i]; }
 
 // Coordinates (z, y, x) of spatial node s; z = 0 in 2D.
 template <int D, int B>
@@ -116,7 +100,7 @@ __device__ __forceinline__ int stride_of(int d) {
 // z contributions) and extrapolation (spaceTimePredictorNonlinear.cpph:517-687)
 // of node s of one cell from its time averages in LDS: Qh [node][ND], Fh
 // [d][node][V] (FP64).  du_add (nullable): W-weighted extra term of the node
-// (the time-averaged source).  Shared by the node-column and slab predictors.
+// (the time-averaged source).
 template <int D, int B, int V, int NP>
 __device__ __forceinline__ void node_volume_and_faces(
     const double* Qh, const double* Fh, int s, long cell, const double (&ta)[D], const double (&tb)[D],
@@ -255,15 +239,6 @@ __device__ __forceinline__ void node_volume_and_faces(
   if (s == 0 && picard) picard[cell] = iters;
 }
 
-// The 3D Euler flux has 12 distinct components: the mass fluxes are the
-// momenta (slots 0-2), the momentum fluxes are symmetric (diagonal 3-5,
-// xy, xz, yz 6-8), the energy fluxes 9-11.  euler_slot(d, v) = slot of F_d[v];
-// the first occurrence (d smallest) of a slot is its canonical component.
-__host__ __device__ constexpr int euler_slot(int d, int v) {
-  return v == 0 ? d : (v == 4 ? 9 + d : (v == d + 1 ? 3 + d : 4 + d + v));
-}
-__host__ __device__ constexpr bool euler_canonical(int d, int v) { return !(v >= 1 && v <= 3 && v < d + 1); }
-
 // Node weight W (reference: w[z] w[y] w[x], 2D w[y] w[x]), the two transverse
 // weights per direction in the reference's multiplication order, the node's
 // coordinate along d and the first node of its line along d.
@@ -288,45 +263,35 @@ __device__ __forceinline__ void node_geometry(int s, const double* w, double& W,
 }
 
 // ---------------------------------------------------------------------------
-// Space-time predictor + volume integral
+// Space-time predictor + volume integral of a PDE with a source and / or a
+// non-conservative product (the conservative PDEs: predictor_columns.h)
 // ---------------------------------------------------------------------------
-// One tile (CPB cells) of the predictor; called by predictor_kernel for
-// tile blk.  Threads of invalid cells return at the end, after the last
-// barrier of the tile.
-//
-// NCS: the PDE has a source and / or a non-conservative product
-// (spaceTimePredictorNonlinear.cpph:104-176, 323-367): per time slice the
-// node also publishes its state, reads the B-point lines through it for
-// gradQ = dudx lQi / dx, adds w_t W dt (S - B(Q) gradQ) to its rhs and
-// accumulates the time-averaged S, which the volume integral adds as W lShi
+// One tile (CPB cells); threads of invalid cells return at the end, after the
+// last barrier of the tile.  Per time slice the node publishes its flux and its
+// state, reads the B-point lines through it for the stiffness terms and for
+// gradQ = dudx lQi / dx, adds w_t W dt (S - B(Q) gradQ) to its rhs
+// (spaceTimePredictorNonlinear.cpph:104-176, 323-367) and accumulates the
+// time-averaged S, which the volume integral adds as W lShi
 // (volumeIntegralNonlinear.cpph:204-222).
-template <int D, int B, int V, int NP, typename R, bool CG, bool NCS = false, bool EUS = false>
+template <int D, int B, int V, int NP>
 __device__ __forceinline__ void predictor_tile(
     long blk, long ncells, const double* luh, const double* __restrict__ hcell,
     const double* __restrict__ dtp, const int* __restrict__ cinst, double* __restrict__ lduh,
     double* __restrict__ lQhbnd, double* __restrict__ lFhbnd, int* __restrict__ picard,
     const DevTables* __restrict__ T, PdeParams P, int maxIter, int adaptive, double* luh_upd, int dialect,
     int hdim) {
+  using R = double;
   using S = Shape<D, B, V, NP>;
   constexpr int ND = S::ND, NS = S::NS, CPB = S::CPB, NSP = S::NSP, THREADS_ = S::THREADS;
-  static_assert(!NCS || V == kUserNVar, "user PDE hooks: the user PDE's variables");
+  static_assert(V == kUserNVar, "user PDE hooks: the user PDE's variables");
   static_assert(CPB > 1 || THREADS_ / 64 <= CPB * NSP, "wave sums fit in red");
-  // EUS (3D Euler, FP64): a slab holds the 12 distinct flux components per
-  // node, in slot order, and the time-averaged flux accumulates the canonical
-  // ones in registers (the reference's F_y[1] = rho^-1 q_y q_x, F_z[1], F_z[2]
-  // are taken from F_x[2], F_x[3], F_y[3]: the same products in another order)
-  static_assert(!EUS || (D == 3 && V == 5 && !NCS), "Euler flux slots: 3D, five variables");
-  // slab values per node (EUS: 12 slots padded to 13, an odd stride in doubles,
-  // so that the nodes a wave reads spread over the LDS banks)
-  constexpr int SW = EUS ? 13 : D * V;
-  constexpr int SLAB = NS * SW + (NCS ? NS * V : 0);  // one flux (+ state) slab, per cell
+  constexpr int SW = D * V;
+  constexpr int SLAB = NS * SW + NS * V;  // one flux + state slab, per cell
   constexpr int SLAB_BYTES = 2 * CPB * SLAB * int(sizeof(R));
   constexpr int END_BYTES = CPB * NS * (ND + D * V) * 8;  // time averages, FP64
   constexpr int BUF_BYTES = SLAB_BYTES > END_BYTES ? SLAB_BYTES : END_BYTES;
-  // slab position of F_d[v] of node n; `keep` is false for the flux components
-  // EUS stores once under another (d, v)
-  auto sidx = [](int n, int d, int v) { return EUS ? n * SW + euler_slot(d, v) : (n * D + d) * V + v; };
-  auto keep = [](int d, int v) { return !EUS || euler_canonical(d, v); };
+  // slab position of F_d[v] of node n
+  auto sidx = [](int n, int d, int v) { return (n * D + d) * V + v; };
   __shared__ __align__(16) unsigned char buf[BUF_BYTES];
   __shared__ double red[CPB * NSP];
 
@@ -370,65 +335,9 @@ __device__ __forceinline__ void predictor_tile(
   // Kxi in LDS: a node reads its stiffness column Kxi[n][c_d] per use instead
   // of holding D B entries in registers (they would cost the second wave per SIMD)
   __shared__ R kxs[B * B];
-  if (tid < B * B) kxs[tid] = tabK<R>(T, tid);  // read after the first barrier below
+  if (tid < B * B) kxs[tid] = T->Kxi[tid];  // read after the first barrier below
 
-  // CERK initial guess of the optimised kernels
-  // (KernelGenerator/kernelgenerator/templates/aderdg/fusedSPTVI_nonlinear_cpp.template:121-173,
-  // templates/subtemplates/RK_loop.template:12-40): K1 = sum_d dudx_d F_d(luh) / dx,
-  // lwh = luh - dt K1, K2 = the same of lwh, lQi(t) = luh - dt xi_t K1 - dt xi_t^2 (K2 - K1) / 2
-  if constexpr (CG) {
-    R* slab = reinterpret_cast<R*>(buf) + cslot * SLAB;
-    R K1[V], K2[V], lw[ND];
-#pragma unroll
-    for (int v = 0; v < ND; v++) lw[v] = q[0][v];
-#pragma unroll
-    for (int stage = 0; stage < 2; stage++) {
-      if (valid) {
-        R F[D][V];
-        pde_flux<D, R>(P, lw, F);
-#pragma unroll
-        for (int d = 0; d < D; d++)
-#pragma unroll
-          for (int v = 0; v < V; v++)
-            if (keep(d, v)) slab[sidx(s, d, v)] = F[d][v];
-      }
-      __syncthreads();
-      R K[V];
-#pragma unroll
-      for (int v = 0; v < V; v++) K[v] = R(0);
-      if (valid) {
-#pragma unroll
-        for (int d = 0; d < D; d++)
-#pragma unroll
-          for (int v = 0; v < V; v++) {
-            R a = R(0);
-#pragma unroll
-            for (int n = 0; n < B; n++)
-              a += slab[sidx(base[d] + n * stride_of<D, B>(d), d, v)] *
-                   (static_cast<R>(invDx[d]) * tabD<R>(T, cc[d] * B + n));
-            K[v] += a;
-          }
-      }
-      __syncthreads();  // slab rewritten by the next stage / the Picard loop
-#pragma unroll
-      for (int v = 0; v < V; v++) {
-        if (stage == 0) {
-          K1[v] = K[v];
-          lw[v] = static_cast<R>(u[v]) - static_cast<R>(dt) * K1[v];
-        } else {
-          K2[v] = K[v];
-        }
-      }
-    }
-    const R rdt = static_cast<R>(dt);
-#pragma unroll
-    for (int t = 0; t < B; t++) {
-      const R xt = static_cast<R>(T->x[t]);
-#pragma unroll
-      for (int v = 0; v < V; v++)
-        q[t][v] = static_cast<R>(u[v]) - (rdt * xt * K1[v]) - (R(0.5) * rdt * xt * xt * (K2[v] - K1[v]));
-    }
-  } else if constexpr (NCS) {
+  {
     // trivial guess: hide that the B slices start equal, or the compiler keeps
     // the copies folded and its schedule of the first iteration spills
 #pragma unroll
@@ -437,22 +346,14 @@ __device__ __forceinline__ void predictor_tile(
       for (int v = 0; v < ND; v++) asm volatile("" : "+v"(q[t][v]));
   }
 
-  // time-averaged flux of the last executed iteration: in registers, or (FH_LDS,
-  // FP64 3D order 5, trivial guess) in LDS [d][node][v], where its 30 registers
-  // would cost spills at two waves per SIMD (64.6 -> 60.0 ms at 81^3; the CERK
-  // form does not spill and is faster with registers); same operations
-  constexpr bool FH_LDS = sizeof(R) == 8 && D == 3 && B == 6 && CPB == 1 && !NCS && !CG && !EUS;
-  __shared__ double fhs[FH_LDS ? D * NS * V : 1];
-  [[maybe_unused]] R fh[FH_LDS ? 1 : D][V];
-  [[maybe_unused]] R sh[V];  // NCS: time-averaged source - ncp of the last executed iteration
+  R fh[D][V];  // time-averaged flux of the last executed iteration
+  R sh[V];     // time-averaged source - ncp of the last executed iteration
 #pragma unroll
-  for (int d = 0; d < (FH_LDS ? 1 : D); d++)
+  for (int d = 0; d < D; d++)
 #pragma unroll
     for (int v = 0; v < V; v++) fh[d][v] = R(0);
-  if constexpr (NCS) {
 #pragma unroll
-    for (int v = 0; v < V; v++) sh[v] = R(0);
-  }
+  for (int v = 0; v < V; v++) sh[v] = R(0);
   bool active = valid;
   int iters = maxIter;
 
@@ -510,86 +411,13 @@ __device__ __forceinline__ void predictor_tile(
   R cd[D];
 #pragma unroll
   for (int d = 0; d < D; d++) cd[d] = static_cast<R>(ta[d] * tb[d] * dt * invDx[d] * iweight);
-  int first = 0;
-  if constexpr (!CG && !NCS) {
-    // Trivial guess: the B time slices of the first iterate all equal luh, so
-    // iteration 0 forms their flux, its time average and the stiffness sum once:
-    // rhs[t] = W F0[t] luh - w[t] sum_d sum_n (ta tb dt / dx)_d Kxi[n][c_d] F_d(luh).
-    // Its squared update is taken against luh, so the B copies of luh are never held.
-    if (maxIter > 0) {
-      R acc[B][V];  // time slice 0 assigns, the others accumulate (active lanes only)
-      R* slab = reinterpret_cast<R*>(buf) + cslot * SLAB;
-      if (active) {
-        R F[D][V];
-        pde_flux<D, R>(P, q[0], F);
-#pragma unroll
-        for (int d = 0; d < D; d++)
-#pragma unroll
-          for (int v = 0; v < V; v++) {
-            R a = R(0);
-#pragma unroll
-            for (int t = 0; t < B; t++) a += F[d][v] * static_cast<R>(w[t]);
-            if constexpr (FH_LDS)
-              fhs[(d * NS + s) * V + v] = a;
-            else if (keep(d, v))
-              fh[d][v] = a;
-            if (keep(d, v)) slab[sidx(s, d, v)] = F[d][v];
-          }
-      }
-      __syncthreads();
-      double sq = 0.0;
-      if (active) {
-        R g[V];
-#pragma unroll
-        for (int v = 0; v < V; v++) g[v] = R(0);
-#pragma unroll
-        for (int d = 0; d < D; d++) {
-          const R upd = cd[d];
-#pragma unroll
-          for (int n = 0; n < B; n++) {
-            const R ukc = upd * kxs[n * B + cc[d]];
-#pragma unroll
-            for (int v = 0; v < V; v++) g[v] += ukc * slab[sidx(base[d] + n * stride_of<D, B>(d), d, v)];
-          }
-        }
-#pragma unroll
-        for (int t = 0; t < B; t++) {
-          const R rw = static_cast<R>(W * T->F0[t] * iweight);
-          const R wt = static_cast<R>(w[t]);
-#pragma unroll
-          for (int v = 0; v < V; v++) {
-            const R r = rw * static_cast<R>(u[v]) - wt * g[v];
-#pragma unroll
-            for (int tp = 0; tp < B; tp++) {
-              if (t == 0)
-                acc[tp][v] = r * tabI<R>(T, tp * B + t);
-              else
-                acc[tp][v] += r * tabI<R>(T, tp * B + t);
-            }
-          }
-        }
-#pragma unroll
-        for (int t = 0; t < B; t++)
-#pragma unroll
-          for (int v = 0; v < V; v++) {
-            const double dq = static_cast<double>(acc[t][v]) - static_cast<double>(static_cast<R>(u[v]));
-            sq += dq * dq;
-            q[t][v] = acc[t][v];
-          }
-      }
-      first = finished(0, sq) ? maxIter : 1;
-    }
-  }
-
-  for (int iter = first; iter < maxIter; iter++) {
+  for (int iter = 0; iter < maxIter; iter++) {
     // the new iterate and the time-averaged flux of this iteration: time slice 0
     // assigns, the others accumulate (active lanes only)
     R acc[B][V];
-    if constexpr (NCS) {
-      if (active) {
+    if (active) {
 #pragma unroll
-        for (int v = 0; v < V; v++) sh[v] = R(0);
-      }
+      for (int v = 0; v < V; v++) sh[v] = R(0);
     }
 
 #pragma unroll
@@ -603,23 +431,14 @@ __device__ __forceinline__ void predictor_tile(
         for (int d = 0; d < D; d++)
 #pragma unroll
           for (int v = 0; v < V; v++) {
-            if constexpr (FH_LDS) {
-              if (t == 0)
-                fhs[(d * NS + s) * V + v] = F[d][v] * wt;  // own node: no other lane touches it
-              else
-                fhs[(d * NS + s) * V + v] += F[d][v] * wt;
-            } else if (keep(d, v)) {
-              if (t == 0)
-                fh[d][v] = F[d][v] * wt;
-              else
-                fh[d][v] += F[d][v] * wt;
-            }
-            if (keep(d, v)) slab[sidx(s, d, v)] = F[d][v];
+            if (t == 0)
+              fh[d][v] = F[d][v] * wt;
+            else
+              fh[d][v] += F[d][v] * wt;
+            slab[sidx(s, d, v)] = F[d][v];
           }
-        if constexpr (NCS) {
 #pragma unroll
-          for (int v = 0; v < V; v++) slab[NS * SW + s * V + v] = q[t][v];
-        }
+        for (int v = 0; v < V; v++) slab[NS * SW + s * V + v] = q[t][v];
       }
       __syncthreads();
       if (active) {
@@ -643,7 +462,7 @@ __device__ __forceinline__ void predictor_tile(
             }
           }
         }
-        if constexpr (NCS) {
+        {
           // gradQ of time slice t (:113-176), then rhs += w_t W dt (S - ncp) (:323-367)
           const R* qs = slab + NS * SW;
           R gq[D][V];
@@ -697,7 +516,7 @@ __device__ __forceinline__ void predictor_tile(
 
   // ---- time averages -> LDS (FP64) ----
   double* Qh = reinterpret_cast<double*>(buf) + cslot * NS * (ND + D * V);
-  double* Fh = FH_LDS ? fhs : Qh + NS * ND;  // [d][node][v]
+  double* Fh = Qh + NS * ND;  // [d][node][v]
   __syncthreads();  // slabs no longer read
   if (valid) {
 #pragma unroll
@@ -707,26 +526,15 @@ __device__ __forceinline__ void predictor_tile(
       for (int t = 0; t < B; t++) a += static_cast<double>(q[t][v]) * w[t];
       Qh[s * ND + v] = a;
     }
-    if constexpr (!FH_LDS) {
 #pragma unroll
-      for (int d = 0; d < D; d++)
+    for (int d = 0; d < D; d++)
 #pragma unroll
-        for (int v = 0; v < V; v++) {
-          // EUS: the component stored once is read from its canonical (d, v)
-          const int dd = keep(d, v) ? d : v - 1, vv = keep(d, v) ? v : d + 1;
-          Fh[(d * NS + s) * V + v] = static_cast<double>(fh[dd][vv]);
-        }
-    }
+      for (int v = 0; v < V; v++) Fh[(d * NS + s) * V + v] = fh[d][v];
   }
   __syncthreads();
   if (!valid) return;
 
   // ---- volume integral and extrapolation ----
-  double shd[V];
-  if constexpr (NCS) {
-#pragma unroll
-    for (int v = 0; v < V; v++) shd[v] = static_cast<double>(sh[v]);
-  }
   // the per-node constants again, from a node index the optimiser cannot
   // equate with s: the loop's copies end with the loop instead of being held
   // (spilled at two waves per SIMD) across it
@@ -739,37 +547,19 @@ __device__ __forceinline__ void predictor_tile(
   for (int d = 0; d < D; d++) invDx2[d] = 1.0 / hcell[hdim ? cell * hdim + d : cell];
   const double dt2 = dtp[cinst ? cinst[cell] : 0];
   node_volume_and_faces<D, B, V, NP>(Qh, Fh, s2, cell, ta2, tb2, cc2, base2, invDx2, W2, dt2, iters,
-                                     NCS ? shd : nullptr, T, lduh, lQhbnd, lFhbnd, picard, luh_upd);
+                                     sh, T, lduh, lQhbnd, lFhbnd, picard, luh_upd);
 }
 
-// Predictor + volume integral, one workgroup per tile of CPB cells.  Two
-// waves per SIMD (at most 256 registers per lane) for the conservative forms;
-// the source / NCP form keeps the extra state of its gradient and source terms
-// and runs at one.
-template <int D, int B, int V, int NP, typename R, bool CG, bool NCS = false, bool EUS = false>
-__global__ __launch_bounds__((Shape<D, B, V, NP>::THREADS), NCS ? 1 : 2) void predictor_kernel(
-    long ncells, long ntiles, const double* luh, const double* __restrict__ hcell,
-    const double* __restrict__ dtp, const int* __restrict__ cinst, double* __restrict__ lduh,
-    double* __restrict__ lQhbnd, double* __restrict__ lFhbnd, int* __restrict__ picard,
-    const DevTables* __restrict__ T, PdeParams P, int maxIter, int adaptive, double* luh_upd, int dialect,
-    int hdim) {
-  predictor_tile<D, B, V, NP, R, CG, NCS, EUS>(blockIdx.x, ncells, luh, hcell, dtp, cinst, lduh, lQhbnd, lFhbnd,
-                                               picard, T, P, maxIter, adaptive, luh_upd, dialect, hdim);
-}
-
-// Persistent form: a grid smaller than ntiles loops over the tiles.
-template <int D, int B, int V, int NP, typename R, bool CG, bool EUS = false>
-__global__ __launch_bounds__((Shape<D, B, V, NP>::THREADS), 2) void predictor_persistent_kernel(
-    long ncells, long ntiles, const double* luh, const double* __restrict__ hcell,
-    const double* __restrict__ dtp, const int* __restrict__ cinst, double* __restrict__ lduh,
-    double* __restrict__ lQhbnd, double* __restrict__ lFhbnd, int* __restrict__ picard,
-    const DevTables* __restrict__ T, PdeParams P, int maxIter, int adaptive, double* luh_upd, int dialect,
-    int hdim) {
-  for (long blk = blockIdx.x; blk < ntiles; blk += gridDim.x) {
-    predictor_tile<D, B, V, NP, R, CG, false, EUS>(blk, ncells, luh, hcell, dtp, cinst, lduh, lQhbnd, lFhbnd,
-                                                   picard, T, P, maxIter, adaptive, luh_upd, dialect, hdim);
-    __syncthreads();  // LDS of this tile fully consumed before the next one
-  }
+// One workgroup per tile of CPB cells; one wave per SIMD: the extra state of the
+// gradient and source terms.
+template <int D, int B, int V, int NP>
+__global__ __launch_bounds__((Shape<D, B, V, NP>::THREADS), 1) void predictor_kernel(
+    long ncells, const double* luh, const double* __restrict__ hcell, const double* __restrict__ dtp,
+    const int* __restrict__ cinst, double* __restrict__ lduh, double* __restrict__ lQhbnd,
+    double* __restrict__ lFhbnd, int* __restrict__ picard, const DevTables* __restrict__ T, PdeParams P, int maxIter,
+    int adaptive, double* luh_upd, int dialect, int hdim) {
+  predictor_tile<D, B, V, NP>(blockIdx.x, ncells, luh, hcell, dtp, cinst, lduh, lQhbnd, lFhbnd, picard, T, P, maxIter,
+                              adaptive, luh_upd, dialect, hdim);
 }
 
 // ---------------------------------------------------------------------------
@@ -1403,70 +1193,22 @@ struct Launch {
   static long grid_of(long tiles, const LaunchOpts& o) { return (o.grid > 0 && o.grid < tiles) ? o.grid : tiles; }
   static int predictor(const KernelCfg& k, hipStream_t st, long n, const double* luh, const double* h,
                        const double* dt, double* lduh, double* qb, double* fb, int* pic, const LaunchOpts& o) {
-    const long tiles = (n + S::CPB - 1) / S::CPB;
-    const long grid = grid_of(tiles, o);
-    // Picard rule: generic (adaptive or fixed count) or the optimised kernels'
-    // (fusedSPTVI_nonlinear_cpp.template:177, tolerance exit always on)
-    const int adaptive = k.dialect ? 1 : k.picard_max <= 0;
-    const int maxIter = k.dialect ? (k.guess ? (B - 3 <= 1 ? 1 : B - 3) : 2 * B + 1)
-                                  : (adaptive ? 2 * (k.order + 1) : k.picard_max);
-    const int dl = k.dialect;
-    const bool cerk = k.guess != 0;
-    // the CERK form is compiled without the persistent variant (one workgroup per tile)
-    const bool persistent = grid < tiles && !cerk;
     if (pde_has_ncs(k.pde)) {
-      // source / non-conservative terms: FP64, trivial guess, one workgroup per tile, 5 variables
+      // source / non-conservative terms: FP64, trivial guess, one workgroup per tile
       if constexpr (V == kUserNVar && NP == 0) {
-        if (k.precision != 0 || cerk) return -1;
-        hipLaunchKernelGGL((predictor_kernel<D, B, V, NP, double, false, true>), dim3(tiles), dim3(S::THREADS), 0,
-                           st, n, tiles, luh, h, dt, o.cinst, lduh, qb, fb, pic, k.tab, k.pde, maxIter, adaptive,
-                           o.luh_update, dl, o.hdim);
+        if (k.precision != 0 || k.guess) return -1;
+        const long tiles = (n + S::CPB - 1) / S::CPB;
+        const int adaptive = k.dialect ? 1 : k.picard_max <= 0;
+        const int maxIter = k.dialect ? 2 * B + 1 : (adaptive ? 2 * (k.order + 1) : k.picard_max);
+        hipLaunchKernelGGL((predictor_kernel<D, B, V, NP>), dim3(tiles), dim3(S::THREADS), 0, st, n, luh, h, dt, o.cinst,
+                           lduh, qb, fb, pic, k.tab, k.pde, maxIter, adaptive, o.luh_update, k.dialect, o.hdim);
         return static_cast<int>(hipGetLastError());
       } else {
         return -1;
       }
     }
-    if (k.precision == 0)
-      launch_predictor_form<double>(st, cerk, persistent, grid, tiles, n, luh, h, dt, lduh, qb, fb, pic, k,
-                                    maxIter, adaptive, o, dl);
-    else
-      launch_predictor_form<float>(st, cerk, persistent, grid, tiles, n, luh, h, dt, lduh, qb, fb, pic, k,
-                                   maxIter, adaptive, o, dl);
-    return static_cast<int>(hipGetLastError());
-  }
-  template <typename R>
-  static void launch_predictor_form(hipStream_t st, bool cerk, bool persistent, long grid, long tiles, long n,
-                                    const double* luh, const double* h, const double* dt, double* lduh, double* qb,
-                                    double* fb, int* pic, const KernelCfg& k, int maxIter, int adaptive,
-                                    const LaunchOpts& o, int dl) {
-    // 3D Euler of orders 4 and 5 in FP64: the slab of the 12 distinct flux components
-    if constexpr (D == 3 && (B == 5 || B == 6) && V == 5 && NP == 0 && sizeof(R) == 8) {
-      if (k.pde.id == kPdeEuler) {
-        if (persistent)
-          hipLaunchKernelGGL((predictor_persistent_kernel<D, B, V, NP, R, false, true>), dim3(grid),
-                             dim3(S::THREADS), 0, st, n, tiles, luh, h, dt, o.cinst, lduh, qb, fb, pic, k.tab, k.pde,
-                             maxIter, adaptive, o.luh_update, dl, o.hdim);
-        else if (cerk)
-          hipLaunchKernelGGL((predictor_kernel<D, B, V, NP, R, true, false, true>), dim3(tiles), dim3(S::THREADS), 0,
-                             st, n, tiles, luh, h, dt, o.cinst, lduh, qb, fb, pic, k.tab, k.pde, maxIter, adaptive,
-                             o.luh_update, dl, o.hdim);
-        else
-          hipLaunchKernelGGL((predictor_kernel<D, B, V, NP, R, false, false, true>), dim3(tiles), dim3(S::THREADS), 0,
-                             st, n, tiles, luh, h, dt, o.cinst, lduh, qb, fb, pic, k.tab, k.pde, maxIter, adaptive,
-                             o.luh_update, dl, o.hdim);
-        return;
-      }
-    }
-    if (cerk)
-      hipLaunchKernelGGL((predictor_kernel<D, B, V, NP, R, true>), dim3(tiles), dim3(S::THREADS), 0, st, n, tiles,
-                         luh, h, dt, o.cinst, lduh, qb, fb, pic, k.tab, k.pde, maxIter, adaptive, o.luh_update, dl, o.hdim);
-    else if (persistent)
-      hipLaunchKernelGGL((predictor_persistent_kernel<D, B, V, NP, R, false>), dim3(grid), dim3(S::THREADS), 0, st,
-                         n, tiles, luh, h, dt, o.cinst, lduh, qb, fb, pic, k.tab, k.pde, maxIter, adaptive,
-                         o.luh_update, dl, o.hdim);
-    else
-      hipLaunchKernelGGL((predictor_kernel<D, B, V, NP, R, false>), dim3(tiles), dim3(S::THREADS), 0, st, n, tiles,
-                         luh, h, dt, o.cinst, lduh, qb, fb, pic, k.tab, k.pde, maxIter, adaptive, o.luh_update, dl, o.hdim);
+    return D == 3 ? launch_predictor_columns_3d(k, st, n, luh, h, dt, lduh, qb, fb, pic, o)
+                  : launch_predictor_columns_2d(k, st, n, luh, h, dt, lduh, qb, fb, pic, o);
   }
   static int riemann(const KernelCfg& k, hipStream_t st, long nf, const int* faces, const double* qb,
                      double* fb, const LaunchOpts& o) {

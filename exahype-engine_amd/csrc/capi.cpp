@@ -157,6 +157,22 @@ void convert_rows(const double* in, double* out, long rows, int n, int ld_in, in
     for (int v = 0; v < n; v++) out[r * ld_out + v] = in[r * ld_in + v];
 }
 
+// The halves of an operator with M[B-1-i][B-1-j] = -M[i][j] (DevTables::dudx_eo).
+void fill_even_odd(const double* M, int B, double* out) {
+  const int H = B / 2;
+  for (int i = 0; i < H; i++)
+    for (int j = 0; j < H; j++) {
+      const double a = M[i * B + j], b = M[i * B + B - 1 - j];
+      out[i * H + j] = 0.5 * (a - b);
+      out[H * H + i * H + j] = 0.5 * (a + b);
+    }
+  if (B % 2)
+    for (int i = 0; i < H; i++) {
+      out[2 * H * H + i] = M[i * B + H];
+      out[2 * H * H + H + i] = M[H * B + i];
+    }
+}
+
 double lagrange(const double* x, int B, int k, double s) {
   double r = 1.0;
   for (int m = 0; m < B; m++)
@@ -349,6 +365,9 @@ int exa_ctx_create(exa_ctx** out, int dim, int order, int nvar, int npar, int pd
   }
   for (int k = 0; k < 3; k++) h.cmom[k] = static_cast<float>(cm[k]);
   for (int i = 0; i < 3 * B * B; i++) h.fgp[i] = c->tab.fgp[i];
+  fill_even_odd(c->tab.dudx, B, h.dudx_eo);
+  fill_even_odd(c->tab.Kxi, B, h.Kxi_eo);
+  for (int i = 0; i < exa::kEvenOdd; i++) h.dudx_eof[i] = static_cast<float>(h.dudx_eo[i]);
   hipError_t e = hipMalloc(&c->d_tab, sizeof(exa::DevTables));
   if (e == hipSuccess) e = hipMemcpy(c->d_tab, &h, sizeof(h), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);

@@ -11,6 +11,8 @@
 
 namespace exa {
 
+constexpr int kEvenOdd = kMaxBasis * kMaxBasis / 2;  // covers 2 H^2 + 2 H for every B <= kMaxBasis
+
 // Operator tables as stored on the device (one block per context).
 struct DevTables {
   double w[kMaxBasis];
@@ -34,6 +36,11 @@ struct DevTables {
   float cmom[3];         // sum_j c[j] x[j]^k, k = 0, 1, 2 (c-weighted time moments)
   double fgp[3 * kMaxBasis * kMaxBasis];  // fineGridProjector[sub][n][m] = phi_n((sub + x_m) / 3), [(sub*B+n)*B+m]
   double iw[kMaxBasis];                   // 1 / w[i]
+  // dudx and Kxi by halves for the even-odd line contraction (H = B / 2, mirror j' = B-1-j):
+  // (M[i][j] - M[i][j']) / 2 [H][H], (M[i][j] + M[i][j']) / 2 [H][H], odd B: M[i][H] [H], M[H][j] [H]
+  double dudx_eo[kEvenOdd];
+  float dudx_eof[kEvenOdd];
+  double Kxi_eo[kEvenOdd];
 };
 
 struct KernelCfg {
@@ -143,6 +150,14 @@ int launch_face_integral(const KernelCfg& k, hipStream_t s, double* lduh, const 
                          int orientation, double invdx_scaled);
 int launch_solution_update(const KernelCfg& k, hipStream_t s, double* luh, const double* luhOld,
                            const double* lduh, const double* dt);
+// Column / line predictor (predictor_columns.h), every compiled shape of the
+// conservative PDEs; -1 for a shape that is not compiled.
+int launch_predictor_columns_2d(const KernelCfg& k, hipStream_t s, long ncells, const double* luh, const double* h,
+                                const double* dt, double* lduh, double* lQhbnd, double* lFhbnd, int* picard,
+                                const LaunchOpts& o);
+int launch_predictor_columns_3d(const KernelCfg& k, hipStream_t s, long ncells, const double* luh, const double* h,
+                                const double* dt, double* lduh, double* lQhbnd, double* lFhbnd, int* picard,
+                                const LaunchOpts& o);
 // Line-decomposed 3D predictor (predictor3d_lines.hip) for the shapes it covers.
 bool lines_supported(const KernelCfg& k);
 // The 3D order-5 line/tile predictors serve k: generic Picard rule, and with the
