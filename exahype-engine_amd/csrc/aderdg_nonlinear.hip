@@ -20,8 +20,8 @@
 //     through its node along x/y/z (stiffness contraction), so the only LDS
 //     traffic is the flux and state slab.  lQi/rhs/lFi never touch HBM: per
 //     cell-step the kernel reads luh once and writes lduh, lQhbnd, lFhbnd once.
-//   * Riemann: one wavefront per face, lanes over face nodes; the face
-//     averages are wave reductions (DPP shuffles).
+//   * Riemann: a power-of-two group of lanes per face, lanes over face nodes;
+//     the face averages are lane reductions in the group.
 //   * corrector: thread per (cell, node); the per-cell CFL minimum is reduced
 //     in LDS and merged with one 64-bit atomicMin per workgroup on the IEEE
 //     bit pattern (exact and order independent for positive doubles), into
@@ -563,11 +563,21 @@ __global__ __launch_bounds__((Shape<D, B, V, NP>::THREADS), 1) void predictor_ke
 }
 
 // ---------------------------------------------------------------------------
-// Rusanov flux, one wavefront per face
+// Rusanov flux, a power-of-two group of lanes per face
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ double wave_sum(double v) {
+// Lanes per face: the face nodes rounded up to a power of two, so that a
+// wavefront takes 64 / kFaceLanes faces (2D order 3: sixteen of four nodes
+// where one wavefront per face leaves 60 lanes idle; 3D order 4: two).  25,000
+// cells of 2D order 4: 66 -> 23 us; 12,167 shuffled cells of 3D order 4, bound
+// by their 220 MB: 66 us either way.
+template <int NF>
+constexpr int kFaceLanes = NF >= 64 ? 64 : next_pow2(NF);
+
+// Sum over a group of G lanes (every lane of the group ends with the same bits).
+template <int G>
+__device__ __forceinline__ double group_sum(double v) {
 #pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
+  for (int m = G / 2; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
   return v;
 }
 
@@ -581,10 +591,10 @@ __global__ __launch_bounds__(256) void riemann_kernel(long nfaces, const int4* _
                                                       double* __restrict__ gf, const DevTables* __restrict__ T,
                                                       PdeParams P) {
   using S = Shape<D, B, V, NP>;
-  constexpr int ND = S::ND, NF = S::NF;
-  const int lane = threadIdx.x & 63;
-  const long f = (long)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  if (f >= nfaces) return;  // uniform per wavefront; no block barriers below
+  constexpr int ND = S::ND, NF = S::NF, G = kFaceLanes<NF>;
+  const int lane = threadIdx.x & (G - 1);
+  const long f = (long)blockIdx.x * (blockDim.x / G) + threadIdx.x / G;
+  if (f >= nfaces) return;  // uniform per group of G lanes; the sums stay in the group, no block barriers below
   const int4 fc = faces[f];
   const int d = fc.z;
   const bool gl = gq && (fc.w & 2) != 0, gr = gq && (fc.w & 1) != 0;  // w is ignored without ghost faces
@@ -596,7 +606,7 @@ __global__ __launch_bounds__(256) void riemann_kernel(long nfaces, const int4* _
   double aL[ND], aR[ND];
 #pragma unroll
   for (int k = 0; k < ND; k++) aL[k] = aR[k] = 0.0;
-  for (int j = lane; j < NF; j += 64) {
+  for (int j = lane; j < NF; j += G) {
     const double wj = (D == 3) ? w[j / B] * w[j % B] : w[j];
 #pragma unroll
     for (int k = 0; k < ND; k++) {
@@ -606,15 +616,15 @@ __global__ __launch_bounds__(256) void riemann_kernel(long nfaces, const int4* _
   }
 #pragma unroll
   for (int k = 0; k < ND; k++) {
-    aL[k] = wave_sum(aL[k]);
-    aR[k] = wave_sum(aR[k]);
+    aL[k] = group_sum<G>(aL[k]);
+    aR[k] = group_sum<G>(aR[k]);
   }
   const double smax = fmax(pde_max_abs_eig<D, V>(P, aL, d), pde_max_abs_eig<D, V>(P, aR, d));
   if constexpr (V == kUserNVar) {
     if (pde_has_ncp(P)) {
       // fluctuations (riemannSolverNonlinear.cpph:95-120): the NCP of the node
       // average with gradQ[d] = QR - QL; FR = F - ncp/2, FL = F + ncp/2
-      for (int j = lane; j < NF; j += 64) {
+      for (int j = lane; j < NF; j += G) {
         double gq[D][V], qa[V], ncp[V];
 #pragma unroll
         for (int e = 0; e < D; e++)
@@ -638,7 +648,7 @@ __global__ __launch_bounds__(256) void riemann_kernel(long nfaces, const int4* _
       return;
     }
   }
-  for (int j = lane; j < NF; j += 64) {
+  for (int j = lane; j < NF; j += G) {
 #pragma unroll
     for (int k = 0; k < V; k++) {
       const double fl = FL[j * V + k], fr = FR[j * V + k];
@@ -656,6 +666,14 @@ __global__ __launch_bounds__(256) void riemann_kernel(long nfaces, const int4* _
 __device__ __forceinline__ void atomic_min_pos_double(double* addr, double v) {
   // positive IEEE doubles order like their bit patterns
   atomicMin(reinterpret_cast<unsigned long long*>(addr), static_cast<unsigned long long>(__double_as_longlong(v)));
+}
+
+// *addr = min(*addr, v) where many workgroups share the address: atomics on one
+// line are served one after the other (~10 ns each across the XCDs), so a value
+// that the address already undercuts is not sent.  The value only falls during a
+// launch, so a load that is late costs an atomic and loses nothing.
+__device__ __forceinline__ void merge_min(double* addr, double v) {
+  if (v < __hip_atomic_load(addr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomic_min_pos_double(addr, v);
 }
 
 // A node's stable dt is CFL*PNPM / den with den = sum_d max_v |lambda_v(Q, d)| / dx
@@ -725,7 +743,7 @@ __device__ __forceinline__ void corrector_tile(
     long blk, long ncells, double* __restrict__ luh, const double* __restrict__ lduh,
     const double* __restrict__ lFhbnd, const double* __restrict__ hcell, const double* __restrict__ dtp,
     const int* __restrict__ cinst, double* __restrict__ dt_next, const DevTables* __restrict__ T, PdeParams P,
-    double cflpnpm, int do_update, double* sred, double* __restrict__ slots, int hdim) {
+    double cflpnpm, int do_update, double* sred, double* __restrict__ slots, int nslots, int hdim) {
   using S = Shape<D, B, V, NP>;
   constexpr int ND = S::ND, NS = S::NS, NF = S::NF, CPB = S::CPB, THREADS = S::THREADS;
   const int tid = threadIdx.x;
@@ -776,15 +794,27 @@ __device__ __forceinline__ void corrector_tile(
     mydt = node_cfl_dt<D, B, V, NP>(Q, P, invDx, cflpnpm);
   }
   // cells of one instance are contiguous: a tile whose first and last cell
-  // share the instance reduces once, otherwise every cell merges its own dt
+  // share the instance reduces once, otherwise every cell merges its own dt (a
+  // merge per node put 250 atomics of a tile on two cache lines: 25,000 cells of
+  // 32 instances 65 -> 21 us with the slots)
   const long first = blk * CPB, last = (first + CPB - 1 < ncells) ? first + CPB - 1 : ncells - 1;
+  auto merge = [&](int i, double v) {
+    if (slots)
+      atomic_min_pos_double(slots + (long(i) * nslots + blk % nslots) * kDtSlotStride, v);
+    else
+      merge_min(dt_next + i, v);
+  };
   const bool uniform = !cinst || cinst[first] == cinst[last];
   if (uniform) {
     const double bmin = block_min<THREADS>(mydt, sred);
-    double* dst = (slots && !cinst) ? slots + (blk % kDtSlots) * kDtSlotStride : dt_next + (cinst ? cinst[first] : 0);
-    if (tid == 0 && bmin < DBL_MAX) atomic_min_pos_double(dst, bmin);
-  } else if (valid && mydt < DBL_MAX) {
-    atomic_min_pos_double(dt_next + inst, mydt);
+    if (tid == 0 && bmin < DBL_MAX) merge(cinst ? cinst[first] : 0, bmin);
+  } else {
+    sred[tid] = mydt;
+    __syncthreads();
+    if (valid && s == 0) {
+      for (int i = 1; i < NS; i++) mydt = fmin(mydt, sred[tid + i]);
+      if (mydt < DBL_MAX) merge(inst, mydt);
+    }
   }
 }
 
@@ -793,10 +823,10 @@ __global__ __launch_bounds__((Shape<D, B, V, NP>::THREADS)) void corrector_kerne
     long ncells, long ntiles, double* __restrict__ luh, const double* __restrict__ lduh,
     const double* __restrict__ lFhbnd, const double* __restrict__ hcell, const double* __restrict__ dtp,
     const int* __restrict__ cinst, double* __restrict__ dt_next, const DevTables* __restrict__ T, PdeParams P,
-    double cflpnpm, int do_update, double* __restrict__ slots, int hdim) {
-  __shared__ double sred[Shape<D, B, V, NP>::THREADS / 64];
+    double cflpnpm, int do_update, double* __restrict__ slots, int nslots, int hdim) {
+  __shared__ double sred[Shape<D, B, V, NP>::THREADS];  // a wave's minimum each, or a node's
   corrector_tile<D, B, V, NP>(blockIdx.x, ncells, luh, lduh, lFhbnd, hcell, dtp, cinst, dt_next, T, P, cflpnpm,
-                              do_update, sred, slots, hdim);
+                              do_update, sred, slots, nslots, hdim);
 }
 
 template <int D, int B, int V, int NP>
@@ -804,11 +834,11 @@ __global__ __launch_bounds__((Shape<D, B, V, NP>::THREADS)) void corrector_persi
     long ncells, long ntiles, double* __restrict__ luh, const double* __restrict__ lduh,
     const double* __restrict__ lFhbnd, const double* __restrict__ hcell, const double* __restrict__ dtp,
     const int* __restrict__ cinst, double* __restrict__ dt_next, const DevTables* __restrict__ T, PdeParams P,
-    double cflpnpm, int do_update, double* __restrict__ slots, int hdim) {
-  __shared__ double sred[Shape<D, B, V, NP>::THREADS / 64];
+    double cflpnpm, int do_update, double* __restrict__ slots, int nslots, int hdim) {
+  __shared__ double sred[Shape<D, B, V, NP>::THREADS];  // a wave's minimum each, or a node's
   for (long blk = blockIdx.x; blk < ntiles; blk += gridDim.x) {
     corrector_tile<D, B, V, NP>(blk, ncells, luh, lduh, lFhbnd, hcell, dtp, cinst, dt_next, T, P, cflpnpm,
-                                do_update, sred, slots, hdim);
+                                do_update, sred, slots, nslots, hdim);
     __syncthreads();
   }
 }
@@ -1169,12 +1199,24 @@ __global__ void solution_update_kernel(double* __restrict__ luh, const double* _
   for (int v = 0; v < V; v++) luh[s * ND + v] = luhOld[s * ND + v] + lduh[s * V + v] * upd;
 }
 
-// state[i] = {t, dt, dt_next, -} per instance; strided layout: t[ninst], dt[ninst], dt_next[ninst]
-__global__ void advance_time_kernel(double* state, int ninst) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < ninst) {
+// Per instance (one workgroup each), strided layout t[ninst], dt[ninst],
+// dt_next[ninst]: the spread minima merged into dt_next (slots: nullptr without)
+// and reset for the next step, t += dt, dt = dt_next.
+__global__ __launch_bounds__(256) void advance_time_kernel(double* state, int ninst, double* slots, int nslots) {
+  __shared__ double sred[4];
+  const int i = blockIdx.x;
+  double m = DBL_MAX;
+  if (slots) {
+    double* p = slots + long(i) * nslots * kDtSlotStride;
+#pragma unroll 4
+    for (int k = threadIdx.x; k < nslots; k += 256) m = fmin(m, p[k * kDtSlotStride]);
+#pragma unroll 4
+    for (int k = threadIdx.x; k < nslots; k += 256) p[k * kDtSlotStride] = DBL_MAX;
+    m = block_min<256>(m, sred);
+  }
+  if (threadIdx.x == 0) {
     state[i] += state[ninst + i];
-    state[ninst + i] = state[2 * ninst + i];
+    state[ninst + i] = fmin(m, state[2 * ninst + i]);
     state[2 * ninst + i] = DBL_MAX;
   }
 }
@@ -1214,7 +1256,8 @@ struct Launch {
                      double* fb, const LaunchOpts& o) {
     // riemann_kernel is compiled for at most 256 threads (4 waves) per workgroup
     const int waves = (o.riemann_waves >= 1 && o.riemann_waves <= 4) ? o.riemann_waves : 4;
-    const long blocks = (nf + waves - 1) / waves;
+    const long per = waves * (64 / kFaceLanes<S::NF>);  // faces per workgroup
+    const long blocks = (nf + per - 1) / per;
     hipLaunchKernelGGL((riemann_kernel<D, B, V, NP>), dim3(blocks), dim3(64 * waves), 0, st, nf,
                        reinterpret_cast<const int4*>(faces), qb, fb, o.ghost_q, o.ghost_f, k.tab, k.pde);
     return static_cast<int>(hipGetLastError());
@@ -1225,10 +1268,10 @@ struct Launch {
     const long grid = grid_of(tiles, o);
     if (grid < tiles)
       hipLaunchKernelGGL((corrector_persistent_kernel<D, B, V, NP>), dim3(grid), dim3(S::THREADS), 0, st, n, tiles,
-                         luh, lduh, fb, h, dt, o.cinst, dt_next, k.tab, k.pde, k.cfl * k.pnpm, do_update, o.dt_slots, o.hdim);
+                         luh, lduh, fb, h, dt, o.cinst, dt_next, k.tab, k.pde, k.cfl * k.pnpm, do_update, o.dt_slots, o.dt_nslots, o.hdim);
     else
       hipLaunchKernelGGL((corrector_kernel<D, B, V, NP>), dim3(grid), dim3(S::THREADS), 0, st, n, tiles, luh, lduh,
-                         fb, h, dt, o.cinst, dt_next, k.tab, k.pde, k.cfl * k.pnpm, do_update, o.dt_slots, o.hdim);
+                         fb, h, dt, o.cinst, dt_next, k.tab, k.pde, k.cfl * k.pnpm, do_update, o.dt_slots, o.dt_nslots, o.hdim);
     return static_cast<int>(hipGetLastError());
   }
   static int corrector_riemann(const KernelCfg& k, hipStream_t st, long n, int nside, double* luh,
@@ -1426,8 +1469,9 @@ __global__ __launch_bounds__(256) void dt_reduce_kernel(double* slots, double* d
   if (threadIdx.x == 0 && bmin < DBL_MAX) atomic_min_pos_double(dt_next, bmin);
 }
 
-__global__ __launch_bounds__(256) void dt_slots_init_kernel(double* slots) {
-  for (int i = threadIdx.x; i < kDtSlots; i += 256) slots[i * kDtSlotStride] = DBL_MAX;
+__global__ __launch_bounds__(256) void dt_slots_init_kernel(double* slots, long n) {
+  const long i = long(blockIdx.x) * 256 + threadIdx.x;
+  if (i < n) slots[i * kDtSlotStride] = DBL_MAX;
 }
 }  // namespace
 
@@ -1436,13 +1480,14 @@ int launch_dt_reduce(hipStream_t s, double* slots, double* dt_next) {
   return static_cast<int>(hipGetLastError());
 }
 
-int launch_dt_slots_init(hipStream_t s, double* slots) {
-  hipLaunchKernelGGL(dt_slots_init_kernel, dim3(1), dim3(256), 0, s, slots);
+int launch_dt_slots_init(hipStream_t s, double* slots, long n) {
+  if (n <= 0) return 0;
+  hipLaunchKernelGGL(dt_slots_init_kernel, dim3(unsigned((n + 255) / 256)), dim3(256), 0, s, slots, n);
   return static_cast<int>(hipGetLastError());
 }
 
-int launch_advance_time(hipStream_t s, double* state, int ninst) {
-  hipLaunchKernelGGL(advance_time_kernel, dim3((ninst + 255) / 256), dim3(256), 0, s, state, ninst);
+int launch_advance_time(hipStream_t s, double* state, int ninst, double* slots, int nslots) {
+  hipLaunchKernelGGL(advance_time_kernel, dim3(ninst), dim3(256), 0, s, state, ninst, slots, nslots);
   return static_cast<int>(hipGetLastError());
 }
 

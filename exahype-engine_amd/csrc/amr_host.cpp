@@ -132,6 +132,11 @@ struct CellSet {
   hipStream_t stream = nullptr;
   double *d_luh = nullptr, *d_lduh = nullptr, *d_qb = nullptr, *d_fb = nullptr, *d_h = nullptr;
   double* d_state = nullptr;  // t[ninst], dt[ninst], dt_next[ninst]
+  // stable-dt minima of the correctors, [ninst][dt_nslots] cache lines (DBL_MAX
+  // between steps): about a thousand lines in all, at least eight an instance --
+  // on one line an instance the first wave of workgroups queues for its atomics
+  double* d_slots = nullptr;
+  int dt_nslots = 0;
   int* d_cinst = nullptr;
   int* d_picard = nullptr;  // per-cell Picard count of the last step
   int* d_faces = nullptr;
@@ -149,7 +154,7 @@ struct CellSet {
     if (graph) (void)hipGraphDestroy(graph);
     graph_exec = nullptr;
     graph = nullptr;
-    double* b[] = {d_luh, d_lduh, d_qb, d_fb, d_h, d_state};
+    double* b[] = {d_luh, d_lduh, d_qb, d_fb, d_h, d_state, d_slots};
     for (double* p : b)
       if (p) (void)hipFree(p);
     int* ib[] = {d_cinst, d_picard, d_faces, d_prolong, d_restrict};
@@ -176,9 +181,23 @@ struct CellSet {
     std::vector<double> st(3 * ninst, 0.0);
     for (int i = ninst; i < 3 * ninst; i++) st[i] = DBL_MAX;
     HIP_OK(hipMemcpy(d_state, st.data(), sizeof(double) * st.size(), hipMemcpyHostToDevice), "state");
+    dt_nslots = exa::kDtSlots / ninst > 8 ? exa::kDtSlots / ninst : 8;
+    HIP_OK(hipMalloc(&d_slots, sizeof(double) * ninst * dt_nslots * exa::kDtSlotStride), "hipMalloc(slots)");
+    RC_OK(reset_slots());
     HIP_OK(hipMemset(d_qb, 0, sizeof(double) * nslots * 2 * D * NF * ND), "clear");
     HIP_OK(hipMemset(d_fb, 0, sizeof(double) * nslots * 2 * D * NF * V), "clear");
     return EXA_OK;
+  }
+
+  int reset_slots() {
+    return status(exa::launch_dt_slots_init(stream, d_slots, long(ninst) * dt_nslots), "dt slots");
+  }
+
+  exa::LaunchOpts corrector_opts(exa::LaunchOpts o) const {
+    o.cinst = d_cinst;
+    o.dt_slots = d_slots;
+    o.dt_nslots = dt_nslots;
+    return o;
   }
 
   exa::LaunchOpts with_cinst(exa::LaunchOpts o) const {
@@ -196,9 +215,9 @@ struct CellSet {
     if (nprolong) RC_OK(status(exa::launch_face_prolong(k, s, nprolong, d_prolong, d_qb, d_fb), "face prolongation"));
     RC_OK(status(exa::launch_riemann(k, s, nfaces, d_faces, d_qb, d_fb, tune.riem), "riemann"));
     if (nrestrict) RC_OK(status(exa::launch_face_restrict(k, s, nrestrict, d_restrict, d_fb), "face restriction"));
-    RC_OK(status(exa::launch_corrector(k, s, ncells, d_luh, d_lduh, d_fb, d_h, dt, dtn, with_cinst(tune.corr)),
+    RC_OK(status(exa::launch_corrector(k, s, ncells, d_luh, d_lduh, d_fb, d_h, dt, dtn, corrector_opts(tune.corr)),
                  "corrector"));
-    return status(exa::launch_advance_time(s, d_state, ninst), "advance time");
+    return status(exa::launch_advance_time(s, d_state, ninst, d_slots, dt_nslots), "advance time");
   }
 
   int init_dt(double dt) {
@@ -291,7 +310,7 @@ struct CellSet {
     }
     for (long g : grids) {
       if (rc) break;
-      exa::LaunchOpts o = with_cinst(exa::LaunchOpts());
+      exa::LaunchOpts o = corrector_opts(exa::LaunchOpts());
       o.grid = g;
       float t = 0;
       rc = time_launch(stream, 3, [&]() {
@@ -302,6 +321,7 @@ struct CellSet {
         best.corr.grid = g;
       }
     }
+    if (!rc) rc = reset_slots();  // the trials' minima
     if (!rc) {
       e = hipMemcpyAsync(d_luh, save_luh, sizeof(double) * ncells * NS * ND, hipMemcpyDeviceToDevice, stream);
       if (e == hipSuccess)

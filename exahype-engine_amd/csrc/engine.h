@@ -74,7 +74,7 @@ struct KernelCfg {
 //                  cells of one instance must be contiguous
 //   grid           > 0: persistent launch with this many workgroups looping over the
 //                  cell tiles (predictor, corrector); 0: one workgroup per tile
-//   riemann_waves  faces (wavefronts) per Riemann workgroup, 1..4 (the kernel's
+//   riemann_waves  wavefronts per Riemann workgroup, 1..4 (the kernel's
 //                  256-thread launch bound; other values fall back to 4)
 //   luh_update     predictor only: add the volume part of the update to this luh
 //                  (the predictor's own input) instead of writing lduh
@@ -94,10 +94,12 @@ struct LaunchOpts {
   // FP32 predictors and the fused corrector: extrapolated faces stored as FP32
   // (the FP32 forms compute them in FP32, so the storage is exact)
   bool faces_f32 = false;
-  // correctors without cinst: workgroup minima of the stable dt go to one of
-  // kDtSlots slots (separate cache lines) instead of all to dt_next; a
-  // launch_dt_reduce then merges the slots into dt_next and resets them
+  // correctors: workgroup minima of the stable dt go to one of dt_nslots slots of
+  // their instance (separate cache lines) instead of all to dt_next;
+  // launch_dt_reduce (one instance, kDtSlots) or launch_advance_time then merges
+  // the slots into dt_next and resets them
   double* dt_slots = nullptr;
+  int dt_nslots = 1024;  // kDtSlots
   // predictor, one-iteration FP32 CERK form: Picard guard buffer of 2 + ncells
   // ints {listed this launch (0 on entry), listed in total, list}; nullptr: no guard
   int* guard = nullptr;
@@ -118,7 +120,7 @@ constexpr int kDtSlots = 1024;
 constexpr int kDtSlotStride = 16;  // doubles: one 128-byte line per slot
 // slots [kDtSlots * kDtSlotStride] -> dt_next = min(dt_next, min slots); slots reset to DBL_MAX
 int launch_dt_reduce(hipStream_t s, double* slots, double* dt_next);
-int launch_dt_slots_init(hipStream_t s, double* slots);
+int launch_dt_slots_init(hipStream_t s, double* slots, long n = kDtSlots);
 
 // Boundary kinds per domain face f = 2d + o (exa_boundary_kind).
 enum BcKind { kBcPeriodic = 0, kBcWall = 1, kBcDirichletEntropyWave = 2, kBcExchange = 3 };
@@ -181,8 +183,9 @@ bool predictor_uses_guard(const KernelCfg& k);
 // cell_end): the one-iteration FP32 CERK line kernel.
 bool predictor_supports_range(const KernelCfg& k);
 // Time bookkeeping of the device step per instance, state = t[ninst], dt[ninst],
-// dt_next[ninst]: t += dt; dt = dt_next; dt_next = DBL_MAX.
-int launch_advance_time(hipStream_t s, double* state, int ninst = 1);
+// dt_next[ninst]: with slots [ninst][nslots] their minima are merged into dt_next
+// and reset; t += dt; dt = dt_next; dt_next = DBL_MAX.
+int launch_advance_time(hipStream_t s, double* state, int ninst = 1, double* slots = nullptr, int nslots = 0);
 
 // Boundary conditions (Euler): outside face data of every boundary face of a
 // uniform n^D mesh (ghost layout of LaunchOpts::ghost_q) at the step's t, dt
@@ -236,7 +239,7 @@ struct LinearCellArgs {
 };
 int launch_linear_cell(int order, const LinearCellArgs& a, hipStream_t s);
 
-// ---- AMR projections (amr.hip), single level, 2D or 3D ---------------------
+// ---- AMR projections (amr.hip), single level; face lists 3D ----------------
 // Face prolongation: per entry {coarse cell, face, subface s0 + 3 s1, target
 // cell}: lQhbnd / lFhbnd of the target's face = the coarse face prolongated
 // (overwrite).  Face restriction: per entry {coarse cell, face, first of

@@ -153,12 +153,18 @@ int enqueue_correct(exa_mesh* m, hipEvent_t* ev) {
                                       st + 2, o),
                 "corrector");
   }
-  if (rc) return rc;
-  return status(exa::launch_dt_reduce(m->stream, m->d_slots, st + 2), "dt reduction");
+  return rc;
 }
 
+// dt_next for a caller that reads it between correct and advance.
+int enqueue_dt_next(exa_mesh* m) {
+  return status(exa::launch_dt_reduce(m->stream, m->d_slots, m->d_state + 2), "dt reduction");
+}
+
+// Merges what the correctors left in the slots (nothing after enqueue_dt_next)
+// into dt_next and advances: in a whole step one launch instead of two.
 int enqueue_advance(exa_mesh* m, hipEvent_t* ev) {
-  const int rc = status(exa::launch_advance_time(m->stream, m->d_state), "advance time");
+  const int rc = status(exa::launch_advance_time(m->stream, m->d_state, 1, m->d_slots, exa::kDtSlots), "advance time");
   if (rc) return rc;
   if (ev) HIP_OK(hipEventRecord(ev[3], m->stream), "event");
   return EXA_OK;
@@ -218,7 +224,6 @@ int enqueue_step_slabs(exa_mesh* m) {
   }
   if (!rc) rc = correct(S - 1, S - 1);
   if (!rc) rc = correct(0, S - 1);
-  if (!rc) rc = status(exa::launch_dt_reduce(m->stream2, m->d_slots, st + 2), "dt reduction");
   // join (also after an error, so that a capture does not end with stream2 forked)
   HIP_OK(hipEventRecord(join, m->stream2), "event");
   HIP_OK(hipStreamWaitEvent(m->stream, join, 0), "stream wait");
@@ -667,7 +672,8 @@ int exa_mesh_step_predict(exa_mesh* m) {
 
 int exa_mesh_step_correct(exa_mesh* m) {
   if (!m) return EXA_ERR_ARG;
-  return enqueue_correct(m, nullptr);
+  const int rc = enqueue_correct(m, nullptr);
+  return rc ? rc : enqueue_dt_next(m);
 }
 
 int exa_mesh_step_advance(exa_mesh* m) {
