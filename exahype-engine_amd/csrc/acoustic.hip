@@ -25,8 +25,8 @@
 // Adjoint (this project's own; the reference has none): the transpose of the
 // step above for fixed (rho, c) plus d/dc through lambda = rho c^2 in the
 // predictor and the Riemann material average, and through the Rusanov speed
-// max(c_L, c_R).  Kernels ac_fbar_kernel, ac_riemann_adj_kernel,
-// ac_predict_adj_kernel.
+// max(c_L, c_R).  Kernels ac_fbar_kernel (before the first transposed step) and
+// ac_adjoint_kernel.
 #include <hip/hip_runtime.h>
 
 #include "engine.h"
@@ -174,7 +174,7 @@ __global__ void __launch_bounds__(kAcThreads) ac_predict_kernel(AcousticArgs a) 
       r.y = u0[1] + a.dt * acc[1];
       r.z = u0[2] + a.dt * acc[2];
       r.w = u0[3] + a.dt * acc[3];
-      reinterpret_cast<double4*>(a.u)[cell * N + nd] = r;
+      reinterpret_cast<double4*>(a.u_out)[cell * N + nd] = r;
     }
   }
 }
@@ -192,7 +192,11 @@ struct AcLineShape {
   static constexpr int N = B * B * B;
   static constexpr int F = B * B;    // lines per cell
   static constexpr int BUF = 3 * N;  // p, v, w of one level
-  static constexpr int CPB_T = kAcThreads / F;
+  // small workgroups: more of them fit beside each other on a CU, so that one
+  // computes while another waits at a barrier or for HBM (order 4 at 54^3: 256
+  // lanes 0.709, 128 lanes 0.639, 64 lanes, of which 50 have a line, 0.691 ms)
+  static constexpr int THREADS = B <= 4 ? 64 : 128;
+  static constexpr int CPB_T = THREADS / F;
   static constexpr int CPB_L = (60 * 1024) / (2 * BUF * 8);  // two level buffers per cell
   static constexpr int CPB = CPB_T < CPB_L ? CPB_T : CPB_L;    // cells per block
 };
@@ -255,7 +259,7 @@ __device__ __forceinline__ void line_derivatives(const double* __restrict__ Dm, 
 // s_k of the per-step row {sigma0, s_0..s_{B-1}}; the volume update is
 // dt * A(qh) - sigma0 g with that A (:474-640).
 template <int B, bool UPDATE, bool SPLIT>
-__global__ void __launch_bounds__(kAcThreads) ac_predict_lines_kernel(AcousticArgs a) {
+__global__ void __launch_bounds__((AcLineShape<B>::THREADS), 2) ac_predict_lines_kernel(AcousticArgs a) {
   using S = AcLineShape<B>;
   constexpr int N = S::N, F = S::F, CPB = S::CPB;
   __shared__ double sbuf[2][CPB][S::BUF];
@@ -354,10 +358,11 @@ __global__ void __launch_bounds__(kAcThreads) ac_predict_lines_kernel(AcousticAr
     double div[B], px[B], py[B], pz[B];
     line_derivatives<B>(Dm, invh, z, y, qh[0], qh[1], sb, div, px, py, pz);
     const double s0 = src ? stp[0] : 0.0;
-    double4* dst = reinterpret_cast<double4*>(a.u) + cell * N + ln * B;
+    const double4* old = reinterpret_cast<const double4*>(a.u) + cell * N + ln * B;
+    double4* dst = reinterpret_cast<double4*>(a.u_out) + cell * N + ln * B;
 #pragma unroll
     for (int x = 0; x < B; x++) {
-      const double4 q = dst[x];
+      const double4 q = old[x];
       dst[x] = make_double4(q.x + a.dt * (lam * div[x]) - (src ? s0 * gp[x] : 0.0), q.y + a.dt * (irho * px[x]),
                             q.z + a.dt * (irho * py[x]), q.w + a.dt * (irho * pz[x]));
     }
@@ -477,7 +482,8 @@ __global__ void __launch_bounds__(64) ac_receivers_kernel(AcousticArgs a, int N)
   if (lane == 0) a.rec[long(step) * a.nrec + r] = s;
 }
 
-// ubar[cell_r][node][0] += res[r] * weight (receivers in order; one block)
+// ubar[cell_r][node][0] += res[r] * weight (receivers in order; one block): the
+// last step's residuals, before the first transposed step
 __global__ void __launch_bounds__(256) ac_receivers_adj_kernel(AcousticArgs a, int N, const double* res) {
   for (int r = 0; r < a.nrec; r++) {
     const long cell = a.rcell[r];
@@ -533,96 +539,58 @@ __global__ void __launch_bounds__(kAcThreads) ac_fbar_kernel(AcousticArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// adjoint 2: Riemann transpose.  For every face of the cell: cotangent of the
-// cell's extrapolated variables (qbbar) and the face's part of dJ/dc_cell.
+// adjoint 2: one transposed step of a cell, in one kernel so that the cotangents
+// between its parts stay in LDS and registers:
+//   Riemann transpose: cotangent of the cell's extrapolated variables (LDS) and
+//     the faces' part of dJ/dc_cell, from qb and fbar of the cell and its neighbours;
+//   predictor + volume update transpose (recomputes the forward levels): ubar
+//     (cotangent of u^{k+1}) becomes the cotangent of u^k;
+//   the residuals of the receivers in the cell at the step before (res_prev) are
+//     added, and fbar_out (another buffer: neighbours still read fbar) is the next
+//     transposed step's fbar.  res_prev == nullptr: the first step, nothing follows.
+// Bound by LDS (34 accesses per node and level, 2 B levels) and the HBM traffic
+// of u, ubar, qb and the two fbar.  As four kernels (Riemann, predictor, fbar and
+// a receiver kernel of one workgroup) the same took 0.31 ms at 27^3 of order 4,
+// now 0.16 ms.
 // ---------------------------------------------------------------------------
 template <int B>
-__global__ void __launch_bounds__(kAcThreads) ac_riemann_adj_kernel(AcousticArgs a) {
-  using S = AcShape<B>;
-  constexpr int N = S::N, F = S::F, CPB = S::CPB;
-  __shared__ double sRed[kAcThreads];
-  const int t = threadIdx.x;
-  const int lc = t / N, nd = t - lc * N;
-  const long cell = long(blockIdx.x) * CPB + lc;
-  const bool on = lc < CPB && cell < a.ncells;
-  double gpart = 0.0;
-  if (on) {
-    const double rho_o = a.mat[2 * cell], c_o = a.mat[2 * cell + 1];
-    for (int task = nd; task < 6 * F; task += N) {
-      const int f = task / F, fn = task - f * F, d = f >> 1, o = f & 1;
-      const long nb = nb_cell(cell, a.n, d, o ? 1 : -1);
-      const double rho_n = a.mat[2 * nb], c_n = a.mat[2 * nb + 1];
-      const long io = (cell * 6 + f) * F + fn, in = (nb * 6 + (f ^ 1)) * F + fn;
-      const double4 qo = reinterpret_cast<const double4*>(a.qb)[io];
-      const double4 qn = reinterpret_cast<const double4*>(a.qb)[in];
-      const double4 bo = reinterpret_cast<const double4*>(a.fbar)[io];
-      const double4 bn = reinterpret_cast<const double4*>(a.fbar)[in];
-      const double4 QL = o ? qo : qn, QR = o ? qn : qo;
-      const double4 FLb = o ? bo : bn, FRb = o ? bn : bo;
-      const double cL = o ? c_o : c_n, cR = o ? c_n : c_o;
-      const double aL = fabs(cL), aR = fabs(cR);
-      const double smax = aL > aR ? aL : aR;
-      const double rhoa = 0.5 * ((o ? rho_n : rho_o) + (o ? rho_o : rho_n));
-      const double ca = 0.5 * (cR + cL);
-      const double lama = rhoa * ca * ca, irhoa = 1.0 / rhoa;
-      const double qd[4] = {0.5 * (QR.x - QL.x), 0.5 * (QR.y - QL.y), 0.5 * (QR.z - QL.z), 0.5 * (QR.w - QL.w)};
-      const double sb[4] = {FLb.x + FRb.x, FLb.y + FRb.y, FLb.z + FRb.z, FLb.w + FRb.w};
-      const double db[4] = {FRb.x - FLb.x, FRb.y - FLb.y, FRb.z - FLb.z, FRb.w - FLb.w};
-      double qdb[4];
-      double gs = 0.0;
-      for (int v = 0; v < 4; v++) {
-        qdb[v] = smax * db[v];
-        gs += db[v] * qd[v];
-      }
-      qdb[1 + d] += -lama * sb[0];
-      qdb[0] += -irhoa * sb[1 + d];
-      const double gl = sb[0] * (-qd[1 + d]);
-      // own share of d/dc: lambda_avg = rho_avg c_avg^2 with dc_avg/dc_own = 1/2;
-      // smax = max(c_L, c_R) goes to the larger one (ties to the left cell)
-      const bool own_max = o ? (aL >= aR) : (aR > aL);
-      gpart += gl * rhoa * ca + (own_max ? gs : 0.0);
-      const double sg = o ? -0.5 : 0.5;  // QL -= qdb/2, QR += qdb/2
-      reinterpret_cast<double4*>(a.qbbar)[io] =
-          make_double4(sg * qdb[0], sg * qdb[1], sg * qdb[2], sg * qdb[3]);
-    }
+struct AcAdjShape {
+  static constexpr int N = B * B * B, F = B * B;
+  // the smallest workgroup of which the cells fill 93 %
+  static constexpr int threads() {
+    for (int t : {64, 128, 256})
+      if (t / N * N * 100 >= 93 * t) return t;
+    return 256;
   }
-  // per-cell sum of gpart over its N threads
-  sRed[t] = gpart;
-  __syncthreads();
-  if (on && nd == 0) {
-    double s = 0.0;
-    for (int k = 0; k < N; k++) s += sRed[lc * N + k];
-    a.gc[cell] += s;
-  }
-}
+  static constexpr int THREADS = threads(), CPB = THREADS / N;
+};
 
-// ---------------------------------------------------------------------------
-// adjoint 3: predictor + volume update transpose (recomputes the forward
-// levels of the cell).  ubar (cotangent of u^{k+1}) is replaced by the
-// cotangent of u^k; gc[cell] += dJ/dc from the material matrix.
-// ---------------------------------------------------------------------------
 template <int B>
-__global__ void __launch_bounds__(kAcThreads) ac_predict_adj_kernel(AcousticArgs a) {
-  using S = AcShape<B>;
-  constexpr int N = S::N, F = S::F, CPB = S::CPB;
+__global__ void __launch_bounds__((AcAdjShape<B>::THREADS)) ac_adjoint_kernel(AcousticArgs a) {
+  using S = AcAdjShape<B>;
+  constexpr int N = S::N, F = S::F, CPB = S::CPB, THREADS = S::THREADS;
   __shared__ double sD[B * B];
   __shared__ double sFc[2][B];
+  __shared__ double sCf[2][B];  // dt/h * F_o[l] / w_l
   __shared__ double sL[CPB][4][N];
   __shared__ double sQb[CPB][6][F][4];
-  __shared__ double sRed[kAcThreads];
+  __shared__ double sRed[CPB][N + F];
   const int t = threadIdx.x;
   const int lc = t / N, nd = t - lc * N;
   const long cell = long(blockIdx.x) * CPB + lc;
   const bool slot = lc < CPB;
   const bool on = slot && cell < a.ncells;
-  if (t < B * B) sD[t] = a.tab->dudx[t] / a.h;
+  for (int i = t; i < B * B; i += THREADS) sD[i] = a.tab->dudx[i] / a.h;
   if (t < B) {
     sFc[0][t] = a.tab->F0[t];
     sFc[1][t] = a.tab->F1[t];
+    sCf[0][t] = a.dt / a.h * a.tab->F0[t] / a.tab->w[t];
+    sCf[1][t] = a.dt / a.h * a.tab->F1[t] / a.tab->w[t];
   }
   const int x = nd % B, y = (nd / B) % B, z = nd / (B * B);
   double u0[4] = {0, 0, 0, 0}, ub[4] = {0, 0, 0, 0};
   double rho = 1.0, c = 1.0;
+  double gpart = 0.0;
   if (on) {
     const double4 q = reinterpret_cast<const double4*>(a.u)[cell * N + nd];
     u0[0] = q.x;
@@ -636,13 +604,46 @@ __global__ void __launch_bounds__(kAcThreads) ac_predict_adj_kernel(AcousticArgs
     ub[3] = b.w;
     rho = a.mat[2 * cell];
     c = a.mat[2 * cell + 1];
+    // Riemann transpose of the cell's faces
     for (int task = nd; task < 6 * F; task += N) {
-      const double4 qb = reinterpret_cast<const double4*>(a.qbbar)[cell * 6 * F + task];
-      double* dst = &sQb[lc][0][0][0] + 4 * task;
-      dst[0] = qb.x;
-      dst[1] = qb.y;
-      dst[2] = qb.z;
-      dst[3] = qb.w;
+      const int f = task / F, fn = task - f * F, d = f >> 1, o = f & 1;
+      const long nb = nb_cell(cell, a.n, d, o ? 1 : -1);
+      const double rho_n = a.mat[2 * nb], c_n = a.mat[2 * nb + 1];
+      const long io = (cell * 6 + f) * F + fn, in = (nb * 6 + (f ^ 1)) * F + fn;
+      const double4 qo = reinterpret_cast<const double4*>(a.qb)[io];
+      const double4 qn = reinterpret_cast<const double4*>(a.qb)[in];
+      const double4 bo = reinterpret_cast<const double4*>(a.fbar)[io];
+      const double4 bn = reinterpret_cast<const double4*>(a.fbar)[in];
+      const double4 QL = o ? qo : qn, QR = o ? qn : qo;
+      const double4 FLb = o ? bo : bn, FRb = o ? bn : bo;
+      const double cL = o ? c : c_n, cR = o ? c_n : c;
+      const double aL = fabs(cL), aR = fabs(cR);
+      const double smax = aL > aR ? aL : aR;
+      const double rhoa = 0.5 * ((o ? rho_n : rho) + (o ? rho : rho_n));
+      const double ca = 0.5 * (cR + cL);
+      const double lama = rhoa * ca * ca, irhoa = 1.0 / rhoa;
+      const double qd[4] = {0.5 * (QR.x - QL.x), 0.5 * (QR.y - QL.y), 0.5 * (QR.z - QL.z), 0.5 * (QR.w - QL.w)};
+      const double sb[4] = {FLb.x + FRb.x, FLb.y + FRb.y, FLb.z + FRb.z, FLb.w + FRb.w};
+      const double db[4] = {FRb.x - FLb.x, FRb.y - FLb.y, FRb.z - FLb.z, FRb.w - FLb.w};
+      // component 1 + d by selection (d differs between lanes)
+      const double qdn = d == 0 ? qd[1] : (d == 1 ? qd[2] : qd[3]);
+      const double sbn = d == 0 ? sb[1] : (d == 1 ? sb[2] : sb[3]);
+      double qdb[4];
+      double gs = 0.0;
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        qdb[v] = smax * db[v] + (v == 1 + d ? -lama * sb[0] : 0.0);
+        gs += db[v] * qd[v];
+      }
+      qdb[0] += -irhoa * sbn;
+      const double gl = sb[0] * (-qdn);
+      // own share of d/dc: lambda_avg = rho_avg c_avg^2 with dc_avg/dc_own = 1/2;
+      // smax = max(c_L, c_R) goes to the larger one (ties to the left cell)
+      const bool own_max = o ? (aL >= aR) : (aR > aL);
+      gpart += gl * rhoa * ca + (own_max ? gs : 0.0);
+      const double sg = o ? -0.5 : 0.5;  // QL -= qdb/2, QR += qdb/2
+#pragma unroll
+      for (int v = 0; v < 4; v++) sQb[lc][f][fn][v] = sg * qdb[v];
     }
   }
   const double lam = rho * c * c, irho = 1.0 / rho;
@@ -691,7 +692,9 @@ __global__ void __launch_bounds__(kAcThreads) ac_predict_adj_kernel(AcousticArgs
   if (on) {
     const int l3[3] = {x, y, z};
     const int fi[3] = {z * B + y, z * B + x, y * B + x};
+#pragma unroll
     for (int d = 0; d < 3; d++)
+#pragma unroll
       for (int v = 0; v < 4; v++)
         qhb[v] += sFc[0][l3[d]] * sQb[lc][2 * d][fi[d]][v] + sFc[1][l3[d]] * sQb[lc][2 * d + 1][fi[d]][v];
   }
@@ -728,16 +731,49 @@ __global__ void __launch_bounds__(kAcThreads) ac_predict_adj_kernel(AcousticArgs
     lb[2] = at[i] * qhb[2] + n2;
     lb[3] = at[i] * qhb[3] + n3;
   }
-  if (on) {
-    reinterpret_cast<double4*>(a.ubar)[cell * N + nd] =
-        make_double4(ub[0] + lb[0], ub[1] + lb[1], ub[2] + lb[2], ub[3] + lb[3]);
+#pragma unroll
+  for (int v = 0; v < 4; v++) ub[v] += lb[v];
+  if (on && a.res_prev) {
+    // receivers of this cell, in their order
+    for (int k = a.rstart[cell]; k < a.rstart[cell + 1]; k++) {
+      const int r = a.rorder[k];
+      ub[0] += a.res_prev[r] * a.rw[long(r) * N + nd];
+    }
   }
-  sRed[t] = on ? glam : 0.0;
+  if (on) reinterpret_cast<double4*>(a.ubar)[cell * N + nd] = make_double4(ub[0], ub[1], ub[2], ub[3]);
+  // dJ/dc of the cell: rows of B nodes, then the rows, in a fixed order
+  __syncthreads();
+  if (slot) {
+    sRed[lc][nd] = gpart + glam * 2.0 * rho * c;
+    for (int v = 0; v < 4; v++) sL[lc][v][nd] = ub[v];
+  }
+  __syncthreads();
+  if (slot && nd < F) {
+    double r = 0.0;
+#pragma unroll
+    for (int i = 0; i < B; i++) r += sRed[lc][nd * B + i];
+    sRed[lc][N + nd] = r;
+  }
   __syncthreads();
   if (on && nd == 0) {
-    double s = 0.0;
-    for (int k = 0; k < N; k++) s += sRed[lc * N + k];
-    a.gc[cell] += s * 2.0 * rho * c;
+    double r = 0.0;
+    for (int i = 0; i < F; i++) r += sRed[lc][N + i];
+    a.gc[cell] += r;
+  }
+  if (on && a.res_prev) {
+    for (int task = nd; task < 6 * F; task += N) {
+      const int f = task / F, fn = task - f * F, d = f >> 1, o = f & 1;
+      const int fa = fn / B, fb = fn - fa * B;
+      double r[4] = {0, 0, 0, 0};
+#pragma unroll
+      for (int l = 0; l < B; l++) {
+        const int node = face_line_node<B>(d, fa, fb, l);
+        const double cf = sCf[o][l];
+#pragma unroll
+        for (int v = 0; v < 4; v++) r[v] -= cf * sL[lc][v][node];
+      }
+      reinterpret_cast<double4*>(a.fbar_out)[(cell * 6 + f) * F + fn] = make_double4(r[0], r[1], r[2], r[3]);
+    }
   }
 }
 
@@ -750,16 +786,16 @@ int launch_all(int which, const AcousticArgs& a, hipStream_t s) {
     case kAcPredictUpdate:
       if (a.split_ck && a.pred_variant != 0) return -1;  // the split predictor has the x-line form only
       if (a.split_ck)
-        ac_predict_lines_kernel<B, true, true><<<lblocks, kAcThreads, 0, s>>>(a);
+        ac_predict_lines_kernel<B, true, true><<<lblocks, AcLineShape<B>::THREADS, 0, s>>>(a);
       else if (a.pred_variant == 0)
-        ac_predict_lines_kernel<B, true, false><<<lblocks, kAcThreads, 0, s>>>(a);
+        ac_predict_lines_kernel<B, true, false><<<lblocks, AcLineShape<B>::THREADS, 0, s>>>(a);
       else
         ac_predict_kernel<B, true><<<blocks, kAcThreads, 0, s>>>(a);
       break;
     case kAcPredictFaces:
       if (a.split_ck) return -1;  // the adjoint sweeps transpose the generic predictor only
       if (a.pred_variant == 0)
-        ac_predict_lines_kernel<B, false, false><<<lblocks, kAcThreads, 0, s>>>(a);
+        ac_predict_lines_kernel<B, false, false><<<lblocks, AcLineShape<B>::THREADS, 0, s>>>(a);
       else
         ac_predict_kernel<B, false><<<blocks, kAcThreads, 0, s>>>(a);
       break;
@@ -769,12 +805,11 @@ int launch_all(int which, const AcousticArgs& a, hipStream_t s) {
     case kAcFbar:
       ac_fbar_kernel<B><<<blocks, kAcThreads, 0, s>>>(a);
       break;
-    case kAcRiemannAdj:
-      ac_riemann_adj_kernel<B><<<blocks, kAcThreads, 0, s>>>(a);
+    case kAcAdjoint: {
+      using A = AcAdjShape<B>;
+      ac_adjoint_kernel<B><<<static_cast<unsigned>((a.ncells + A::CPB - 1) / A::CPB), A::THREADS, 0, s>>>(a);
       break;
-    case kAcPredictAdj:
-      ac_predict_adj_kernel<B><<<blocks, kAcThreads, 0, s>>>(a);
-      break;
+    }
     case kAcReceivers:
       if (a.nrec > 0) ac_receivers_kernel<<<a.nrec, 64, 0, s>>>(a, S::N);
       break;

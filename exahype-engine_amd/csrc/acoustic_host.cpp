@@ -24,6 +24,7 @@
 #include <cmath>
 #include <cstring>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/exahype_amd.h"
@@ -43,7 +44,7 @@ struct exa_acoustic {
   int step = 0;  // host mirror of the device step counter
   hipStream_t stream = nullptr;
   double *d_u = nullptr, *d_mat = nullptr, *d_qb = nullptr;
-  double *d_ubar = nullptr, *d_fbar = nullptr, *d_qbbar = nullptr, *d_gc = nullptr;
+  double *d_ubar = nullptr, *d_fbar = nullptr, *d_fbar2 = nullptr, *d_gc = nullptr;
   int* d_step = nullptr;
   std::vector<double> mat;  // host copy of (rho, c) per cell
   // source
@@ -56,6 +57,7 @@ struct exa_acoustic {
   // receivers
   int nrec = 0;
   int* d_rcell = nullptr;
+  int *d_rstart = nullptr, *d_rorder = nullptr;  // receivers by cell [nc + 1], [nrec]
   double* d_rw = nullptr;
   double* d_rec = nullptr;
   long rec_cap = 0;  // doubles
@@ -221,23 +223,27 @@ exa::AcousticArgs args(exa_acoustic* ac, double* u) {
   a.rw = ac->d_rw;
   a.ubar = ac->d_ubar;
   a.fbar = ac->d_fbar;
-  a.qbbar = ac->d_qbbar;
+  a.u_out = u;
+  a.rstart = ac->d_rstart;
+  a.rorder = ac->d_rorder;
   a.gc = ac->d_gc;
   a.pred_variant = ac->pred_variant;
   a.split_ck = ac->k.split_ck;
   return a;
 }
 
-// one forward step on u (step index `step`, or the device counter if < 0);
+// one forward step from u to u_out (step index `step`, or the device counter if < 0);
 // receivers recorded into rec[(step - rec_base) * nrec + r] when rec != nullptr
-int enqueue_forward(exa_acoustic* ac, double* u, int step, double* rec, hipEvent_t* ev = nullptr) {
+int enqueue_forward(exa_acoustic* ac, double* u, double* u_out, int step, double* rec, hipEvent_t* ev = nullptr) {
   exa::TraceRange tr("exa.acoustic.step");
   exa::AcousticArgs a = args(ac, u);
+  a.u_out = u_out;
   a.step_override = step;
   const int o = ac->k.order;
   if (ev) HIP_OK(hipEventRecord(ev[0], ac->stream), "event");
   RC_OK(status(exa::launch_acoustic(exa::kAcPredictUpdate, o, a, ac->stream), "acoustic predictor"));
   if (ev) HIP_OK(hipEventRecord(ev[1], ac->stream), "event");
+  a.u = u_out;
   RC_OK(status(exa::launch_acoustic(exa::kAcCorrector, o, a, ac->stream), "acoustic corrector"));
   if (ev) HIP_OK(hipEventRecord(ev[2], ac->stream), "event");
   if (rec && ac->nrec > 0) {
@@ -248,12 +254,13 @@ int enqueue_forward(exa_acoustic* ac, double* u, int step, double* rec, hipEvent
 }
 
 void free_acoustic(exa_acoustic* ac) {
-  double* bufs[] = {ac->d_u,     ac->d_mat,   ac->d_qb,     ac->d_ubar,  ac->d_fbar, ac->d_qbbar,
+  double* bufs[] = {ac->d_u,     ac->d_mat,   ac->d_qb,     ac->d_ubar,  ac->d_fbar, ac->d_fbar2,
                     ac->d_gc,    ac->d_src_g, ac->d_src_tab, ac->d_rw,   ac->d_rec,  ac->d_res};
   for (double* b : bufs)
     if (b) (void)hipFree(b);
   if (ac->d_step) (void)hipFree(ac->d_step);
-  if (ac->d_rcell) (void)hipFree(ac->d_rcell);
+  for (int* p : {ac->d_rcell, ac->d_rstart, ac->d_rorder})
+    if (p) (void)hipFree(p);
   for (hipEvent_t e : ac->ev) (void)hipEventDestroy(e);
   if (ac->stream) (void)hipStreamDestroy(ac->stream);
   delete ac;
@@ -461,9 +468,10 @@ int exa_acoustic_set_source(exa_acoustic* ac, const double* x, double amp, doubl
 
 int exa_acoustic_set_receivers(exa_acoustic* ac, int nrec, const double* xr) {
   if (!ac || nrec < 0 || (nrec > 0 && !xr)) return argerr("exa_acoustic_set_receivers: invalid argument");
-  if (ac->d_rcell) (void)hipFree(ac->d_rcell);
+  for (int* p : {ac->d_rcell, ac->d_rstart, ac->d_rorder})
+    if (p) (void)hipFree(p);
   if (ac->d_rw) (void)hipFree(ac->d_rw);
-  ac->d_rcell = nullptr;
+  ac->d_rcell = ac->d_rstart = ac->d_rorder = nullptr;
   ac->d_rw = nullptr;
   ac->nrec = 0;
   if (nrec == 0) return EXA_OK;
@@ -480,6 +488,16 @@ int exa_acoustic_set_receivers(exa_acoustic* ac, int nrec, const double* xr) {
       for (int y = 0; y < B; y++)
         for (int x = 0; x < B; x++) wts[size_t(r) * N + (z * B + y) * B + x] = phi[0][x] * phi[1][y] * phi[2][z];
   }
+  // by cell, each cell's receivers in their order
+  std::vector<int> start(size_t(ac->nc) + 1, 0), order(nrec);
+  for (int r = 0; r < nrec; r++) start[cells[r] + 1]++;
+  for (long c = 0; c < ac->nc; c++) start[c + 1] += start[c];
+  std::vector<int> at(start.begin(), start.end() - 1);
+  for (int r = 0; r < nrec; r++) order[at[cells[r]]++] = r;
+  HIP_OK(hipMalloc(&ac->d_rstart, sizeof(int) * start.size()), "hipMalloc(receivers)");
+  HIP_OK(hipMalloc(&ac->d_rorder, sizeof(int) * nrec), "hipMalloc(receivers)");
+  HIP_OK(hipMemcpy(ac->d_rstart, start.data(), sizeof(int) * start.size(), hipMemcpyHostToDevice), "upload receivers");
+  HIP_OK(hipMemcpy(ac->d_rorder, order.data(), sizeof(int) * nrec, hipMemcpyHostToDevice), "upload receivers");
   HIP_OK(hipMalloc(&ac->d_rcell, sizeof(int) * nrec), "hipMalloc(receivers)");
   HIP_OK(hipMalloc(&ac->d_rw, sizeof(double) * wts.size()), "hipMalloc(receivers)");
   HIP_OK(hipMemcpy(ac->d_rcell, cells.data(), sizeof(int) * nrec, hipMemcpyHostToDevice), "upload receivers");
@@ -535,7 +553,7 @@ int exa_acoustic_run(exa_acoustic* ac, int nsteps, int use_graph, double* rec) {
       ac->timed_steps = nsteps;
     }
     for (int i = 0; !rc && i < nsteps; i++) {
-      rc = enqueue_forward(ac, ac->d_u, s0 + i, ac->d_rec - long(s0) * ac->nrec,
+      rc = enqueue_forward(ac, ac->d_u, ac->d_u, s0 + i, ac->d_rec - long(s0) * ac->nrec,
                            ac->timing ? &ac->ev[size_t(3) * i] : nullptr);
     }
   }
@@ -572,7 +590,7 @@ int exa_acoustic_misfit_gradient(exa_acoustic* ac, int nsteps, int every, const 
   }
   const int s0 = ac->step, K = nsteps, R = ac->nrec, o = ac->k.order;
   const int nck = (K + every - 1) / every;
-  const int seg = every < K ? every : K;
+  const int seg = (every < K ? every : K) - 1;  // states of a segment besides its checkpoint
   const size_t su = size_t(ac->nc) * ac->N * 4, sq = size_t(ac->nc) * 6 * ac->F * 4;
   RC_OK(ensure_source_table(ac, s0 + K));
   RC_OK(grow(&ac->d_rec, &ac->rec_cap, long(K) * R));
@@ -580,13 +598,13 @@ int exa_acoustic_misfit_gradient(exa_acoustic* ac, int nsteps, int every, const 
   if (!ac->d_ubar) {
     HIP_OK(hipMalloc(&ac->d_ubar, sizeof(double) * su), "hipMalloc(adjoint)");
     HIP_OK(hipMalloc(&ac->d_fbar, sizeof(double) * sq), "hipMalloc(adjoint)");
-    HIP_OK(hipMalloc(&ac->d_qbbar, sizeof(double) * sq), "hipMalloc(adjoint)");
+    HIP_OK(hipMalloc(&ac->d_fbar2, sizeof(double) * sq), "hipMalloc(adjoint)");
     HIP_OK(hipMalloc(&ac->d_gc, sizeof(double) * ac->nc), "hipMalloc(adjoint)");
   }
   double* d_ck = nullptr;
   double* d_seg = nullptr;
   HIP_OK(hipMalloc(&d_ck, sizeof(double) * su * nck), "hipMalloc(checkpoints)");
-  hipError_t ea = hipMalloc(&d_seg, sizeof(double) * su * seg);
+  hipError_t ea = seg > 0 ? hipMalloc(&d_seg, sizeof(double) * su * seg) : hipSuccess;
   if (ea != hipSuccess) {
     (void)hipFree(d_ck);
     return fail(ea, "hipMalloc(segment)");
@@ -605,7 +623,7 @@ int exa_acoustic_misfit_gradient(exa_acoustic* ac, int nsteps, int every, const 
                                           hipMemcpyDeviceToDevice, ac->stream);
       if (e != hipSuccess) rc = fail(e, "checkpoint");
     }
-    if (!rc) rc = enqueue_forward(ac, ac->d_u, s0 + k, rec_base);
+    if (!rc) rc = enqueue_forward(ac, ac->d_u, ac->d_u, s0 + k, rec_base);
   }
   if (!rc && hipEventRecord(ev[1], ac->stream) != hipSuccess) rc = fail(hipErrorUnknown, "event");
   std::vector<double> rec(size_t(K) * R), res(size_t(K) * R);
@@ -632,23 +650,22 @@ int exa_acoustic_misfit_gradient(exa_acoustic* ac, int nsteps, int every, const 
   for (int j = nck - 1; !rc && j >= 0; j--) {
     const int k0 = j * every, k1 = (k0 + every < K) ? k0 + every : K;
     (void)hipEventRecord(ev[2 + 3 * j], ac->stream);
-    hipError_t e = hipMemcpyAsync(d_seg, d_ck + su * j, sizeof(double) * su, hipMemcpyDeviceToDevice, ac->stream);
-    for (int k = k0; e == hipSuccess && !rc && k < k1 - 1; k++) {
-      double* dst = d_seg + su * (k - k0 + 1);
-      e = hipMemcpyAsync(dst, d_seg + su * (k - k0), sizeof(double) * su, hipMemcpyDeviceToDevice, ac->stream);
-      if (e == hipSuccess) rc = enqueue_forward(ac, dst, s0 + k, nullptr);
-    }
-    if (e != hipSuccess && !rc) rc = fail(e, "recompute");
+    // states k0 + 1 .. k1 - 1 of the segment; state k0 is the checkpoint
+    auto state = [&](int k) { return k == k0 ? d_ck + su * j : d_seg + su * (k - k0 - 1); };
+    for (int k = k0; !rc && k < k1 - 1; k++) rc = enqueue_forward(ac, state(k), state(k + 1), s0 + k, nullptr);
     (void)hipEventRecord(ev[3 + 3 * j], ac->stream);
     for (int k = k1 - 1; !rc && k >= k0; k--) {
-      double* uk = d_seg + su * (k - k0);
-      exa::AcousticArgs a = args(ac, uk);
+      exa::AcousticArgs a = args(ac, state(k));
       a.step_override = s0 + k;
-      rc = status(exa::launch_acoustic_receivers_adj(o, a, ac->d_res + long(k) * R, ac->stream), "receiver adjoint");
+      if (k == K - 1) {
+        rc = status(exa::launch_acoustic_receivers_adj(o, a, ac->d_res + long(k) * R, ac->stream), "receiver adjoint");
+        if (!rc) rc = status(exa::launch_acoustic(exa::kAcFbar, o, a, ac->stream), "adjoint fbar");
+      }
       if (!rc) rc = status(exa::launch_acoustic(exa::kAcPredictFaces, o, a, ac->stream), "acoustic faces");
-      if (!rc) rc = status(exa::launch_acoustic(exa::kAcFbar, o, a, ac->stream), "adjoint fbar");
-      if (!rc) rc = status(exa::launch_acoustic(exa::kAcRiemannAdj, o, a, ac->stream), "adjoint riemann");
-      if (!rc) rc = status(exa::launch_acoustic(exa::kAcPredictAdj, o, a, ac->stream), "adjoint predictor");
+      if (k > 0) a.res_prev = ac->d_res + long(k - 1) * R;
+      a.fbar_out = ac->d_fbar2;
+      if (!rc) rc = status(exa::launch_acoustic(exa::kAcAdjoint, o, a, ac->stream), "adjoint step");
+      std::swap(ac->d_fbar, ac->d_fbar2);
     }
     (void)hipEventRecord(ev[4 + 3 * j], ac->stream);
   }

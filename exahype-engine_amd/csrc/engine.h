@@ -258,7 +258,8 @@ int launch_volume_project(const KernelCfg& k, hipStream_t s, int nv, const doubl
 // ---- linear acoustics (acoustic.hip) ---------------------------------------
 // Device arrays of the acoustic mesh: u[cell][node][4] (p,u,v,w), mat[cell][2]
 // (rho, c), qb[cell][6][B*B][4] (time-averaged variables on the faces),
-// adjoint cotangents ubar (like u), fbar and qbbar (like qb), gc[cell].
+// adjoint cotangents ubar (like u), fbar and fbar_out (like qb), gc[cell].  The
+// predictor reads u and writes the volume update to u_out (u itself in a plain step).
 struct AcousticArgs {
   long ncells = 0;
   int n = 0;  // cells per direction (periodic n^3 mesh)
@@ -278,12 +279,17 @@ struct AcousticArgs {
   double* rec = nullptr;           // [steps][nrec]
   double* ubar = nullptr;
   double* fbar = nullptr;
-  double* qbbar = nullptr;
+  double* fbar_out = nullptr;
+  double* u_out = nullptr;
+  // receivers by cell: those of cell c are rorder[rstart[c] .. rstart[c + 1])
+  const int* rstart = nullptr;
+  const int* rorder = nullptr;
+  const double* res_prev = nullptr;  // residuals [nrec] of the step before, nullptr at the first
   double* gc = nullptr;
   int pred_variant = 0;  // forward predictor: 0 x-line form, 1 node form
   int split_ck = 0;      // split Cauchy-Kowalevski predictor (x-line form only)
 };
-enum { kAcPredictUpdate = 0, kAcPredictFaces, kAcCorrector, kAcFbar, kAcRiemannAdj, kAcPredictAdj, kAcReceivers };
+enum { kAcPredictUpdate = 0, kAcPredictFaces, kAcCorrector, kAcFbar, kAcAdjoint, kAcReceivers };
 bool acoustic_order_supported(int order);
 int launch_acoustic(int which, int order, const AcousticArgs& a, hipStream_t s);
 int launch_acoustic_receivers_adj(int order, const AcousticArgs& a, const double* res, hipStream_t s);

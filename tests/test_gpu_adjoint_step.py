@@ -1,0 +1,52 @@
+"""GPU: the fused transposed step of the acoustic mesh at every compiled order,
+against the oracle's FP64 adjoint.
+
+The mesh sizes leave the last workgroup with empty cell slots, two receivers sit
+in one cell and one in the source's (their residuals are added inside the step),
+and the checkpoint intervals cover a segment of one step, a shorter last segment
+and one segment for the whole run.  Bar: 1e-10 relative L2 of the gradient, as of
+the other gradient tests; J and the forward state 1e-12.
+"""
+import numpy as np
+import pytest
+
+import exahype_amd as E
+import oracle as O
+from exahype_amd import problems as P
+
+pytestmark = pytest.mark.gpu
+
+
+def rel_l2(a, b):
+    return np.linalg.norm(np.ravel(a) - np.ravel(b)) / np.linalg.norm(np.ravel(b))
+
+
+@pytest.mark.parametrize("every", [1, 3, 50])
+@pytest.mark.parametrize("order,n", [(1, 3), (2, 5), (3, 3), (4, 3), (5, 2)])
+def test_gradient_at_every_order(order, n, every):
+    print(f"[adjoint step] order={order} n={n} every={every}", flush=True)
+    rng = np.random.default_rng(100 * order + n)
+    h, steps = 1.0 / n, 5
+    c = 1.0 + 0.2 * rng.uniform(-1, 1, n ** 3)
+    rho = 1.0 + 0.1 * rng.uniform(-1, 1, n ** 3)
+    u = 0.1 * rng.normal(size=(n ** 3, (order + 1) ** 3, 4))
+    luh = P.acoustic_state(n, order, c, rho, u)
+    ctx = E.Context(3, order, 4, 2, E.PDE_ACOUSTIC)
+    ac = E.Acoustic(ctx, n, h)
+    ac.set_solution(luh)
+    ac.set_dt(0.0)
+    dt = ac.time()[2]
+    src = ((0.4 * h, 0.6 * h, 0.3 * h), 1.0, 5.0, 0.05)
+    rec = np.array([[0.2, 0.3, 0.4], [0.9, 0.8, 0.1], [0.55, 0.15, 0.75]]) * 0.999
+    rec = np.concatenate([rec, rec[1:2] * 0.99, np.array([[0.3 * h, 0.3 * h, 0.3 * h]])])
+    obs = rng.normal(0.0, 0.1, (steps, len(rec)))
+    orc = O.LinearOracle(3, order)
+    J_ref, g_ref = orc.misfit_grad(luh, n, h, dt, steps, src, rec, obs)
+    ac.set_source(*src)
+    ac.set_receivers(rec)
+    J, g = ac.misfit_gradient(steps, obs, checkpoint_every=every)
+    assert abs(J - J_ref) <= 1e-12 * abs(J_ref)
+    assert rel_l2(g, g_ref) <= 1e-10
+    ref = luh.copy()
+    orc.run(ref, n, h, dt, steps, src, rec)
+    assert rel_l2(ac.get_solution(), ref) <= 1e-12
