@@ -13,7 +13,7 @@
 // Decomposition: a lane owns one spatial node and its whole time column
 // lQi[0..B)[V] in registers, so flux evaluation and the time solve need no
 // exchange.  A spatial derivative is taken line by line: the owners write
-// their fluxes into LDS with the B values of each (direction, line, variable)
+// their fluxes into LDS with the B values of each (variable, direction, line)
 // contiguous, then the workgroup's lanes take those lines one each, contract
 // them with the operator (uniform coefficients in scalar registers) and write
 // the B results back in place, and the owners read their values.  An LDS value
@@ -25,8 +25,7 @@
 // node-column form before it (each lane reading the lines through its node;
 // MI355X, predictor alone): 3D order 5 FP64 at 81^3 36.3 -> 23.9 ms (20 TF/s of
 // executed contraction work, 78.6 peak), with the CERK guess at 40^3 2.60 ->
-// 1.86 ms, 3D order 3 FP64 at 35^3 0.573 -> 0.398 ms and FP32 at 45^3 0.536 ->
-// 0.462 ms, 2D order 4 at 243^2 0.284 -> 0.212 ms.
+// 1.86 ms, 2D order 4 at 243^2 0.284 -> 0.212 ms.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -54,22 +53,18 @@ struct Shape {
   }
   static constexpr int THREADS = threads();
   static constexpr int CPB = THREADS / NS;  // cells per workgroup
-  // Distance of two lines.  FP64 lines of four start an odd number of doubles
-  // apart: at 4 the lanes' 16-byte pieces meet on the LDS banks two to one (3D
-  // order 3 at 35^3: 0.409 -> 0.398 ms); longer lines and FP32 need no padding
-  // (3D order 5 with 7 instead of 6: 23.9 -> 24.4 ms at 81^3).
-  static constexpr int LS = sizeof(R) == 8 && B == 4 ? 5 : B;
-  static constexpr int SLICE = CPB * NL * V * LS;  // values of one time slice
+  static constexpr int SLICE = CPB * NL * V * B;  // values of one time slice
   // Time slices between two barriers.  Two fill the rounds of line tasks better
   // and halve the barriers where the registers allow two workgroups per CU
   // anyway (3D order 5 in FP64 at 81^3: 26.4 -> 23.9 ms; three leave LDS for one
-  // workgroup: 38.3 ms); the smaller 3D cells gain more from the workgroups that
-  // the LDS of a second slice would cost (3D order 3 at 35^3: 0.456 -> 0.398 ms).
+  // workgroup: 38.3 ms); smaller 3D cells gain as much from the workgroups that
+  // the LDS of a second slice would cost (batched 3D order 4: equal).
   static constexpr int TS = D == 3 && B <= 5 ? 1 : 2;
   static constexpr int NROW = NS / B;
-  static constexpr int LINE_BYTES = TS * SLICE * int(sizeof(R));
-  static constexpr int END = CPB * NL * V * B;
-  static constexpr int END_BYTES = (END + CPB * NS * ND) * 8;
+  // order 3 exchanges its lines between lanes and needs the buffer at the end only
+  static constexpr bool LANES = B == 4;
+  static constexpr int LINE_BYTES = LANES ? 0 : TS * SLICE * int(sizeof(R));
+  static constexpr int END_BYTES = (SLICE + CPB * NS * ND) * 8;
   static constexpr int BUF_BYTES = LINE_BYTES > END_BYTES ? LINE_BYTES : END_BYTES;
   static constexpr int RED = CPB * (NS + NROW);
 };
@@ -98,16 +93,16 @@ __device__ __forceinline__ Const<X>* opaque(const X* p) {
 }
 
 // Line of B values at p (16-byte pieces where the line start allows them).
-template <typename R, int B, int LS>
+template <typename R, int B>
 __device__ __forceinline__ void load_line(const R* p, R (&f)[B]) {
-  if constexpr (sizeof(R) == 8 && B % 2 == 0 && LS % 2 == 0) {
+  if constexpr (sizeof(R) == 8 && B % 2 == 0) {
 #pragma unroll
     for (int i = 0; i < B / 2; i++) {
       const double2 v = reinterpret_cast<const double2*>(p)[i];
       f[2 * i] = v.x;
       f[2 * i + 1] = v.y;
     }
-  } else if constexpr (sizeof(R) == 4 && B % 4 == 0 && LS % 4 == 0) {
+  } else if constexpr (sizeof(R) == 4 && B % 4 == 0) {
 #pragma unroll
     for (int i = 0; i < B / 4; i++) {
       const float4 v = reinterpret_cast<const float4*>(p)[i];
@@ -116,7 +111,7 @@ __device__ __forceinline__ void load_line(const R* p, R (&f)[B]) {
       f[4 * i + 2] = v.z;
       f[4 * i + 3] = v.w;
     }
-  } else if constexpr (sizeof(R) == 4 && B % 2 == 0 && LS % 2 == 0) {
+  } else if constexpr (sizeof(R) == 4 && B % 2 == 0) {
 #pragma unroll
     for (int i = 0; i < B / 2; i++) {
       const float2 v = reinterpret_cast<const float2*>(p)[i];
@@ -128,16 +123,16 @@ __device__ __forceinline__ void load_line(const R* p, R (&f)[B]) {
     for (int i = 0; i < B; i++) f[i] = p[i];
   }
 }
-template <typename R, int B, int LS>
+template <typename R, int B>
 __device__ __forceinline__ void store_line(R* p, const R (&f)[B]) {
-  if constexpr (sizeof(R) == 8 && B % 2 == 0 && LS % 2 == 0) {
+  if constexpr (sizeof(R) == 8 && B % 2 == 0) {
 #pragma unroll
     for (int i = 0; i < B / 2; i++) reinterpret_cast<double2*>(p)[i] = make_double2(f[2 * i], f[2 * i + 1]);
-  } else if constexpr (sizeof(R) == 4 && B % 4 == 0 && LS % 4 == 0) {
+  } else if constexpr (sizeof(R) == 4 && B % 4 == 0) {
 #pragma unroll
     for (int i = 0; i < B / 4; i++)
       reinterpret_cast<float4*>(p)[i] = make_float4(f[4 * i], f[4 * i + 1], f[4 * i + 2], f[4 * i + 3]);
-  } else if constexpr (sizeof(R) == 4 && B % 2 == 0 && LS % 2 == 0) {
+  } else if constexpr (sizeof(R) == 4 && B % 2 == 0) {
 #pragma unroll
     for (int i = 0; i < B / 2; i++) reinterpret_cast<float2*>(p)[i] = make_float2(f[2 * i], f[2 * i + 1]);
   } else {
@@ -186,6 +181,59 @@ struct EvenOdd {
     }
   }
 };
+
+// Four-node lines (order 3) stay in one wavefront: 16 consecutive lanes hold a
+// plane (x fastest) and, in 3D, the wave's four rows the planes.  The other
+// values of a line come by lane exchange instead of LDS: rotations of the quad
+// (x) and of the row by four lanes (y), and the swaps of half waves and of rows
+// for z.  A cell's lanes are all active or none.  Costs 6 to 12 register moves a
+// value where LDS takes 4 accesses and their waits: bound by FP64 issue instead
+// of LDS; predictor in FP64 at 35^3 0.398 (0.573 node-column) -> 0.375 ms and
+// in 2D at 27^2, where the waits dominate, 15.8 -> 12.1 us, in FP32 at 45^3
+// 0.480 -> 0.447 ms.
+template <int CTRL, typename R>
+__device__ __forceinline__ R dpp(R v) {
+  if constexpr (sizeof(R) == 8) {
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(b), CTRL, 0xf, 0xf, true);
+    const unsigned hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(b >> 32), CTRL, 0xf, 0xf, true);
+    return __builtin_bit_cast(R, (static_cast<unsigned long long>(hi) << 32) | lo);
+  } else {
+    return __builtin_bit_cast(R, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+  }
+}
+constexpr int quad_rotate(int k) {  // lane i of a quad takes lane (i + k) % 4
+  return (k & 3) | ((1 + k) & 3) << 2 | ((2 + k) & 3) << 4 | ((3 + k) & 3) << 6;
+}
+constexpr int row_take(int n) { return 0x120 + 16 - n; }  // lane i of a row takes lane (i + n) % 16
+
+// The values of the four rows at this lane's place in its row, in every row.
+__device__ __forceinline__ void all_rows(unsigned v, unsigned (&r)[4]) {
+  const auto h = __builtin_amdgcn_permlane32_swap(v, v, false, false);  // rows 0 1 0 1 and 2 3 2 3
+  const auto a = __builtin_amdgcn_permlane16_swap(h[0], h[0], false, false);
+  const auto b = __builtin_amdgcn_permlane16_swap(h[1], h[1], false, false);
+  r[0] = a[0];
+  r[1] = a[1];
+  r[2] = b[0];
+  r[3] = b[1];
+}
+template <typename R>
+__device__ __forceinline__ void all_rows(R v, R (&r)[4]) {
+  if constexpr (sizeof(R) == 8) {
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+    unsigned lo[4], hi[4];
+    all_rows(static_cast<unsigned>(b), lo);
+    all_rows(static_cast<unsigned>(b >> 32), hi);
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      r[i] = __builtin_bit_cast(R, (static_cast<unsigned long long>(hi[i]) << 32) | lo[i]);
+  } else {
+    unsigned w[4];
+    all_rows(__builtin_bit_cast(unsigned, v), w);
+#pragma unroll
+    for (int i = 0; i < 4; i++) r[i] = __builtin_bit_cast(R, w[i]);
+  }
+}
 
 // Component of the Euler flux that F_d[v] shares with an earlier direction
 // (the momentum fluxes are symmetric: F_d[1+e] = F_e[1+d]).
@@ -236,28 +284,30 @@ template <int D, int B, int V, int NP, typename R, bool CG, bool EU>
 struct Tile {
   using S = Shape<D, B, V, NP, R>;
   static constexpr int ND = S::ND, NS = S::NS, NF = S::NF, NL = S::NL, CPB = S::CPB, THREADS = S::THREADS,
-                       SLICE = S::SLICE, TS = S::TS, LS = S::LS, VS = CPB * NL * LS;
+                       SLICE = S::SLICE, TS = S::TS, VS = CPB * NL * B;
 
   // Two waves per SIMD leave the registers for the average in the loop (CERK at
   // 40^3, order 5: 2.02 -> 1.86 ms); the other shapes run at three or four.
   static constexpr bool FHL = sizeof(R) == 8 && B >= 5;
+
+  static constexpr bool LANES = S::LANES;
 
   static __device__ __forceinline__ bool keep(int d, int v) { return !EU || euler_canonical(D, d, v); }
 
   // The line tasks of n slices: contract every line of the buffer in place,
   // the next line of a lane on its way while this one is contracted.
   static __device__ __forceinline__ void lines(R* buf, int n, const DevTables* __restrict__ T) {
-    const int last = n * (SLICE / LS);
+    const int last = n * (SLICE / B);
     const EvenOdd<R, B> M(opaque(tab_dudx<R>(T)));
     int id = threadIdx.x;
     R f[B], o[B];
-    if (id < last) load_line<R, B, LS>(buf + id * LS, f);
+    if (id < last) load_line<R, B>(buf + id * B, f);
 #pragma unroll 1
     while (id < last) {
       M.apply(f, o);
       const int next = id + THREADS;
-      if (next < last) load_line<R, B, LS>(buf + next * LS, f);
-      store_line<R, B, LS>(buf + id * LS, o);
+      if (next < last) load_line<R, B>(buf + next * B, f);
+      store_line<R, B>(buf + id * B, o);
       id = next;
     }
   }
@@ -282,7 +332,7 @@ struct Tile {
 #pragma unroll
     for (int d = 0; d < D; d++) {
       line[d] = cs * NL + d * NF + (D == 3 ? (d == 0 ? z * B + y : (d == 1 ? z * B + x : y * B + x)) : (d == 0 ? y : x));
-      off[d] = line[d] * LS + (d == 0 ? x : (d == 1 ? y : z));
+      off[d] = line[d] * B + (d == 0 ? x : (d == 1 ? y : z));
     }
     R* slab = reinterpret_cast<R*>(buf);
     const double dt = dtp[(cinst && valid) ? cinst[cell] : 0];
@@ -313,8 +363,50 @@ struct Tile {
         g[v] = a;
       }
     };
+    // LANES: row c_d of dt / dx_d dudx; x and y from the node's own entry on round
+    // the line, z from plane 0
+    R cl[LANES ? D : 1][4];
+    if constexpr (LANES) {
+#pragma unroll
+      for (int d = 0; d < D; d++) {
+        const int c = d == 0 ? x : (d == 1 ? y : z);
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+          cl[d][k] = cd[d] * (sizeof(R) == 8 ? static_cast<R>(T->dudx[c * B + (d == 2 ? k : (c + k) % B)])
+                                             : static_cast<R>(T->dudxf[c * B + (d == 2 ? k : (c + k) % B)]));
+      }
+    }
+    // dt times the divergence of the flux F by lane exchange
+    auto exchange = [&](const R(&F)[D][V], R(&g)[V]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int v = 0; v < V; v++) {
+        R a = cl[0][0] * F[0][v];
+        a += cl[0][1] * dpp<quad_rotate(1)>(F[0][v]);
+        a += cl[0][2] * dpp<quad_rotate(2)>(F[0][v]);
+        a += cl[0][3] * dpp<quad_rotate(3)>(F[0][v]);
+        a += cl[1][0] * F[1][v];
+        a += cl[1][1] * dpp<row_take(4)>(F[1][v]);
+        a += cl[1][2] * dpp<row_take(8)>(F[1][v]);
+        a += cl[1][3] * dpp<row_take(12)>(F[1][v]);
+        if constexpr (D == 3) {
+          R r[4];
+          all_rows(F[D - 1][v], r);
+#pragma unroll
+          for (int k = 0; k < 4; k++) a += cl[D - 1][k] * r[k];
+        }
+        asm volatile("" : "+v"(a));  // formed here: sunk to its use, it would keep the exchanged values alive
+        g[v] = a;
+      }
+    };
     // dt times the flux divergence of the one state Q at the node
-    auto divergence = [&](const R* Q, R(&F)[D][V], R(&g)[V]) {
+    auto divergence = [&](const R* Q, R(&F)[D][V], R(&g)[V]) __attribute__((always_inline)) {
+      if constexpr (LANES) {
+        if (valid) {
+          flux<D, V, R, EU>(P, Q, F);
+          exchange(F, g);
+        }
+        return;
+      }
       if (valid) {
         flux<D, V, R, EU>(P, Q, F);
         publish(0, F);
@@ -449,23 +541,35 @@ struct Tile {
 #pragma unroll
           for (int v = 0; v < V; v++) q[t][v] = g[t][v];
       }
-#pragma unroll
-      for (int t0 = 0; t0 < B; t0 += TS) {
+      if constexpr (LANES) {
         if (active) {
 #pragma unroll
-          for (int t = t0; t < t0 + TS && t < B; t++) {
+          for (int t = 0; t < B; t++) {
             R F[D][V];
             flux<D, V, R, EU>(P, q[t], F);
-            if constexpr (FHL) average(t, F);
-            publish(t - t0, F);
+            exchange(F, g[t]);
+            __builtin_amdgcn_sched_barrier(0);  // slices one after the other: interleaved, they spill
           }
         }
-        __syncthreads();
-        lines(slab, t0 + TS <= B ? TS : B - t0, T);
-        __syncthreads();
-        if (active) {
+      } else {
 #pragma unroll
-          for (int t = t0; t < t0 + TS && t < B; t++) gather(t - t0, g[t]);
+        for (int t0 = 0; t0 < B; t0 += TS) {
+          if (active) {
+#pragma unroll
+            for (int t = t0; t < t0 + TS && t < B; t++) {
+              R F[D][V];
+              flux<D, V, R, EU>(P, q[t], F);
+              if constexpr (FHL) average(t, F);
+              publish(t - t0, F);
+            }
+          }
+          __syncthreads();
+          lines(slab, t0 + TS <= B ? TS : B - t0, T);
+          __syncthreads();
+          if (active) {
+#pragma unroll
+            for (int t = t0; t < t0 + TS && t < B; t++) gather(t - t0, g[t]);
+          }
         }
       }
       // time solve in place and squared update (variables only; parameters are carried)
@@ -514,7 +618,7 @@ struct Tile {
 
     // ---- time averages -> LDS (FP64): the fluxes as lines, the states by node ----
     double* Fl = reinterpret_cast<double*>(buf);
-    double* Qh = Fl + S::END + cs * NS * ND;
+    double* Qh = Fl + SLICE + cs * NS * ND;
     int end[D];
 #pragma unroll
     for (int d = 0; d < D; d++) end[d] = line[d] * V * B + (d == 0 ? x : (d == 1 ? y : z));
@@ -554,7 +658,7 @@ struct Tile {
 #pragma unroll 1
       for (int id = tid; id < CPB * NLV; id += THREADS) {
         double f[B], o[B];
-        load_line<double, B, B>(Fl + id * B, f);
+        load_line<double, B>(Fl + id * B, f);
         double f0 = 0.0, f1 = 0.0;
 #pragma unroll
         for (int l = 0; l < B; l++) {
@@ -562,7 +666,7 @@ struct Tile {
           f1 += f[l] * T->F1[l];
         }
         M.apply(f, o);
-        store_line<double, B, B>(Fl + id * B, o);
+        store_line<double, B>(Fl + id * B, o);
         const int c = CPB == 1 ? 0 : id / NLV;
         const int r = id - c * NLV;
         const int d = r / NFV;
@@ -633,10 +737,10 @@ struct Tile {
 
 // Waves per SIMD the register allocation aims at: the two columns (2 B V values)
 // and a line's working set; one wave more spills (FP64 order 5 at three: 52
-// registers, 24 -> 30 ms at 81^3).
+// registers, 24 -> 30 ms at 81^3; order 3 at three: 27, 0.375 -> 0.390 ms at 35^3).
 template <int D, int B, int V, int NP, typename R>
 constexpr int min_waves() {
-  return sizeof(R) == 8 ? (B >= 5 ? 2 : 3) : 4;
+  return sizeof(R) == 8 ? (B >= 4 ? 2 : 3) : 4;
 }
 
 // One workgroup per tile of CPB cells, or a smaller grid that loops over the tiles.
