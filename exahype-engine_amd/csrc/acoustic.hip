@@ -73,6 +73,28 @@ __device__ __forceinline__ void taylor(double dt, double (&a)[B]) {
   }
 }
 
+// Riemann fluctuation of the own side of face (d, o) of a cell (o = 1: the cell is
+// the left state): FL = acc - smax qd on the left, FR = acc + smax qd on the right.
+// One function with its fused operations spelled out, so that the corrector and
+// the fused step give the same bits.
+__device__ __forceinline__ void ac_fluctuation(int d, int o, const double4& qo, const double4& qn, double rho_o,
+                                               double c_o, double rho_n, double c_n, double (&fl)[4]) {
+  const double4 QL = o ? qo : qn, QR = o ? qn : qo;
+  const double cL = o ? c_o : c_n, cR = o ? c_n : c_o;
+  const double aL = fabs(cL), aR = fabs(cR);
+  const double smax = aL > aR ? aL : aR;
+  const double rhoa = 0.5 * ((o ? rho_n : rho_o) + (o ? rho_o : rho_n));
+  const double ca = 0.5 * (cR + cL);
+  const double lama = rhoa * ca * ca, irhoa = 1.0 / rhoa;
+  const double qd[4] = {0.5 * (QR.x - QL.x), 0.5 * (QR.y - QL.y), 0.5 * (QR.z - QL.z), 0.5 * (QR.w - QL.w)};
+  const double qdn = d == 0 ? qd[1] : (d == 1 ? qd[2] : qd[3]);
+  const double s = o ? -smax : smax;
+  const double ncp = irhoa * (-qd[0]);  // non-conservative product, times 1/rho
+  fl[0] = __builtin_fma(s, qd[0], lama * (-qdn));  // flux, times lambda
+#pragma unroll
+  for (int v = 1; v < 4; v++) fl[v] = __builtin_fma(s, qd[v], v == 1 + d ? ncp : 0.0);
+}
+
 // ---------------------------------------------------------------------------
 // forward predictor (+ volume update when UPDATE)
 // ---------------------------------------------------------------------------
@@ -192,12 +214,14 @@ struct AcLineShape {
   static constexpr int N = B * B * B;
   static constexpr int F = B * B;    // lines per cell
   static constexpr int BUF = 3 * N;  // p, v, w of one level
+  // LDS values per cell: two level buffers, before them the fluctuations of the six faces
+  static constexpr int LDS = 2 * BUF > 24 * F ? 2 * BUF : 24 * F;
   // small workgroups: more of them fit beside each other on a CU, so that one
   // computes while another waits at a barrier or for HBM (order 4 at 54^3: 256
   // lanes 0.709, 128 lanes 0.639, 64 lanes, of which 50 have a line, 0.691 ms)
   static constexpr int THREADS = B <= 4 ? 64 : 128;
   static constexpr int CPB_T = THREADS / F;
-  static constexpr int CPB_L = (60 * 1024) / (2 * BUF * 8);  // two level buffers per cell
+  static constexpr int CPB_L = (60 * 1024) / (LDS * 8);
   static constexpr int CPB = CPB_T < CPB_L ? CPB_T : CPB_L;    // cells per block
 };
 
@@ -258,17 +282,24 @@ __device__ __forceinline__ void line_derivatives(const double* __restrict__ Dm, 
 // factors f_0 = dt/2, f_{k+1} = f_k dt/(k+2) (:196, :346-353), source terms
 // s_k of the per-step row {sigma0, s_0..s_{B-1}}; the volume update is
 // dt * A(qh) - sigma0 g with that A (:474-640).
-template <int B, bool UPDATE, bool SPLIT>
+// CORR: the kernel starts with the corrector of the step before (face fluctuations
+// from qb, face part of the update; ac_corrector_kernel) and writes its faces to
+// qb_out, because neighbours still read qb: between two steps u then stays in
+// registers.  The corrected p of a cell with receivers goes to rec_p.  Bound by
+// HBM (u in and out, own faces in, neighbours' from the caches, faces out: 2.8 GB
+// at 54^3 of order 4 where predictor and corrector move 4.0) and the LDS reads of the levels: 0.95 ms a step
+// there instead of 0.64 + 0.40.
+template <int B, bool UPDATE, bool SPLIT, bool CORR = false>
 __global__ void __launch_bounds__((AcLineShape<B>::THREADS), 2) ac_predict_lines_kernel(AcousticArgs a) {
   using S = AcLineShape<B>;
   constexpr int N = S::N, F = S::F, CPB = S::CPB;
-  __shared__ double sbuf[2][CPB][S::BUF];
+  __shared__ double smem[CPB * S::LDS];
   const int t = threadIdx.x;
   const int lc = t / F, ln = t - lc * F;
   const int z = ln / B, y = ln - z * B;
   const long cell = long(blockIdx.x) * CPB + lc;
   const bool slot = lc < CPB;
-  const int cs = slot ? lc : 0;
+  double* cellbuf = smem + (slot ? lc : 0) * S::LDS;
   const bool on = slot && cell < a.ncells;
   const double invh = 1.0 / a.h;
   const double* Dm = a.tab->dudx;  // dudx[i][m]
@@ -289,6 +320,68 @@ __global__ void __launch_bounds__((AcLineShape<B>::THREADS), 2) ac_predict_lines
   } else {
 #pragma unroll
     for (int x = 0; x < B; x++) P[x] = U[x] = Vv[x] = Wv[x] = 0.0;
+  }
+  if constexpr (CORR) {
+    // face node ln of every face, fluctuations to LDS [face][node][4]
+    if (on) {
+      const unsigned n = a.n, c32 = static_cast<unsigned>(cell), iz = c32 / (n * n), rem = c32 - iz * n * n,
+                     iy = rem / n, ix = rem - iy * n;
+      const unsigned at[3] = {ix, iy, iz}, stride[3] = {1, n, n * n};
+#pragma unroll
+      for (int f = 0; f < 6; f++) {
+        const int d = f >> 1, o = f & 1;
+        const unsigned i = at[d];
+        const long nb = o ? (i + 1 == n ? cell - long(i) * stride[d] : cell + stride[d])
+                          : (i == 0 ? cell + long(n - 1) * stride[d] : cell - stride[d]);
+        const double rho_n = a.mat[2 * nb], c_n = a.mat[2 * nb + 1];
+        const double4 qo = reinterpret_cast<const double4*>(a.qb)[(cell * 6 + f) * F + ln];
+        const double4 qn = reinterpret_cast<const double4*>(a.qb)[(nb * 6 + (f ^ 1)) * F + ln];
+        double fl[4];
+        ac_fluctuation(d, o, qo, qn, rho, c, rho_n, c_n, fl);
+#pragma unroll
+        for (int v = 0; v < 4; v++) cellbuf[(f * F + ln) * 4 + v] = fl[v];
+      }
+    }
+    __syncthreads();
+    if (on) {
+      const double dth = a.dt / a.h;
+      const double *F0 = a.tab->F0, *F1 = a.tab->F1, *w = a.tab->w;
+      const double cy[2] = {dth * F0[y] / w[y], dth * F1[y] / w[y]}, cz[2] = {dth * F0[z] / w[z], dth * F1[z] / w[z]};
+#pragma unroll
+      for (int x = 0; x < B; x++) {
+        double du[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (int f = 0; f < 6; f++) {
+          const int d = f >> 1, o = f & 1;
+          const double cf = d == 0 ? dth * (o ? F1[x] : F0[x]) / w[x] : (d == 1 ? cy[o] : cz[o]);
+          const double* fl = cellbuf + (f * F + (d == 0 ? ln : (d == 1 ? z * B + x : y * B + x))) * 4;
+#pragma unroll
+          for (int v = 0; v < 4; v++) du[v] -= cf * fl[v];
+        }
+        P[x] += du[0];
+        U[x] += du[1];
+        Vv[x] += du[2];
+        Wv[x] += du[3];
+      }
+      if (a.rec_p) {
+        const int r0 = a.rstart[cell];
+        if (a.rstart[cell + 1] > r0) {
+#pragma unroll
+          for (int x = 0; x < B; x++) a.rec_p[long(r0) * N + ln * B + x] = P[x];
+        }
+      }
+    }
+    __syncthreads();  // the fluctuations are read: the level buffers take their place
+  }
+  double p0[CORR ? 4 : 1][CORR ? B : 1];  // CORR: the corrected state, for the update at the end
+  if constexpr (CORR) {
+#pragma unroll
+    for (int x = 0; x < B; x++) {
+      p0[0][x] = P[x];
+      p0[1][x] = U[x];
+      p0[2][x] = Vv[x];
+      p0[3][x] = Wv[x];
+    }
   }
   const double lam = rho * c * c, irho = SPLIT ? 1.0 : 1.0 / rho;
   const int step = a.step_override >= 0 ? a.step_override : *a.step_ptr;
@@ -311,7 +404,7 @@ __global__ void __launch_bounds__((AcLineShape<B>::THREADS), 2) ac_predict_lines
   constexpr int LEVELS = SPLIT ? B : B - 1;
 #pragma unroll 1
   for (int i = 0; i < LEVELS; i++) {
-    double* sb = sbuf[i & 1][cs];
+    double* sb = cellbuf + (i & 1) * S::BUF;
     if (slot) {
 #pragma unroll
       for (int x = 0; x < B; x++) {
@@ -339,7 +432,7 @@ __global__ void __launch_bounds__((AcLineShape<B>::THREADS), 2) ac_predict_lines
   }
   // A(qh): the volume update, and qh on the faces
   constexpr int LAST = LEVELS & 1;  // the buffer the last level did not use
-  double* sb = sbuf[LAST][cs];
+  double* sb = cellbuf + LAST * S::BUF;
   if (slot) {
 #pragma unroll
     for (int x = 0; x < B; x++) {
@@ -349,7 +442,7 @@ __global__ void __launch_bounds__((AcLineShape<B>::THREADS), 2) ac_predict_lines
     }
   }
   __syncthreads();  // also: every read of the other buffer (last level) is done
-  double* su = sbuf[LAST ^ 1][cs];
+  double* su = cellbuf + (LAST ^ 1) * S::BUF;
   if (slot) {
 #pragma unroll
     for (int x = 0; x < B; x++) su[ln * B + x] = qh[1][x];
@@ -362,7 +455,11 @@ __global__ void __launch_bounds__((AcLineShape<B>::THREADS), 2) ac_predict_lines
     double4* dst = reinterpret_cast<double4*>(a.u_out) + cell * N + ln * B;
 #pragma unroll
     for (int x = 0; x < B; x++) {
-      const double4 q = old[x];
+      double4 q;
+      if constexpr (CORR)
+        q = make_double4(p0[0][x], p0[1][x], p0[2][x], p0[3][x]);
+      else
+        q = old[x];
       dst[x] = make_double4(q.x + a.dt * (lam * div[x]) - (src ? s0 * gp[x] : 0.0), q.y + a.dt * (irho * px[x]),
                             q.z + a.dt * (irho * py[x]), q.w + a.dt * (irho * pz[x]));
     }
@@ -371,7 +468,7 @@ __global__ void __launch_bounds__((AcLineShape<B>::THREADS), 2) ac_predict_lines
   if (on) {
     const double* F0 = a.tab->F0;
     const double* F1 = a.tab->F1;
-    double4* qb = reinterpret_cast<double4*>(a.qb) + cell * 6 * F;
+    double4* qb = reinterpret_cast<double4*>(a.qb_out) + cell * 6 * F;
     // x-faces, node (z, y) = ln, from registers
     double l0[4] = {0, 0, 0, 0}, l1[4] = {0, 0, 0, 0};
 #pragma unroll
@@ -432,20 +529,9 @@ __global__ void __launch_bounds__(kAcThreads) ac_corrector_kernel(AcousticArgs a
       const double rho_n = a.mat[2 * nb], c_n = a.mat[2 * nb + 1];
       const double4 qo = reinterpret_cast<const double4*>(a.qb)[(cell * 6 + f) * F + fn];
       const double4 qn = reinterpret_cast<const double4*>(a.qb)[(nb * 6 + (f ^ 1)) * F + fn];
-      // own face o = 1: own cell is the left state; o = 0: own cell is the right state
-      const double4 QL = o ? qo : qn, QR = o ? qn : qo;
-      const double cL = o ? c_o : c_n, cR = o ? c_n : c_o;
-      const double aL = fabs(cL), aR = fabs(cR);
-      const double smax = aL > aR ? aL : aR;
-      const double rhoa = 0.5 * ((o ? rho_n : rho_o) + (o ? rho_o : rho_n));
-      const double ca = 0.5 * (cR + cL);
-      const double lama = rhoa * ca * ca, irhoa = 1.0 / rhoa;
-      double qd[4] = {0.5 * (QR.x - QL.x), 0.5 * (QR.y - QL.y), 0.5 * (QR.z - QL.z), 0.5 * (QR.w - QL.w)};
-      double accv[4] = {0, 0, 0, 0};
-      accv[1 + d] += irhoa * (-qd[0]);  // non-conservative product, times 1/rho
-      accv[0] += lama * (-qd[1 + d]);   // flux, times lambda
-      const double sgn = o ? -1.0 : 1.0;  // FL = acc - smax qd, FR = acc + smax qd
-      for (int v = 0; v < 4; v++) sFl[lc][f][fn][v] = accv[v] + sgn * smax * qd[v];
+      double fl[4];
+      ac_fluctuation(d, o, qo, qn, rho_o, c_o, rho_n, c_n, fl);
+      for (int v = 0; v < 4; v++) sFl[lc][f][fn][v] = fl[v];
     }
   }
   __syncthreads();
@@ -470,13 +556,16 @@ __global__ void __launch_bounds__(kAcThreads) ac_corrector_kernel(AcousticArgs a
 }
 
 // ---------------------------------------------------------------------------
-// receivers: rec[step][r] = sum_node p * weight (one wave per receiver)
+// receivers: rec[step][r] = sum_node p * weight (one wave per receiver); p from u
+// or, after a fused step, from rec_p [first receiver of the cell][node]
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(64) ac_receivers_kernel(AcousticArgs a, int N) {
   const int r = blockIdx.x, lane = threadIdx.x;
   const long cell = a.rcell[r];
+  const double* p = a.rec_p ? a.rec_p + long(a.rstart[cell]) * N : a.u + cell * N * 4;
+  const int stride = a.rec_p ? 1 : 4;
   double s = 0.0;
-  for (int nd = lane; nd < N; nd += 64) s += a.u[(cell * N + nd) * 4] * a.rw[long(r) * N + nd];
+  for (int nd = lane; nd < N; nd += 64) s += p[nd * stride] * a.rw[long(r) * N + nd];
   for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
   const int step = a.step_override >= 0 ? a.step_override : *a.step_ptr;
   if (lane == 0) a.rec[long(step) * a.nrec + r] = s;
@@ -791,6 +880,13 @@ int launch_all(int which, const AcousticArgs& a, hipStream_t s) {
         ac_predict_lines_kernel<B, true, false><<<lblocks, AcLineShape<B>::THREADS, 0, s>>>(a);
       else
         ac_predict_kernel<B, true><<<blocks, kAcThreads, 0, s>>>(a);
+      break;
+    case kAcStep:
+      if (a.pred_variant != 0) return -1;  // the x-line form
+      if (a.split_ck)
+        ac_predict_lines_kernel<B, true, true, true><<<lblocks, AcLineShape<B>::THREADS, 0, s>>>(a);
+      else
+        ac_predict_lines_kernel<B, true, false, true><<<lblocks, AcLineShape<B>::THREADS, 0, s>>>(a);
       break;
     case kAcPredictFaces:
       if (a.split_ck) return -1;  // the adjoint sweeps transpose the generic predictor only

@@ -44,6 +44,7 @@ struct exa_acoustic {
   int step = 0;  // host mirror of the device step counter
   hipStream_t stream = nullptr;
   double *d_u = nullptr, *d_mat = nullptr, *d_qb = nullptr;
+  double *d_qb2 = nullptr, *d_rec_p = nullptr;  // fused steps: the other face buffer, p at the receivers' cells
   double *d_ubar = nullptr, *d_fbar = nullptr, *d_fbar2 = nullptr, *d_gc = nullptr;
   int* d_step = nullptr;
   std::vector<double> mat;  // host copy of (rho, c) per cell
@@ -224,6 +225,7 @@ exa::AcousticArgs args(exa_acoustic* ac, double* u) {
   a.ubar = ac->d_ubar;
   a.fbar = ac->d_fbar;
   a.u_out = u;
+  a.qb_out = ac->d_qb;
   a.rstart = ac->d_rstart;
   a.rorder = ac->d_rorder;
   a.gc = ac->d_gc;
@@ -253,8 +255,46 @@ int enqueue_forward(exa_acoustic* ac, double* u, double* u_out, int step, double
   return EXA_OK;
 }
 
+// nsteps forward steps on d_u from step s0, receivers as enqueue_forward: the
+// corrector of a step and the predictor of the next run as one kernel.
+int enqueue_forward_steps(exa_acoustic* ac, int s0, int nsteps, double* rec) {
+  if (nsteps < 2 || ac->pred_variant != 0) {
+    for (int i = 0; i < nsteps; i++) RC_OK(enqueue_forward(ac, ac->d_u, ac->d_u, s0 + i, rec));
+    return EXA_OK;
+  }
+  if (!ac->d_qb2) HIP_OK(hipMalloc(&ac->d_qb2, sizeof(double) * ac->nc * 6 * ac->F * 4), "hipMalloc(faces)");
+  const bool receive = rec && ac->nrec > 0;
+  if (receive && !ac->d_rec_p) HIP_OK(hipMalloc(&ac->d_rec_p, sizeof(double) * ac->nrec * ac->N), "hipMalloc(receivers)");
+  exa::TraceRange tr("exa.acoustic.steps");
+  const int o = ac->k.order;
+  exa::AcousticArgs a = args(ac, ac->d_u);
+  a.step_override = s0;
+  RC_OK(status(exa::launch_acoustic(exa::kAcPredictUpdate, o, a, ac->stream), "acoustic predictor"));
+  for (int i = 1; i < nsteps; i++) {
+    a = args(ac, ac->d_u);
+    a.qb_out = ac->d_qb2;
+    a.step_override = s0 + i;
+    a.rec_p = receive ? ac->d_rec_p : nullptr;
+    RC_OK(status(exa::launch_acoustic(exa::kAcStep, o, a, ac->stream), "acoustic step"));
+    std::swap(ac->d_qb, ac->d_qb2);
+    if (receive) {
+      a.step_override = s0 + i - 1;
+      a.rec = rec;
+      RC_OK(status(exa::launch_acoustic(exa::kAcReceivers, o, a, ac->stream), "acoustic receivers"));
+    }
+  }
+  a = args(ac, ac->d_u);
+  a.step_override = s0 + nsteps - 1;
+  RC_OK(status(exa::launch_acoustic(exa::kAcCorrector, o, a, ac->stream), "acoustic corrector"));
+  if (receive) {
+    a.rec = rec;
+    RC_OK(status(exa::launch_acoustic(exa::kAcReceivers, o, a, ac->stream), "acoustic receivers"));
+  }
+  return EXA_OK;
+}
+
 void free_acoustic(exa_acoustic* ac) {
-  double* bufs[] = {ac->d_u,     ac->d_mat,   ac->d_qb,     ac->d_ubar,  ac->d_fbar, ac->d_fbar2,
+  double* bufs[] = {ac->d_qb2,   ac->d_rec_p, ac->d_u,     ac->d_mat,   ac->d_qb,     ac->d_ubar,  ac->d_fbar, ac->d_fbar2,
                     ac->d_gc,    ac->d_src_g, ac->d_src_tab, ac->d_rw,   ac->d_rec,  ac->d_res};
   for (double* b : bufs)
     if (b) (void)hipFree(b);
@@ -472,6 +512,8 @@ int exa_acoustic_set_receivers(exa_acoustic* ac, int nrec, const double* xr) {
     if (p) (void)hipFree(p);
   if (ac->d_rw) (void)hipFree(ac->d_rw);
   ac->d_rcell = ac->d_rstart = ac->d_rorder = nullptr;
+  if (ac->d_rec_p) (void)hipFree(ac->d_rec_p);
+  ac->d_rec_p = nullptr;
   ac->d_rw = nullptr;
   ac->nrec = 0;
   if (nrec == 0) return EXA_OK;
@@ -552,10 +594,12 @@ int exa_acoustic_run(exa_acoustic* ac, int nsteps, int use_graph, double* rec) {
       }
       ac->timed_steps = nsteps;
     }
-    for (int i = 0; !rc && i < nsteps; i++) {
-      rc = enqueue_forward(ac, ac->d_u, ac->d_u, s0 + i, ac->d_rec - long(s0) * ac->nrec,
-                           ac->timing ? &ac->ev[size_t(3) * i] : nullptr);
-    }
+    double* rec_base = ac->d_rec - long(s0) * ac->nrec;
+    if (!ac->timing)
+      rc = enqueue_forward_steps(ac, s0, nsteps, rec_base);
+    else  // predictor and corrector apart, to time each
+      for (int i = 0; !rc && i < nsteps; i++)
+        rc = enqueue_forward(ac, ac->d_u, ac->d_u, s0 + i, rec_base, &ac->ev[size_t(3) * i]);
   }
   if (!rc) {
     const hipError_t e = hipEventRecord(e1, ac->stream);
@@ -617,13 +661,11 @@ int exa_acoustic_misfit_gradient(exa_acoustic* ac, int nsteps, int every, const 
   // forward sweep with checkpoints
   if (!rc && hipEventRecord(ev[0], ac->stream) != hipSuccess) rc = fail(hipErrorUnknown, "event");
   exa::TraceRange tr_fwd("exa.acoustic.adjoint.forward");
-  for (int k = 0; !rc && k < K; k++) {
-    if (k % every == 0) {
-      const hipError_t e = hipMemcpyAsync(d_ck + su * (k / every), ac->d_u, sizeof(double) * su,
-                                          hipMemcpyDeviceToDevice, ac->stream);
-      if (e != hipSuccess) rc = fail(e, "checkpoint");
-    }
-    if (!rc) rc = enqueue_forward(ac, ac->d_u, ac->d_u, s0 + k, rec_base);
+  for (int k = 0; !rc && k < K; k += seg + 1) {
+    const hipError_t e = hipMemcpyAsync(d_ck + su * (k / every), ac->d_u, sizeof(double) * su,
+                                        hipMemcpyDeviceToDevice, ac->stream);
+    if (e != hipSuccess) rc = fail(e, "checkpoint");
+    if (!rc) rc = enqueue_forward_steps(ac, s0 + k, k + every < K ? every : K - k, rec_base);
   }
   if (!rc && hipEventRecord(ev[1], ac->stream) != hipSuccess) rc = fail(hipErrorUnknown, "event");
   std::vector<double> rec(size_t(K) * R), res(size_t(K) * R);

@@ -281,6 +281,8 @@ struct AcousticArgs {
   double* fbar = nullptr;
   double* fbar_out = nullptr;
   double* u_out = nullptr;
+  double* qb_out = nullptr;  // faces the x-line predictor writes (qb itself but in kAcStep)
+  double* rec_p = nullptr;   // kAcStep: corrected p of the cells with receivers [nrec][B^3], nullptr: none
   // receivers by cell: those of cell c are rorder[rstart[c] .. rstart[c + 1])
   const int* rstart = nullptr;
   const int* rorder = nullptr;
@@ -289,7 +291,8 @@ struct AcousticArgs {
   int pred_variant = 0;  // forward predictor: 0 x-line form, 1 node form
   int split_ck = 0;      // split Cauchy-Kowalevski predictor (x-line form only)
 };
-enum { kAcPredictUpdate = 0, kAcPredictFaces, kAcCorrector, kAcFbar, kAcAdjoint, kAcReceivers };
+// kAcStep: corrector of a step and predictor of the next (step_override) in one kernel
+enum { kAcPredictUpdate = 0, kAcStep, kAcPredictFaces, kAcCorrector, kAcFbar, kAcAdjoint, kAcReceivers };
 bool acoustic_order_supported(int order);
 int launch_acoustic(int which, int order, const AcousticArgs& a, hipStream_t s);
 int launch_acoustic_receivers_adj(int order, const AcousticArgs& a, const double* res, hipStream_t s);

@@ -50,3 +50,27 @@ def test_gradient_at_every_order(order, n, every):
     ref = luh.copy()
     orc.run(ref, n, h, dt, steps, src, rec)
     assert rel_l2(ac.get_solution(), ref) <= 1e-12
+
+
+@pytest.mark.parametrize("order,n", [(1, 1), (2, 1), (2, 2), (3, 2), (4, 1), (4, 2), (5, 1)])
+def test_fused_steps_on_the_smallest_meshes(order, n):
+    """Corrector and next predictor in one kernel where a cell is its own neighbour, or both
+    neighbours of a direction are one cell; receivers in the same cell. <= 1e-12 (the parity bar)."""
+    print(f"[fused steps] order={order} n={n}", flush=True)
+    rng = np.random.default_rng(7 * order + n)
+    h, steps = 1.0 / n, 4
+    c, rho = 1.0 + 0.2 * rng.uniform(-1, 1, n ** 3), 1.0 + 0.1 * rng.uniform(-1, 1, n ** 3)
+    luh = P.acoustic_state(n, order, c, rho, 0.1 * rng.normal(size=(n ** 3, (order + 1) ** 3, 4)))
+    src = ((0.4 * h, 0.6 * h, 0.3 * h), 1.0, 5.0, 0.05)
+    rec = rng.uniform(0.05, 0.95, size=(6, 3))
+    ac = E.Acoustic(E.Context(3, order, 4, 2, E.PDE_ACOUSTIC), n, h)
+    ac.set_solution(luh)
+    ac.set_dt(0.0)
+    dt = ac.time()[2]
+    ac.set_source(*src)
+    ac.set_receivers(rec)
+    got = np.concatenate([ac.run(steps - 1), ac.run(1)])  # fused steps, then a single plain one
+    ref = luh.copy()
+    want, _ = O.LinearOracle(3, order).run(ref, n, h, dt, steps, src, rec)
+    assert rel_l2(got, want) <= 1e-12
+    assert rel_l2(ac.get_solution(), ref) <= 1e-12
