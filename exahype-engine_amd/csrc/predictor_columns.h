@@ -287,8 +287,11 @@ struct Tile {
                        SLICE = S::SLICE, TS = S::TS, VS = CPB * NL * B;
 
   // Two waves per SIMD leave the registers for the average in the loop (CERK at
-  // 40^3, order 5: 2.02 -> 1.86 ms); the other shapes run at three or four.
-  static constexpr bool FHL = sizeof(R) == 8 && B >= 5;
+  // 40^3, order 5: 2.02 -> 1.86 ms); the other shapes run at three or four, order
+  // 4 with a few spilled registers, and gain more from the third wave (batched 3D
+  // order 4 at 23^3, whole step: 518 us at two waves, 539 at three with the
+  // average in the loop, 481 this way; 2D at 243^2 0.220, 0.249 and 0.200 ms).
+  static constexpr bool FHL = sizeof(R) == 8 && B >= 6;
 
   static constexpr bool LANES = S::LANES;
 
@@ -740,7 +743,7 @@ struct Tile {
 // registers, 24 -> 30 ms at 81^3; order 3 at three: 27, 0.375 -> 0.390 ms at 35^3).
 template <int D, int B, int V, int NP, typename R>
 constexpr int min_waves() {
-  return sizeof(R) == 8 ? (B >= 4 ? 2 : 3) : 4;
+  return sizeof(R) == 8 ? (B == 4 || B >= 6 ? 2 : 3) : 4;
 }
 
 // One workgroup per tile of CPB cells, or a smaller grid that loops over the tiles.
