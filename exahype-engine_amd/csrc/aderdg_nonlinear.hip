@@ -1164,22 +1164,26 @@ __global__ __launch_bounds__((Shape<D, B, V, NP>::THREADS)) void corrector_riema
 }
 
 // Single-cell helpers used by the per-cell compatibility entry points.
+// faces [f0, f1) of the cell in order, F the flux of face f0 (the others follow)
 template <int D, int B, int V, int NP>
-__global__ void face_integral_kernel(double* __restrict__ lduh, const double* __restrict__ F, int d, int o,
-                                     double invdx, const DevTables* __restrict__ T) {
+__global__ void face_integral_kernel(double* __restrict__ lduh, const double* __restrict__ F, int f0, int f1,
+                                     double invdx0, double invdx1, double invdx2, const DevTables* __restrict__ T) {
   using S = Shape<D, B, V, NP>;
   constexpr int NS = S::NS;
   const int s = threadIdx.x;
   if (s >= NS) return;
   int z, y, x;
   node_zyx<D, B>(s, z, y, x);
-  const int c = coord<D, B>(d, z, y, x);
-  const int fn = face_node<D, B>(d, z, y, x);
-  const double scaling = invdx * (2.0 * o - 1.0);
-  const double sw = transverse_weight<D>(T->w, d, z, y, x) * scaling;
-  const double fcoef = o ? T->F1[c] : T->F0[c];
+  for (int f = f0; f < f1; f++, F += S::NF * V) {
+    const int d = f >> 1, o = f & 1;
+    const int c = coord<D, B>(d, z, y, x);
+    const int fn = face_node<D, B>(d, z, y, x);
+    const double scaling = (d == 0 ? invdx0 : (d == 1 ? invdx1 : invdx2)) * (2.0 * o - 1.0);
+    const double sw = transverse_weight<D>(T->w, d, z, y, x) * scaling;
+    const double fcoef = o ? T->F1[c] : T->F0[c];
 #pragma unroll
-  for (int v = 0; v < V; v++) lduh[s * V + v] -= sw * fcoef * F[fn * V + v];
+    for (int v = 0; v < V; v++) lduh[s * V + v] -= sw * fcoef * F[fn * V + v];
+  }
 }
 
 template <int D, int B, int V, int NP>
@@ -1309,10 +1313,10 @@ struct Launch {
       return -1;
     }
   }
-  static int face_integral(const KernelCfg& k, hipStream_t st, double* lduh, const double* F, int d, int o,
-                           double invdx) {
-    hipLaunchKernelGGL((face_integral_kernel<D, B, V, NP>), dim3(1), dim3(ceil64(S::NS)), 0, st, lduh, F, d, o,
-                       invdx, k.tab);
+  static int face_integral(const KernelCfg& k, hipStream_t st, double* lduh, const double* F, int f0, int f1,
+                           const double* invdx) {
+    hipLaunchKernelGGL((face_integral_kernel<D, B, V, NP>), dim3(1), dim3(ceil64(S::NS)), 0, st, lduh, F, f0, f1,
+                       invdx[0], invdx[1], invdx[2], k.tab);
     return static_cast<int>(hipGetLastError());
   }
   static int solution_update(const KernelCfg& k, hipStream_t st, double* luh, const double* luhOld,
@@ -1332,7 +1336,7 @@ struct Entry {
                    const double*, double*, int, const LaunchOpts&);
   int (*corrector_riemann)(const KernelCfg&, hipStream_t, long, int, double*, const double*, const double*,
                            const double*, const double*, double*, const LaunchOpts&);
-  int (*face_integral)(const KernelCfg&, hipStream_t, double*, const double*, int, int, double);
+  int (*face_integral)(const KernelCfg&, hipStream_t, double*, const double*, int, int, const double*);
   int (*solution_update)(const KernelCfg&, hipStream_t, double*, const double*, const double*, const double*);
 };
 
@@ -1447,7 +1451,14 @@ int launch_face_integral(const KernelCfg& k, hipStream_t s, double* lduh, const 
                          double invdx) {
   const Entry* e = find_entry(k);
   if (!e) return -1;
-  return e->face_integral(k, s, lduh, F, d, o, invdx);
+  const double inv[3] = {invdx, invdx, invdx};
+  return e->face_integral(k, s, lduh, F, 2 * d + o, 2 * d + o + 1, inv);
+}
+
+int launch_surface_integral(const KernelCfg& k, hipStream_t s, double* lduh, const double* F, const double* invdx) {
+  const Entry* e = find_entry(k);
+  if (!e) return -1;
+  return e->face_integral(k, s, lduh, F, 0, 2 * k.dim, invdx);
 }
 
 int launch_solution_update(const KernelCfg& k, hipStream_t s, double* luh, const double* luhOld,

@@ -33,7 +33,10 @@ struct exa_ctx {
   exa::DevTables* d_tab = nullptr;
   hipStream_t stream = nullptr;
   // scratch for the per-cell compatibility entry points
+  // and its host image in pinned memory: a call lays out its inputs there, copies
+  // them in one piece, and reads its outputs back in one
   double* d_scratch = nullptr;
+  double* h_scratch = nullptr;
   size_t scratch_bytes = 0;
   // point source of the linear path (per-cell predictor)
   bool has_src = false;
@@ -74,10 +77,32 @@ int launch_status(int rc, const char* what) {
 int ensure_scratch(exa_ctx* c, size_t bytes) {
   if (c->scratch_bytes >= bytes) return EXA_OK;
   if (c->d_scratch) (void)hipFree(c->d_scratch);
-  c->d_scratch = nullptr;
+  if (c->h_scratch) (void)hipHostFree(c->h_scratch);
+  c->d_scratch = c->h_scratch = nullptr;
   c->scratch_bytes = 0;
   HIP_OK(hipMalloc(&c->d_scratch, bytes), "hipMalloc(scratch)");
+  HIP_OK(hipHostMalloc(reinterpret_cast<void**>(&c->h_scratch), bytes, hipHostMallocDefault), "hipHostMalloc(scratch)");
   c->scratch_bytes = bytes;
+  return EXA_OK;
+}
+
+// Host image of a scratch position, and the copies of [p, p + n) doubles between
+// the two; from_device waits for the stream.
+double* image(const exa_ctx* c, const void* p) {
+  return c->h_scratch + (static_cast<const double*>(p) - c->d_scratch);
+}
+void put(const exa_ctx* c, double* p, const double* src, size_t n) { std::copy(src, src + n, image(c, p)); }
+void get(const exa_ctx* c, const double* p, double* dst, size_t n) {
+  const double* h = image(c, p);
+  std::copy(h, h + n, dst);
+}
+int to_device(exa_ctx* c, double* p, size_t n) {
+  HIP_OK(hipMemcpyAsync(p, image(c, p), n * sizeof(double), hipMemcpyHostToDevice, c->stream), "copy in");
+  return EXA_OK;
+}
+int from_device(exa_ctx* c, const double* p, size_t n) {
+  HIP_OK(hipMemcpyAsync(image(c, p), p, n * sizeof(double), hipMemcpyDeviceToHost, c->stream), "copy out");
+  HIP_OK(hipStreamSynchronize(c->stream), "sync");
   return EXA_OK;
 }
 
@@ -386,6 +411,7 @@ int exa_ctx_destroy(exa_ctx* c) {
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   if (c->d_guard) (void)hipFree(c->d_guard);
   if (c->d_scratch) (void)hipFree(c->d_scratch);
+  if (c->h_scratch) (void)hipHostFree(c->h_scratch);
   if (c->d_tab) (void)hipFree(c->d_tab);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
@@ -634,41 +660,45 @@ int exa_fusedSpaceTimePredictorVolumeIntegral(exa_ctx* c, double* lduh, double* 
   for (int d = 1; d < D; d++) cubic = cubic && dx[d] == dx[0];
   const size_t nLuh = size_t(NS) * ND, nLduh = size_t(NS) * V;
   const size_t nQb = size_t(2 * D) * NF * ND, nFb = size_t(2 * D) * NF * V;
-  const size_t total = nLuh + nLduh + nQb + nFb + 3 + 1 + 1 + 2;
+  const size_t total = nLuh + 8 + nLduh + nQb + nFb;
   int rc = ensure_scratch(c, total * sizeof(double));
   if (rc) return rc;
+  // inputs, the Picard count, outputs
   double* d_luh = c->d_scratch;
-  double* d_lduh = d_luh + nLuh;
+  double* d_h = d_luh + nLuh;  // dx[D] (one value for cubic cells)
+  double* d_dt = d_h + 3;
+  int* d_guard = reinterpret_cast<int*>(d_dt + 1);  // {count, total, list[1]}
+  int* d_pic = reinterpret_cast<int*>(d_dt + 3);
+  double* d_lduh = d_dt + 4;
   double* d_qb = d_lduh + nLduh;
   double* d_fb = d_qb + nQb;
-  double* d_h = d_fb + nFb;  // dx[D] (one value for cubic cells)
-  double* d_dt = d_h + 3;
-  int* d_pic = reinterpret_cast<int*>(d_dt + 1);
-  int* d_guard = reinterpret_cast<int*>(d_dt + 2);  // {count, total, list[1]}
-  HIP_OK(hipMemcpyAsync(d_luh, luh, nLuh * sizeof(double), hipMemcpyHostToDevice, c->stream), "copy luh");
-  HIP_OK(hipMemcpyAsync(d_h, dx, (cubic ? 1 : D) * sizeof(double), hipMemcpyHostToDevice, c->stream), "copy dx");
-  HIP_OK(hipMemcpyAsync(d_dt, &dt, sizeof(double), hipMemcpyHostToDevice, c->stream), "copy dt");
-  HIP_OK(hipMemsetAsync(d_guard, 0, 2 * sizeof(double), c->stream), "clear guard");
+  put(c, d_luh, luh, nLuh);
+  put(c, d_h, dx, cubic ? 1 : D);
+  put(c, d_dt, &dt, 1);
+  const double clear[2] = {0.0, 0.0};
+  put(c, d_dt + 1, clear, 2);
+  rc = to_device(c, d_luh, nLuh + 6);
+  if (rc) return rc;
   exa::LaunchOpts po;
   po.guard = d_guard;
-  po.hdim = cubic ? 0 : D;  // non-cubic cells: FP64 node-column or slab predictor, dx per direction
+  po.hdim = cubic ? 0 : D;  // non-cubic cells: dx per direction, not the x-line kernels
   rc = launch_status(exa::launch_predictor(c->k, c->stream, 1, d_luh, d_h, d_dt, d_lduh, d_qb, d_fb, d_pic, po),
                      "predictor");
   if (rc) return rc;
   if (!addVolumeIntegralResultToUpdate) {
     // luh += dt/w * volume integral (AbstractGenericADERDGSolverImplementation.template:206-210)
     rc = launch_status(exa::launch_solution_update(c->k, c->stream, d_luh, d_luh, d_lduh, d_dt), "update");
+    if (!rc) rc = from_device(c, d_luh, total);
     if (rc) return rc;
-    HIP_OK(hipMemcpyAsync(luh, d_luh, nLuh * sizeof(double), hipMemcpyDeviceToHost, c->stream), "copy luh");
+    get(c, d_luh, luh, nLuh);
   } else {
-    HIP_OK(hipMemcpyAsync(lduh, d_lduh, nLduh * sizeof(double), hipMemcpyDeviceToHost, c->stream), "copy lduh");
+    rc = from_device(c, d_dt + 3, 1 + nLduh + nQb + nFb);
+    if (rc) return rc;
+    get(c, d_lduh, lduh, nLduh);
   }
-  HIP_OK(hipMemcpyAsync(lQhbnd, d_qb, nQb * sizeof(double), hipMemcpyDeviceToHost, c->stream), "copy lQhbnd");
-  HIP_OK(hipMemcpyAsync(lFhbnd, d_fb, nFb * sizeof(double), hipMemcpyDeviceToHost, c->stream), "copy lFhbnd");
-  int pic = 0;
-  HIP_OK(hipMemcpyAsync(&pic, d_pic, sizeof(int), hipMemcpyDeviceToHost, c->stream), "copy picard");
-  HIP_OK(hipStreamSynchronize(c->stream), "sync");
-  if (picard_iterations) *picard_iterations = pic;
+  get(c, d_qb, lQhbnd, nQb);
+  get(c, d_fb, lFhbnd, nFb);
+  if (picard_iterations) *picard_iterations = *reinterpret_cast<const int*>(image(c, d_dt + 3));
   return EXA_OK;
 }
 
@@ -774,28 +804,27 @@ int exa_riemannSolver(exa_ctx* c, double* FL, double* FR, const double* QL, cons
     return EXA_OK;
   }
   const int NF = nface(c), ND = ndata(c), V = c->k.nvar, D = c->k.dim;
-  // two pseudo cells: cell 0 holds the left state on face 2d+1, cell 1 the right state on face 2d
-  const size_t qcell = size_t(2 * D) * NF * ND, fcell = size_t(2 * D) * NF * V;
-  const size_t total = 2 * qcell + 2 * fcell + 2;
+  // one pseudo cell: the left side on its face 2d+1, the right side on its face 2d
+  const size_t nq = size_t(NF) * ND, nf = size_t(NF) * V;
+  const size_t total = 2 + size_t(2 * D) * (nq + nf);
   int rc = ensure_scratch(c, total * sizeof(double));
   if (rc) return rc;
-  double* d_qb = c->d_scratch;
-  double* d_fb = d_qb + 2 * qcell;
-  int* d_face = reinterpret_cast<int*>(d_fb + 2 * fcell);
+  double* d_face = c->d_scratch;
+  double* d_qb = d_face + 2;
+  double* d_fb = d_qb + size_t(2 * D) * nq;
   const int d = direction;
-  const size_t ql = (size_t(2 * d + 1)) * NF * ND, qr = qcell + size_t(2 * d) * NF * ND;
-  const size_t fl = (size_t(2 * d + 1)) * NF * V, fr = fcell + size_t(2 * d) * NF * V;
-  const int face[4] = {0, 1, d, 0};
-  HIP_OK(hipMemcpyAsync(d_qb + ql, QL, NF * ND * sizeof(double), hipMemcpyHostToDevice, c->stream), "copy QL");
-  HIP_OK(hipMemcpyAsync(d_qb + qr, QR, NF * ND * sizeof(double), hipMemcpyHostToDevice, c->stream), "copy QR");
-  HIP_OK(hipMemcpyAsync(d_fb + fl, FL, NF * V * sizeof(double), hipMemcpyHostToDevice, c->stream), "copy FL");
-  HIP_OK(hipMemcpyAsync(d_fb + fr, FR, NF * V * sizeof(double), hipMemcpyHostToDevice, c->stream), "copy FR");
-  HIP_OK(hipMemcpyAsync(d_face, face, sizeof(face), hipMemcpyHostToDevice, c->stream), "copy face");
-  rc = launch_status(exa::launch_riemann(c->k, c->stream, 1, d_face, d_qb, d_fb), "riemann");
+  const int face[4] = {0, 0, d, 0};
+  std::copy(face, face + 4, reinterpret_cast<int*>(image(c, d_face)));
+  put(c, d_qb + (2 * d + 1) * nq, QL, nq);
+  put(c, d_qb + 2 * d * nq, QR, nq);
+  put(c, d_fb + (2 * d + 1) * nf, FL, nf);
+  put(c, d_fb + 2 * d * nf, FR, nf);
+  rc = to_device(c, d_face, total);
+  if (!rc) rc = launch_status(exa::launch_riemann(c->k, c->stream, 1, reinterpret_cast<int*>(d_face), d_qb, d_fb), "riemann");
+  if (!rc) rc = from_device(c, d_fb + 2 * d * nf, 2 * nf);
   if (rc) return rc;
-  HIP_OK(hipMemcpyAsync(FL, d_fb + fl, NF * V * sizeof(double), hipMemcpyDeviceToHost, c->stream), "copy FL");
-  HIP_OK(hipMemcpyAsync(FR, d_fb + fr, NF * V * sizeof(double), hipMemcpyDeviceToHost, c->stream), "copy FR");
-  HIP_OK(hipStreamSynchronize(c->stream), "sync");
+  get(c, d_fb + (2 * d + 1) * nf, FL, nf);
+  get(c, d_fb + 2 * d * nf, FR, nf);
   return EXA_OK;
 }
 
@@ -959,6 +988,21 @@ int exa_surfaceIntegral(exa_ctx* c, double* lduh, const double* lFhbnd, const do
     return EXA_ERR_ARG;
   }
   const int NF = nface(c), V = c->k.nvar, D = c->k.dim;
+  if (!is_linear(c)) {
+    const size_t nL = size_t(nspace(c)) * V, nF = size_t(2 * D) * NF * V;
+    int rc = ensure_scratch(c, (nL + nF) * sizeof(double));
+    if (rc) return rc;
+    double* d_lduh = c->d_scratch;
+    put(c, d_lduh, lduh, nL);
+    put(c, d_lduh + nL, lFhbnd, nF);
+    double invdx[3] = {1.0 / dx[0], 1.0 / dx[1], D > 2 ? 1.0 / dx[2] : 0.0};
+    rc = to_device(c, d_lduh, nL + nF);
+    if (!rc) rc = launch_status(exa::launch_surface_integral(c->k, c->stream, d_lduh, d_lduh + nL, invdx), "surface integral");
+    if (!rc) rc = from_device(c, d_lduh, nL);
+    if (rc) return rc;
+    get(c, d_lduh, lduh, nL);
+    return EXA_OK;
+  }
   for (int d = 0; d < D; d++)
     for (int o = 0; o < 2; o++) {
       const int rc = exa_faceIntegral(c, lduh, lFhbnd + size_t(2 * d + o) * NF * V, d, o, nullptr, 0, dx, 0.0, 1);
@@ -996,25 +1040,24 @@ int exa_addUpdateToSolution(exa_ctx* c, double* luh, const double* luhOld, const
     return EXA_OK;
   }
   const int NS = nspace(c), ND = ndata(c), V = c->k.nvar;
-  const size_t total = 2 * size_t(NS) * ND + size_t(NS) * V + 1;
-  int rc = ensure_scratch(c, total * sizeof(double));
+  const size_t nL = size_t(NS) * ND, nD = size_t(NS) * V;
+  int rc = ensure_scratch(c, (2 * nL + nD + 1) * sizeof(double));
   if (rc) return rc;
-  double* d_luh = c->d_scratch;
-  double* d_old = d_luh + size_t(NS) * ND;
-  double* d_lduh = d_old + size_t(NS) * ND;
-  double* d_dt = d_lduh + size_t(NS) * V;
-  HIP_OK(hipMemcpyAsync(d_old, luhOld, NS * ND * sizeof(double), hipMemcpyHostToDevice, c->stream), "copy");
-  HIP_OK(hipMemcpyAsync(d_luh, luhOld, NS * ND * sizeof(double), hipMemcpyHostToDevice, c->stream), "copy");
-  HIP_OK(hipMemcpyAsync(d_lduh, lduh, NS * V * sizeof(double), hipMemcpyHostToDevice, c->stream), "copy");
-  HIP_OK(hipMemcpyAsync(d_dt, &dt, sizeof(double), hipMemcpyHostToDevice, c->stream), "copy");
-  rc = launch_status(exa::launch_solution_update(c->k, c->stream, d_luh, d_old, d_lduh, d_dt), "update");
+  double* d_old = c->d_scratch;
+  double* d_lduh = d_old + nL;
+  double* d_dt = d_lduh + nD;
+  double* d_luh = d_dt + 1;
+  put(c, d_old, luhOld, nL);
+  put(c, d_lduh, lduh, nD);
+  put(c, d_dt, &dt, 1);
+  rc = to_device(c, d_old, nL + nD + 1);
+  if (!rc) rc = launch_status(exa::launch_solution_update(c->k, c->stream, d_luh, d_old, d_lduh, d_dt), "update");
+  if (!rc) rc = from_device(c, d_luh, nL);
   if (rc) return rc;
   // parameters of luh are left untouched (solutionUpdate.cpph:55-60 updates variables only)
-  std::vector<double> tmp(size_t(NS) * ND);
-  HIP_OK(hipMemcpyAsync(tmp.data(), d_luh, NS * ND * sizeof(double), hipMemcpyDeviceToHost, c->stream), "copy");
-  HIP_OK(hipStreamSynchronize(c->stream), "sync");
+  const double* got = image(c, d_luh);
   for (int s = 0; s < NS; s++)
-    for (int v = 0; v < V; v++) luh[s * ND + v] = tmp[size_t(s) * ND + v];
+    for (int v = 0; v < V; v++) luh[s * ND + v] = got[size_t(s) * ND + v];
   return EXA_OK;
 }
 
@@ -1056,14 +1099,16 @@ int exa_stableTimeStepSize(exa_ctx* c, const double* luh, const double* dx, doub
   double* d_h = d_luh + size_t(NS) * ND;  // dx[D]
   double* d_out = d_h + 3;
   const double init[4] = {dx[0], D > 1 ? dx[1] : 0.0, D > 2 ? dx[2] : 0.0, DBL_MAX};
-  HIP_OK(hipMemcpyAsync(d_luh, luh, NS * ND * sizeof(double), hipMemcpyHostToDevice, c->stream), "copy");
-  HIP_OK(hipMemcpyAsync(d_h, init, 4 * sizeof(double), hipMemcpyHostToDevice, c->stream), "copy");
+  put(c, d_luh, luh, size_t(NS) * ND);
+  put(c, d_h, init, 4);
+  rc = to_device(c, d_luh, total);
+  if (rc) return rc;
   exa::LaunchOpts o;
   o.hdim = D;  // dx per direction
   rc = launch_status(exa::launch_stable_dt(c->k, c->stream, 1, d_luh, d_h, d_out, o), "stable dt");
+  if (!rc) rc = from_device(c, d_out, 1);
   if (rc) return rc;
-  HIP_OK(hipMemcpyAsync(dt_out, d_out, sizeof(double), hipMemcpyDeviceToHost, c->stream), "copy");
-  HIP_OK(hipStreamSynchronize(c->stream), "sync");
+  get(c, d_out, dt_out, 1);
   return EXA_OK;
 }
 

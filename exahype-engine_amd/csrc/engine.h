@@ -150,6 +150,8 @@ bool corrector_riemann_supported(const KernelCfg& k);
 // Single-cell helper kernels for the compatibility entry points.
 int launch_face_integral(const KernelCfg& k, hipStream_t s, double* lduh, const double* lFface, int direction,
                          int orientation, double invdx_scaled);
+// all 2D faces in order, F [2D][B^(D-1)][V], invdx[3]
+int launch_surface_integral(const KernelCfg& k, hipStream_t s, double* lduh, const double* F, const double* invdx);
 int launch_solution_update(const KernelCfg& k, hipStream_t s, double* luh, const double* luhOld,
                            const double* lduh, const double* dt);
 // Column / line predictor (predictor_columns.h), every compiled shape of the
