@@ -46,6 +46,10 @@ struct exa_acoustic {
   double *d_u = nullptr, *d_mat = nullptr, *d_qb = nullptr;
   double *d_qb2 = nullptr, *d_rec_p = nullptr;  // fused steps: the other face buffer, p at the receivers' cells
   double *d_ubar = nullptr, *d_fbar = nullptr, *d_fbar2 = nullptr, *d_gc = nullptr;
+  // gradient: checkpoints, the states of a segment behind its checkpoint, and the
+  // faces of its steps (optional)
+  double *d_ck = nullptr, *d_seg = nullptr, *d_segq = nullptr;
+  long ck_cap = 0, seg_cap = 0, segq_cap = 0;  // doubles
   int* d_step = nullptr;
   std::vector<double> mat;  // host copy of (rho, c) per cell
   // source
@@ -234,12 +238,42 @@ exa::AcousticArgs args(exa_acoustic* ac, double* u) {
   return a;
 }
 
+// Buffers of one gradient: grown on demand and kept for the next unless they take
+// more than an eighth of the GPU's memory.  The faces of a segment's steps are
+// kept (and not formed a second time) when they fit a quarter of what is free.
+int gradient_buffers(exa_acoustic* ac, size_t su, size_t sq, int nck, int seg) {
+  RC_OK(grow(&ac->d_ck, &ac->ck_cap, long(su) * nck));
+  if (seg > 0) RC_OK(grow(&ac->d_seg, &ac->seg_cap, long(su) * seg));
+  const long faces = long(sq) * (seg + 1);
+  if (ac->segq_cap < faces) {
+    size_t free = 0, total = 0;
+    HIP_OK(hipMemGetInfo(&free, &total), "memory");
+    if (sizeof(double) * size_t(faces) <= free / 4) RC_OK(grow(&ac->d_segq, &ac->segq_cap, faces));
+  }
+  return EXA_OK;
+}
+
+void release_gradient_buffers(exa_acoustic* ac, bool all) {
+  size_t free = 0, total = 0;
+  if (!all && hipMemGetInfo(&free, &total) == hipSuccess &&
+      sizeof(double) * size_t(ac->ck_cap + ac->seg_cap + ac->segq_cap) <= total / 8)
+    return;
+  for (double** p : {&ac->d_ck, &ac->d_seg, &ac->d_segq}) {
+    if (*p) (void)hipFree(*p);
+    *p = nullptr;
+  }
+  ac->ck_cap = ac->seg_cap = ac->segq_cap = 0;
+}
+
 // one forward step from u to u_out (step index `step`, or the device counter if < 0);
-// receivers recorded into rec[(step - rec_base) * nrec + r] when rec != nullptr
-int enqueue_forward(exa_acoustic* ac, double* u, double* u_out, int step, double* rec, hipEvent_t* ev = nullptr) {
+// receivers recorded into rec[(step - rec_base) * nrec + r] when rec != nullptr; the
+// step's faces in qb (nullptr: the mesh's face buffer)
+int enqueue_forward(exa_acoustic* ac, double* u, double* u_out, int step, double* rec, hipEvent_t* ev = nullptr,
+                    double* qb = nullptr) {
   exa::TraceRange tr("exa.acoustic.step");
   exa::AcousticArgs a = args(ac, u);
   a.u_out = u_out;
+  if (qb) a.qb = a.qb_out = qb;
   a.step_override = step;
   const int o = ac->k.order;
   if (ev) HIP_OK(hipEventRecord(ev[0], ac->stream), "event");
@@ -294,7 +328,7 @@ int enqueue_forward_steps(exa_acoustic* ac, int s0, int nsteps, double* rec) {
 }
 
 void free_acoustic(exa_acoustic* ac) {
-  double* bufs[] = {ac->d_qb2,   ac->d_rec_p, ac->d_u,     ac->d_mat,   ac->d_qb,     ac->d_ubar,  ac->d_fbar, ac->d_fbar2,
+  double* bufs[] = {ac->d_ck,    ac->d_seg,   ac->d_segq,  ac->d_qb2,   ac->d_rec_p, ac->d_u,     ac->d_mat,   ac->d_qb,     ac->d_ubar,  ac->d_fbar, ac->d_fbar2,
                     ac->d_gc,    ac->d_src_g, ac->d_src_tab, ac->d_rw,   ac->d_rec,  ac->d_res};
   for (double* b : bufs)
     if (b) (void)hipFree(b);
@@ -645,14 +679,15 @@ int exa_acoustic_misfit_gradient(exa_acoustic* ac, int nsteps, int every, const 
     HIP_OK(hipMalloc(&ac->d_fbar2, sizeof(double) * sq), "hipMalloc(adjoint)");
     HIP_OK(hipMalloc(&ac->d_gc, sizeof(double) * ac->nc), "hipMalloc(adjoint)");
   }
-  double* d_ck = nullptr;
-  double* d_seg = nullptr;
-  HIP_OK(hipMalloc(&d_ck, sizeof(double) * su * nck), "hipMalloc(checkpoints)");
-  hipError_t ea = seg > 0 ? hipMalloc(&d_seg, sizeof(double) * su * seg) : hipSuccess;
-  if (ea != hipSuccess) {
-    (void)hipFree(d_ck);
-    return fail(ea, "hipMalloc(segment)");
+  {
+    const int rb = gradient_buffers(ac, su, sq, nck, seg);
+    if (rb) {
+      release_gradient_buffers(ac, true);
+      return rb;
+    }
   }
+  double *d_ck = ac->d_ck, *d_seg = ac->d_seg;
+  double* d_segq = ac->segq_cap >= long(sq) * (seg + 1) ? ac->d_segq : nullptr;
   std::vector<hipEvent_t> ev(2 + 3 * nck, nullptr);
   int rc = EXA_OK;
   for (auto& e : ev)
@@ -661,11 +696,19 @@ int exa_acoustic_misfit_gradient(exa_acoustic* ac, int nsteps, int every, const 
   // forward sweep with checkpoints
   if (!rc && hipEventRecord(ev[0], ac->stream) != hipSuccess) rc = fail(hipErrorUnknown, "event");
   exa::TraceRange tr_fwd("exa.acoustic.adjoint.forward");
-  for (int k = 0; !rc && k < K; k += seg + 1) {
-    const hipError_t e = hipMemcpyAsync(d_ck + su * (k / every), ac->d_u, sizeof(double) * su,
-                                        hipMemcpyDeviceToDevice, ac->stream);
+  // states k0 .. of segment j (k0 = j every): the checkpoint, then d_seg; their steps' faces
+  auto state = [&](int j, int k) { return k == j * every ? d_ck + su * j : d_seg + su * (k - j * every - 1); };
+  auto faces = [&](int j, int k) { return d_segq ? d_segq + sq * (k - j * every) : nullptr; };
+  for (int j = 0; !rc && j < nck; j++) {
+    const int k0 = j * every;
+    const hipError_t e = hipMemcpyAsync(d_ck + su * j, ac->d_u, sizeof(double) * su, hipMemcpyDeviceToDevice,
+                                        ac->stream);
     if (e != hipSuccess) rc = fail(e, "checkpoint");
-    if (!rc) rc = enqueue_forward_steps(ac, s0 + k, k + every < K ? every : K - k, rec_base);
+    if (!rc && j + 1 < nck) rc = enqueue_forward_steps(ac, s0 + k0, every, rec_base);
+    // the backward sweep starts in the last segment: keep its states
+    for (int k = k0; !rc && j + 1 == nck && k < K; k++)
+      rc = enqueue_forward(ac, state(j, k), k + 1 < K ? state(j, k + 1) : ac->d_u, s0 + k, rec_base, nullptr,
+                           faces(j, k));
   }
   if (!rc && hipEventRecord(ev[1], ac->stream) != hipSuccess) rc = fail(hipErrorUnknown, "event");
   std::vector<double> rec(size_t(K) * R), res(size_t(K) * R);
@@ -692,18 +735,20 @@ int exa_acoustic_misfit_gradient(exa_acoustic* ac, int nsteps, int every, const 
   for (int j = nck - 1; !rc && j >= 0; j--) {
     const int k0 = j * every, k1 = (k0 + every < K) ? k0 + every : K;
     (void)hipEventRecord(ev[2 + 3 * j], ac->stream);
-    // states k0 + 1 .. k1 - 1 of the segment; state k0 is the checkpoint
-    auto state = [&](int k) { return k == k0 ? d_ck + su * j : d_seg + su * (k - k0 - 1); };
-    for (int k = k0; !rc && k < k1 - 1; k++) rc = enqueue_forward(ac, state(k), state(k + 1), s0 + k, nullptr);
+    for (int k = k0; !rc && j + 1 < nck && k < k1 - 1; k++)
+      rc = enqueue_forward(ac, state(j, k), state(j, k + 1), s0 + k, nullptr, nullptr, faces(j, k));
     (void)hipEventRecord(ev[3 + 3 * j], ac->stream);
     for (int k = k1 - 1; !rc && k >= k0; k--) {
-      exa::AcousticArgs a = args(ac, state(k));
+      exa::AcousticArgs a = args(ac, state(j, k));
       a.step_override = s0 + k;
+      if (d_segq) a.qb = a.qb_out = faces(j, k);
       if (k == K - 1) {
         rc = status(exa::launch_acoustic_receivers_adj(o, a, ac->d_res + long(k) * R, ac->stream), "receiver adjoint");
         if (!rc) rc = status(exa::launch_acoustic(exa::kAcFbar, o, a, ac->stream), "adjoint fbar");
       }
-      if (!rc) rc = status(exa::launch_acoustic(exa::kAcPredictFaces, o, a, ac->stream), "acoustic faces");
+      // the faces are there from the segment's steps, all but its last one's
+      if (!rc && (!d_segq || (k == k1 - 1 && j + 1 < nck)))
+        rc = status(exa::launch_acoustic(exa::kAcPredictFaces, o, a, ac->stream), "acoustic faces");
       if (k > 0) a.res_prev = ac->d_res + long(k - 1) * R;
       a.fbar_out = ac->d_fbar2;
       if (!rc) rc = status(exa::launch_acoustic(exa::kAcAdjoint, o, a, ac->stream), "adjoint step");
@@ -732,8 +777,7 @@ int exa_acoustic_misfit_gradient(exa_acoustic* ac, int nsteps, int every, const 
   (void)hipStreamSynchronize(ac->stream);
   for (auto& e : ev)
     if (e) (void)hipEventDestroy(e);
-  (void)hipFree(d_ck);
-  (void)hipFree(d_seg);
+  release_gradient_buffers(ac, false);
   if (rc) return rc;
   *J = Jv;
   return set_step(ac, s0 + K);
