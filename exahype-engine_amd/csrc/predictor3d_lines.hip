@@ -28,7 +28,10 @@
 //   (volumeIntegralNonlinear.cpph:133-223) follow as in the reference.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "engine.h"
+#include "predictor_columns.h"
 
 namespace exa {
 namespace {
@@ -57,17 +60,6 @@ __device__ __forceinline__ const X* opaque(const X* p) {
   const unsigned lo = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(a));
   const unsigned hi = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(a >> 32));
   return reinterpret_cast<const X*>((static_cast<unsigned long long>(hi) << 32) | lo);
-}
-
-// Index of a line's first value in an LDS array, held in a register of its
-// own: the line's reads then differ from it by immediate offsets, and the
-// compiler pairs them into ds_read2_b32 off this one register.  A base it can
-// see through gets folded into the offsets, which overflow ds_read2's 8-bit
-// field, and each pair then costs a vector add for a fresh base.  x lines (B^2
-// points per step) take one per two points.
-__device__ __forceinline__ int line_base(int i) {
-  asm volatile("" : "+v"(i));
-  return i;
 }
 
 // Makes register values opaque to the optimiser at a phase boundary.  Without
@@ -390,6 +382,54 @@ __device__ __forceinline__ void finish_cell(R (&q)[B][LShape<B>::V], R* tl, unsi
   }
 }
 
+// dudx along d applied in place to the d-lines of F_d, for the three directions of
+// f = [3][NS][V] in the LDS point order.  A direction has B B V lines, three
+// wave-rounds of 60 lanes; the nine rounds go round the waves, so a round's
+// direction is wave-uniform and its strides are immediate offsets.  A line's B
+// values are read and written once (the node form before it read the three lines
+// through its node, 15 B values, and its operator rows).  The rows of dudx sum to
+// zero, so it acts on the differences to the line's first value: 35 operations and
+// rounding of the order of the line's variation.  By the mirrored halves of dudx and
+// Kxi, 30 operations, the predictor took 4.58 against 4.75 ms at 81^3, but the state
+// was further from FP64 than with the products (3.8e-8 against 3.5e-8).  Nine rounds on four
+// waves give one of them three: turn moves that one from phase to phase (1 % of the
+// one-iteration kernel at 81^3).
+template <int B>
+__device__ __forceinline__ void contract_lines(float* f, int l, const DevTables* __restrict__ T, int turn) {
+  constexpr int V = 5, NS = B * B * B, LINES = B * B * V, LANES = LINES / 3;
+  static_assert(LINES % 3 == 0 && LANES <= 64 && LANES % (B * V) == 0, "three rounds of whole planes");
+  const auto D = columns::opaque(T->dudxf);
+  const int w = __builtin_amdgcn_readfirstlane(l >> 6), k = l & 63;
+  if (k >= LANES) return;
+  auto line = [&](float* p, auto stride) {
+    constexpr int S = decltype(stride)::value;
+    float a[B], o[B];
+#pragma unroll
+    for (int n = 0; n < B; n++) a[n] = p[n * S];
+#pragma unroll
+    for (int n = 1; n < B; n++) a[n] -= a[0];
+#pragma unroll
+    for (int i = 0; i < B; i++) {
+      o[i] = D[i * B + 1] * a[1];
+#pragma unroll
+      for (int n = 2; n < B; n++) o[i] += D[i * B + n] * a[n];
+    }
+#pragma unroll
+    for (int n = 0; n < B; n++) p[n * S] = o[n];
+  };
+#pragma nounroll
+  for (int r = (w + turn) & 3; r < 9; r += 4) {
+    const int d = r / 3, part = r - 3 * d;
+    if (d == 0)  // x-lines: (z, y, v) contiguous
+      line(f + part * LANES + k, std::integral_constant<int, lds_stride<B>(0) * V>());
+    else if (d == 1)  // y-lines (x, z): B V apart, v contiguous
+      line(f + NS * V + part * (LANES * B) + k + (k / V) * (B * V - V), std::integral_constant<int, lds_stride<B>(1) * V>());
+    else  // z-lines: (y, v) contiguous, x planes apart
+      line(f + 2 * NS * V + part * (LANES * B) + k + (k / (B * V)) * (B * B * V - B * V),
+           std::integral_constant<int, lds_stride<B>(2) * V>());
+  }
+}
+
 // Post-Picard phase of the FP32 kernels, one lane per spatial node s:
 // P = previous iterate, Q = final iterate, both FP32 tiles [t][s][v].
 //   lQhi[s] = sum_t w_t Q[t][s],  lFhi_d[s] = sum_t w_t F_d(P[t][s])
@@ -400,18 +440,18 @@ __device__ __forceinline__ void finish_cell(R (&q)[B][LShape<B>::V], R* tl, unsi
 // point for all three directions.  avg: FP32 LDS scratch of 4 B^3 V values,
 // which may overlap P (it is written after a barrier).
 template <int B>
-__device__ __forceinline__ void finish_from_averages(const float* aq, const float* af, int l, long cell, double dt,
+__device__ __forceinline__ void finish_from_averages(const float* aq, float* af, int l, long cell, double dt,
                                                      double h, int iters, const DevTables* __restrict__ T,
                                                      double* __restrict__ lduh, double* __restrict__ lQhbnd,
                                                      double* __restrict__ lFhbnd, int* __restrict__ picard,
-                                                     double* luh_upd, int nthreads, int f32faces);
+                                                     double* luh_upd, int f32faces);
 
 template <int B>
 __device__ __forceinline__ void finish_cell_points(const float* P, const float* Q, float* avg, int l, long cell,
                                                    double dt, double h, int iters, const DevTables* __restrict__ T,
                                                    double* __restrict__ lduh, double* __restrict__ lQhbnd,
                                                    double* __restrict__ lFhbnd, int* __restrict__ picard,
-                                                   double* luh_upd, int nthreads, int f32faces) {
+                                                   double* luh_upd, int f32faces) {
   constexpr int V = 5, NS = B * B * B, COLS = NS * V;
   float qh[V], fh[3][V];
 #pragma unroll
@@ -455,21 +495,88 @@ __device__ __forceinline__ void finish_cell_points(const float* P, const float* 
     }
   }
   __syncthreads();
-  finish_from_averages<B>(aq, af, l, cell, dt, h, iters, T, lduh, lQhbnd, lFhbnd, picard, luh_upd, nthreads,
+  finish_from_averages<B>(aq, af, l, cell, dt, h, iters, T, lduh, lQhbnd, lFhbnd, picard, luh_upd,
                           f32faces);
 }
 
 // Volume integral and extrapolation of the FP32 forms from the time averages
-// in LDS: aq = lQhi [NS][V], af = lFhi_d [3][NS][V] (node index (z, y, x), x
-// fastest).  Lane l < NS handles node l of the volume integral; the
-// extrapolation runs over (direction, face node, variable) triples.
+// in LDS: aq = lQhi [NS][V], af = lFhi_d [3][NS][V] (LDS point order; the flux
+// lines are overwritten).  All four wavefronts of the workgroup call it.
 template <int B>
-__device__ __forceinline__ void finish_from_averages(const float* aq, const float* af, int l, long cell, double dt,
+__device__ __forceinline__ void finish_from_averages(const float* aq, float* af, int l, long cell, double dt,
                                                      double h, int iters, const DevTables* __restrict__ T,
                                                      double* __restrict__ lduh, double* __restrict__ lQhbnd,
                                                      double* __restrict__ lFhbnd, int* __restrict__ picard,
-                                                     double* luh_upd, int nthreads, int f32faces) {
-  constexpr int V = 5, NS = B * B * B, NF = B * B;
+                                                     double* luh_upd, int f32faces) {
+  constexpr int V = 5, NS = B * B * B, NF = B * B, NPAIR = NF * V, LANES = NPAIR / 3;
+  static_assert(NPAIR % 3 == 0 && LANES <= 64, "three rounds per direction");
+  // The line of (variable, face node) along d gives both its faces' states and
+  // fluxes, and its part of the volume integral, which overwrites the fluxes: a
+  // line is read once.  Three wave-rounds of 60 lanes per direction, as in
+  // contract_lines.  FP64 faces: the reference layout [face][node][var] (var
+  // fastest across lanes); FP32 faces: [face][var][node] (node fastest), the
+  // mesh-internal layout of the FP32 step whose corrector loads one variable row
+  // per step.  Both put lane o's value at place o of the face.
+  {
+    const auto Kxi = columns::opaque(T->Kxif);
+    const auto F0 = columns::opaque(T->F0f), F1 = columns::opaque(T->F1f);
+    const int w = __builtin_amdgcn_readfirstlane(l >> 6), k = l & 63;
+    auto line = [&](auto dir, int o) {
+      constexpr int d = decltype(dir)::value, S = lds_stride<B>(d) * V;
+      const int v = f32faces ? o / NF : o % V;
+      const int fn = f32faces ? o % NF : o / V;
+      const int a = fn / B, b = fn % B;  // (z, y), (z, x), (y, x) along x, y, z
+      const int base = ((d == 0) ? lds_point<B>(a, b, 0) : (d == 1 ? lds_point<B>(a, 0, b) : lds_point<B>(0, a, b))) * V + v;
+      const float* pq = aq + base;
+      float* pf = af + d * NS * V + base;
+      float f[B], g[B], q0 = 0.f, q1 = 0.f, f0 = 0.f, f1 = 0.f;
+#pragma unroll
+      for (int m = 0; m < B; m++) {
+        const float qv = pq[m * S];
+        f[m] = pf[m * S];
+        q0 += qv * F0[m];
+        q1 += qv * F1[m];
+        f0 += f[m] * F0[m];
+        f1 += f[m] * F1[m];
+      }
+      // all 36 products: the mirrored halves of Kxi take 30 operations with a larger error
+#pragma unroll
+      for (int i = 0; i < B; i++) {
+        g[i] = 0.f;
+#pragma unroll
+        for (int m = 0; m < B; m++) g[i] += Kxi[i * B + m] * f[m];
+      }
+#pragma unroll
+      for (int m = 0; m < B; m++) pf[m * S] = g[m];
+      const long fb = (cell * 6 + 2 * d) * NPAIR + o;
+      if (f32faces) {  // the values are FP32 numbers: FP32 storage is exact
+        float* qf = reinterpret_cast<float*>(lQhbnd) + fb;
+        float* ff = reinterpret_cast<float*>(lFhbnd) + fb;
+        qf[0] = q0;
+        qf[NPAIR] = q1;
+        ff[0] = f0;
+        ff[NPAIR] = f1;
+      } else {
+        lQhbnd[fb] = q0;
+        lQhbnd[fb + NPAIR] = q1;
+        lFhbnd[fb] = f0;
+        lFhbnd[fb + NPAIR] = f1;
+      }
+    };
+    if (k < LANES) {
+#pragma nounroll
+      for (int r = (w + 3) & 3; r < 9; r += 4) {
+        const int d = r / 3, o = (r - 3 * d) * LANES + k;
+        if (d == 0)
+          line(std::integral_constant<int, 0>(), o);
+        else if (d == 1)
+          line(std::integral_constant<int, 1>(), o);
+        else
+          line(std::integral_constant<int, 2>(), o);
+      }
+    }
+  }
+  __syncthreads();
   if (l < NS) {
     // volume integral at the node of LDS point l = (x B + z) B + y
     const int y = l % B, z = (l / B) % B, x = l / (B * B);
@@ -481,23 +588,8 @@ __device__ __forceinline__ void finish_from_averages(const float* aq, const floa
 #pragma unroll
     for (int d = 0; d < 3; d++) {
       const float tw = (d == 0) ? T->wf[z] * T->wf[y] : (d == 1 ? T->wf[z] * T->wf[x] : T->wf[y] * T->wf[x]);
-      const int c = (d == 0) ? x : (d == 1 ? y : z);
-      const int stride = lds_stride<B>(d) * V;  // [point][v] stride along d
-      const int lb = line_base((d * NS + l) * V - c * stride);
-      int pb = lb;
-      float part[V];
 #pragma unroll
-      for (int v = 0; v < V; v++) part[v] = 0.f;
-#pragma unroll
-      for (int m = 0; m < B; m++) {
-        const float k = T->Kxif[c * B + m];
-        if (d == 0 && m > 0 && !(m & 1)) pb = line_base(lb + m * stride);  // x: a base per two points
-        const int nb = d == 0 ? pb + (m & 1) * stride : lb + m * stride;
-#pragma unroll
-        for (int v = 0; v < V; v++) part[v] += k * af[nb + v];
-      }
-#pragma unroll
-      for (int v = 0; v < V; v++) du[v] += part[v] * (tw * invDx);
+      for (int v = 0; v < V; v++) du[v] += af[(d * NS + l) * V + v] * (tw * invDx);
     }
     if (luh_upd) {
       const double upd = dt * (T->iw[z] * T->iw[y] * T->iw[x]);
@@ -506,51 +598,6 @@ __device__ __forceinline__ void finish_from_averages(const float* aq, const floa
     } else {
 #pragma unroll
       for (int v = 0; v < V; v++) lduh[(cell * NS + nl) * V + v] = static_cast<double>(du[v]);
-    }
-  }
-  // extrapolation: a lane takes one (variable, face node) pair and gives both
-  // faces of the three directions (d unrolled: compile-time line strides and
-  // face offsets; the pair is decoded once).
-  // FP64 faces: the reference layout [face][node][var] (var fastest across
-  // lanes); FP32 faces: [face][var][node] (node fastest), the mesh-internal
-  // layout of the FP32 step whose corrector loads one variable row per step.
-  constexpr int NPAIR = NF * V;
-  for (int o = l; o < NPAIR; o += nthreads) {
-    const int v = f32faces ? o / NF : o % V;
-    const int fn = f32faces ? o % NF : o / V;
-    const int a = fn / B, b = fn % B;
-    const long fb = cell * 6 * NF * V + (f32faces ? v * NF + fn : fn * V + v);
-#pragma unroll
-    for (int d = 0; d < 3; d++) {
-      // the line through face node (a, b) along d, (a, b) = (z, y), (z, x), (y, x):
-      // LDS point(m) = base + m * stride
-      const int base = (d == 0) ? lds_point<B>(a, b, 0) : (d == 1 ? lds_point<B>(a, 0, b) : lds_point<B>(0, a, b));
-      const int sv = lds_stride<B>(d) * V;
-      const float* pq = aq + base * V + v;
-      const float* pf = af + d * NS * V + base * V + v;
-      float q0 = 0.f, q1 = 0.f, f0 = 0.f, f1 = 0.f;
-#pragma unroll
-      for (int m = 0; m < B; m++) {
-        const float qv = pq[m * sv], fv = pf[m * sv];
-        const float c0 = T->F0f[m], c1 = T->F1f[m];
-        q0 += qv * c0;
-        q1 += qv * c1;
-        f0 += fv * c0;
-        f1 += fv * c1;
-      }
-      if (f32faces) {  // the values are FP32 numbers: FP32 storage is exact
-        float* qf = reinterpret_cast<float*>(lQhbnd);
-        float* ff = reinterpret_cast<float*>(lFhbnd);
-        qf[fb + (2 * d) * NF * V] = q0;
-        qf[fb + (2 * d + 1) * NF * V] = q1;
-        ff[fb + (2 * d) * NF * V] = f0;
-        ff[fb + (2 * d + 1) * NF * V] = f1;
-      } else {
-        lQhbnd[fb + (2 * d) * NF * V] = q0;
-        lQhbnd[fb + (2 * d + 1) * NF * V] = q1;
-        lFhbnd[fb + (2 * d) * NF * V] = f0;
-        lFhbnd[fb + (2 * d + 1) * NF * V] = f1;
-      }
     }
   }
   if (l == 0 && picard) picard[cell] = iters;
@@ -570,8 +617,14 @@ struct GuardArgs {
 
 template <int B, typename R, bool MF, bool FIX, bool CG, bool ONE = false, bool LIST = false, bool PART = false>
 // Fixed-count form: four workgroups per CU (LDS 39 KB each; the register
-// budget of 128 costs a few spills, measured faster than three workgroups)
-__global__ __launch_bounds__((LShape<B>::THREADS), (ONE ? 5 : (FIX ? 4 : 1))) void predictor3d_lines_kernel(
+// budget of 128 costs a few spills, measured faster than three workgroups).
+// One iteration: bound by LDS accesses and VALU issue together (81^3 cells).
+// Its four spatial contractions (two CERK stages, the collapsed divergence, the
+// volume integral with the extrapolation) are line tasks: 5.95 ms with each lane
+// reading the lines through its node -> 5.48 with the first three as line tasks
+// -> 4.99 with all four; lQhi on top of Fc_x leaves LDS for six workgroups per
+// CU at 80 VGPRs instead of five: 4.75.
+__global__ __launch_bounds__((LShape<B>::THREADS), (ONE ? 6 : (FIX ? 4 : 1))) void predictor3d_lines_kernel(
     long ncells, const double* luh, const double* __restrict__ hcell, const double* __restrict__ dtp,
     const int* __restrict__ cinst, double* __restrict__ lduh, double* __restrict__ lQhbnd,
     double* __restrict__ lFhbnd, int* __restrict__ picard, const DevTables* __restrict__ T, PdeParams P,
@@ -597,11 +650,12 @@ __global__ __launch_bounds__((LShape<B>::THREADS), (ONE ? 5 : (FIX ? 4 : 1))) vo
   // iteration; the tile then holds lQhi.
   constexpr int AF_BYTES = 3 * NS * V * 4;
   // ONE (one Picard iteration, collapsed): no sweep through the tile; the
-  // buffer holds the CERK stage fluxes / Fc_d [3][NS][V] and lQhi [NS][V], then af
+  // buffer holds the CERK stage fluxes / Fc_d [3][NS][V], lQhi [NS][V] in place of
+  // the first (each lane takes its point's values before it writes), then af
   static_assert(!ONE || FIX, "one collapsed iteration: fixed-count form");
   static_assert(!LIST || (FIX && CG && !ONE), "cell list: the fixed-count CERK form");
   static_assert(!PART || (ONE && CG && !LIST), "a part of the mesh: the one-iteration CERK form");
-  constexpr int ONE_BYTES = 4 * NS * V * 4;
+  constexpr int ONE_BYTES = 3 * NS * V * 4;
   constexpr int NEED = ONE ? ONE_BYTES + AF_BYTES
                           : (FIX ? TILE_BYTES + AF_BYTES : (sizeof(R) == 4 ? 2 * TILE_BYTES : TILE_BYTES));
   constexpr int BUF_BYTES = (FIX || NEED > AVG_BYTES) ? NEED : AVG_BYTES;
@@ -619,7 +673,7 @@ __global__ __launch_bounds__((LShape<B>::THREADS), (ONE ? 5 : (FIX ? 4 : 1))) vo
   // phase (registers are the occupancy limit): opl[0][r][h][n] = dudx[4h + r][n],
   // opl[1][r][h][n] = P[4h + r][n] (zero rows >= B); a lane uses r = l % 4
   __shared__ __align__(16) float opl[2][4][2 * B];
-  if constexpr (MF) {
+  if constexpr (MF && !ONE) {
     if (l < 16 * B) {
       const int op = l / (8 * B), r = (l / (2 * B)) % 4, hh = (l % (2 * B)) / B, n = l % B;
       const int row = 4 * hh + r;
@@ -703,28 +757,13 @@ __global__ __launch_bounds__((LShape<B>::THREADS), (ONE ? 5 : (FIX ? 4 : 1))) vo
       }
       __syncthreads();
       // K = h K_stage = sum_d dudx_d F_d; the 1/h goes into the step coefficients
+      contract_lines<B>(fl, l, T, stage);
+      __syncthreads();
       float K[V] = {0.f, 0.f, 0.f, 0.f, 0.f};
-      if (lane_on) {
+      if (lane_on) {  // no barrier behind it: the next stage and Fc_d go to this lane's own point
 #pragma unroll
-        for (int d = 0; d < 3; d++) {
-          const int c = d == 0 ? t : (d == 1 ? y : z);              // coordinate of p along d
-          const int stride = lds_stride<B>(d) * V;                    // [point][v] stride along d
-          // dudx[c][n] from the operator columns in LDS (opl[0][r][hh B + n] = dudx[4 hh + r][n])
-          float dr[B];
-#pragma unroll
-          for (int n = 0; n < B; n++) dr[n] = opl[0][c & 3][(c >> 2) * B + n];
-          const int lb = line_base(d * NS * V + pv - c * stride);
-          int pb = lb;
-#pragma unroll
-          for (int n = 0; n < B; n++) {
-            if (d == 0 && n > 0 && !(n & 1)) pb = line_base(lb + n * stride);  // x: a base per two points
-            const int nb = d == 0 ? pb + (n & 1) * stride : lb + n * stride;
-#pragma unroll
-            for (int v = 0; v < V; v++) K[v] += fl[nb + v] * dr[n];
-          }
-        }
+        for (int v = 0; v < V; v++) K[v] = (fl[pv + v] + fl[NS * V + pv + v]) + fl[2 * NS * V + pv + v];
       }
-      __syncthreads();  // fl is rewritten by the next stage / the guess
 #pragma unroll
       for (int v = 0; v < V; v++) {
         if (stage == 0) {
@@ -749,6 +788,7 @@ __global__ __launch_bounds__((LShape<B>::THREADS), (ONE ? 5 : (FIX ? 4 : 1))) vo
 #pragma unroll
       for (int v = 0; v < V; v++) qg[i][v] = u[v] - a1 * K1[v] - a2 * (K2[v] - K1[v]);
     }
+    if constexpr (!ONE) __syncthreads();  // the stage's values are read: the guess may overwrite them
     if (lane_on) {
       if (nfull > 0) {
 #pragma unroll
@@ -1002,32 +1042,18 @@ __global__ __launch_bounds__((LShape<B>::THREADS), (ONE ? 5 : (FIX ? 4 : 1))) vo
   // ---- after the Picard loop: q = previous iterate, the tile holds the final one ----
   if constexpr (FIX) {
     // collapsed last iteration: Fc_d [3][NS][V] at the tile's start (stored
-    // above), lQhi [NS][V] behind it
+    // above), lQhi [NS][V] behind it (ONE: over Fc_x, a lane reads and writes its
+    // own point only)
     float* fcb = tl;
-    float* aq = tl + 3 * NS * V;
+    float* aq = ONE ? tl : tl + 3 * NS * V;
     [[maybe_unused]] float gsq = 0.f, qsq = 0.f;
     __syncthreads();
+    contract_lines<B>(fcb, l, T, 2);
+    __syncthreads();
     if (lane_on) {
-      // coordinates of p = (z, y, x = t), recomputed from pv (not kept live through the loop)
-      const int pp = pv / V, py = pp % B, pz = (pp / B) % B, px = pp / (B * B);
-      float dv[V] = {0.f, 0.f, 0.f, 0.f, 0.f};
+      float dv[V];
 #pragma unroll
-      for (int d = 0; d < 3; d++) {
-        const int c = d == 0 ? px : (d == 1 ? py : pz);              // coordinate of p along d
-        const int stride = lds_stride<B>(d) * V;                      // [point][v] stride along d
-        float dr[B];                                                  // dudx[c][n]
-#pragma unroll
-        for (int n = 0; n < B; n++) dr[n] = opl[0][c & 3][(c >> 2) * B + n];
-        const int lb = line_base(d * NS * V + pv - c * stride);
-        int pb = lb;
-#pragma unroll
-        for (int n = 0; n < B; n++) {
-          if (d == 0 && n > 0 && !(n & 1)) pb = line_base(lb + n * stride);  // x: a base per two points
-          const int nb = d == 0 ? pb + (n & 1) * stride : lb + n * stride;
-#pragma unroll
-          for (int v = 0; v < V; v++) dv[v] += dr[n] * fcb[nb + v];
-        }
-      }
+      for (int v = 0; v < V; v++) dv[v] = (fcb[pv + v] + fcb[NS * V + pv + v]) + fcb[2 * NS * V + pv + v];
 #pragma unroll
       for (int v = 0; v < V; v++) {
         const float qh = u[v] - cdt * dv[v];
@@ -1067,7 +1093,7 @@ __global__ __launch_bounds__((LShape<B>::THREADS), (ONE ? 5 : (FIX ? 4 : 1))) vo
         }
       }
     }
-    finish_from_averages<B>(aq, af, l, cell, dt, h, iters, T, lduh, lQhbnd, lFhbnd, picard, luh_upd, S::THREADS,
+    finish_from_averages<B>(aq, af, l, cell, dt, h, iters, T, lduh, lQhbnd, lFhbnd, picard, luh_upd,
                             f32faces);
   } else if constexpr (sizeof(R) == 4) {
     float* t2 = reinterpret_cast<float*>(buf) + TILE;
@@ -1079,7 +1105,7 @@ __global__ __launch_bounds__((LShape<B>::THREADS), (ONE ? 5 : (FIX ? 4 : 1))) vo
     }
     __syncthreads();
     finish_cell_points<B>(t2, tl, t2, l, cell, dt, h, iters, T, lduh, lQhbnd, lFhbnd, picard, luh_upd,
-                          S::THREADS, f32faces);
+                          f32faces);
   } else {
     finish_cell<B, R>(q, tl, buf, l, cell, dt, h, iters, T, lduh, lQhbnd, lFhbnd, picard, luh_upd);
   }
@@ -1378,7 +1404,7 @@ __global__ __launch_bounds__(256, 3) void predictor3d_tile_kernel(
   }
 
   // ---- tB = final iterate, tA = previous iterate ----
-  finish_cell_points<B>(tA, tB, tA, l, cell, dt, h, iters, T, lduh, lQhbnd, lFhbnd, picard, luh_upd, S::THREADS,
+  finish_cell_points<B>(tA, tB, tA, l, cell, dt, h, iters, T, lduh, lQhbnd, lFhbnd, picard, luh_upd,
                         f32faces);
 }
 
