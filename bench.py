@@ -83,14 +83,16 @@ def predictor_flops_per_cell(dim, B, V, ND, iters, cerk=False):
 
 
 def equal_slice_savings_per_cell(dim, B, V, iters):
-    """Contraction flops the node-column kernel does not execute with the trivial
+    """Contraction flops the column kernel does not execute with the trivial
     guess: the first iterate is constant in time, so its D stiffness contractions
-    run for one time slice instead of B (cells that iterate at least once)."""
+    run for one time slice instead of B (cells that iterate at least once).  What the
+    mirrored halves of the operator save within a line (30 operations instead of 36
+    at B = 6) is not counted."""
     return np.where(np.asarray(iters) > 0, dim * 2 * V * B ** (dim + 1) * (B - 1), 0)
 
 
-def kind_is_node_column(precision, variant, E):
-    """Whether the mesh runs the node-column kernel for 3D order 5: FP64 with the
+def kind_is_column(precision, variant, E):
+    """Whether the mesh runs the column kernel for 3D order 5: FP64 with the
     default variant (0) or variant 1 or 4, and any precision with variant 1; the
     line / tile kernels otherwise."""
     return (precision == E.PREC_FP64 and variant in (0, 1, 4)) or variant == 1
@@ -159,11 +161,11 @@ def run_form(E, P, n, order, steps, warmup, precision, picard, seed, modes, vari
     # divergences are reported apart
     flops = float(np.sum(predictor_flops_per_cell(dim, B, V, V, iters)))
     cerk_flops = float(np.sum(predictor_flops_per_cell(dim, B, V, V, iters, cerk=True))) - flops if guess else 0.0
-    # contraction flops the kernel executes: the node-column kernel (the FP64 form, FP32
+    # contraction flops the kernel executes: the column kernel (the FP64 form, FP32
     # variant 1) forms the trivial guess's first iteration from one time slice
-    node_column = kind_is_node_column(precision, variant, E)
+    column_form = kind_is_column(precision, variant, E)
     executed = flops - (float(np.sum(equal_slice_savings_per_cell(dim, B, V, iters)))
-                        if node_column and not guess else 0.0)
+                        if column_form and not guess else 0.0)
     pred_ms = ph["predictor_ms"] / steps
     kind = {E.PREC_FP64: "fp64", E.PREC_FP32: "fp32", E.PREC_BF16: "bf16"}[precision]
     achieved = flops / (pred_ms * 1e-3) / 1e12
@@ -473,7 +475,7 @@ def main():
     ap.add_argument("--cpu-n", type=int, default=None)
     ap.add_argument("--cpu-steps", type=int, default=None)
     ap.add_argument("--sweep-variants", action="store_true",
-                    help="only time the predictor kernel variants (node-column, line, line+MFMA, tile+MFMA) and exit")
+                    help="only time the predictor kernel variants (column, line, line+MFMA, tile+MFMA) and exit")
     ap.add_argument("--variant", type=int, default=None,
                     help="with --sweep-variants: time only this predictor variant (1..4)")
     ap.add_argument("--copy-calibration", action="store_true",
@@ -525,7 +527,7 @@ def main():
     if args.sweep_variants:
         k32 = args.picard_fp32 if args.picard_fp32 > 0 else 3
         for prec, name, pic in ((E.PREC_FP64, "fp64", 0), (E.PREC_FP32, "fp32", k32)):
-            for variant, vname in ((1, "node-column"), (2, "line"), (3, "line+mfma"), (4, "tile+mfma")):
+            for variant, vname in ((1, "column"), (2, "line"), (3, "line+mfma"), (4, "tile+mfma")):
                 if (prec == E.PREC_FP64 and variant in (3, 4)) or \
                         (args.variant is not None and variant != args.variant):
                     continue

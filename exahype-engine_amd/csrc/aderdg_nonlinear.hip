@@ -12,7 +12,7 @@
 //                       stableTimeStepSize.cpph:14-62 with the global min reduction
 //
 // Work decomposition (MI355X-first, not the reference's loop nests):
-//   * predictor: one workgroup holds CPB whole cells; one thread owns one
+//   * predictor_kernel: one workgroup holds CPB whole cells; one thread owns one
 //     spatial node s of one cell and keeps that node's whole space-time
 //     column lQi[s][0..B)[0..nData) plus its Picard accumulators in VGPRs.
 //     Per time slice the node's flux is evaluated in registers and published
@@ -26,7 +26,8 @@
 //     in LDS and merged with one 64-bit atomicMin per workgroup on the IEEE
 //     bit pattern (exact and order independent for positive doubles), into
 //     the instance's dt_next or, on the uniform mesh, into one of 1024 slots
-//     on separate cache lines that dt_reduce_kernel merges afterwards.
+//     on separate cache lines that advance_time_kernel merges (dt_reduce_kernel
+//     for the first dt and the split step).
 #include <hip/hip_runtime.h>
 
 #include <cfloat>
@@ -1389,8 +1390,8 @@ int launch_predictor(const KernelCfg& k, hipStream_t s, long n, const double* lu
     if (!line_kernels_serve(k) || k.guess || o.hdim) return -1;
     return launch_predictor3d_tile(k, s, n, luh, h, dt, lduh, qb, fb, pic, o.cinst, o.luh_update, o.faces_f32);
   }
-  // auto: FP32 -> line kernel on the matrix cores; FP64 -> node-column kernel
-  // (non-cubic cells: node-column kernel)
+  // auto: FP32 -> line kernel on the matrix cores; FP64 -> column kernel
+  // (non-cubic cells: column kernel)
   if (line_kernels_serve(k) && !o.hdim) {
     const int v = k.pred_variant;
     const bool fp32 = k.precision != 0;

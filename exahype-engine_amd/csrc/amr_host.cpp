@@ -75,7 +75,7 @@ int ipow(int b, int e) {
   return r;
 }
 
-// cells per workgroup of the node-column predictor / corrector (Shape::CPB)
+// workgroups of the corrector for ncells (the predictors of small cells have at least as many)
 long tiles_of(const exa::KernelCfg& k, long ncells) {
   const int NS = ipow(k.order + 1, k.dim);
   const int cpb = NS >= 128 ? 1 : 256 / NS;

@@ -50,12 +50,12 @@ struct KernelCfg {
   double cfl, pnpm;
   PdeParams pde;
   const DevTables* tab;  // device pointer
-  int pred_variant;      // 0 auto, 1 node-column, 2 line (VALU), 3 line (FP32 matrix cores),
+  int pred_variant;      // 0 auto, 1 column, 2 line (VALU), 3 line (FP32 matrix cores),
                          // 4 tile (FP32, full-rate matrix cores)
   int dialect;           // 0 generic Picard rule; 1 the optimised kernels' rule (MaxIterations
                          // 2B+1, or max(B-3, 1) with the CERK guess; tolerance exit always on;
-                         // count min(iter+1, Max)); runs on the node-column kernel
-  int guess;             // initial guess: 0 luh at every time node; 1 CERK (node-column kernel,
+                         // count min(iter+1, Max)); runs on the column kernel
+  int guess;             // initial guess: 0 luh at every time node; 1 CERK (column kernel,
                          // and the FP32 matrix-core line kernel with a fixed Picard count)
   // Picard guard of the one-iteration FP32 CERK form: a cell whose relative
   // proxy residual |lQhi(1) - lQhi(0)| / |lQhi(1)| reaches guard_tol (<= 0:
@@ -103,7 +103,7 @@ struct LaunchOpts {
   // predictor, one-iteration FP32 CERK form: Picard guard buffer of 2 + ncells
   // ints {listed this launch (0 on entry), listed in total, list}; nullptr: no guard
   int* guard = nullptr;
-  // node-column predictor and corrector: 0 = one edge length per cell (h[cell]),
+  // column predictor and corrector: 0 = one edge length per cell (h[cell]),
   // D = one per direction (h[cell][d]); the other kernels take cubic cells only
   int hdim = 0;
   // the one-iteration FP32 CERK line predictor and the fused corrector: the

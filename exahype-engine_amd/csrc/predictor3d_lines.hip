@@ -1456,7 +1456,7 @@ int launch_predictor3d_lines(const KernelCfg& k, hipStream_t st, long n, const d
   const dim3 grid(blocks), block(S::THREADS);
   const GuardArgs none;
   if (k.precision == 0) {
-    if (range || k.guess) return -1;  // the FP64 line kernel has no CERK guess (the node-column kernel has)
+    if (range || k.guess) return -1;  // the FP64 line kernel has no CERK guess (the column kernel has)
     hipLaunchKernelGGL((predictor3d_lines_kernel<B, double, false, false, false>), grid, block, 0, st, n, luh, h, dt,
                        cinst, lduh, qb, fb, pic, k.tab, k.pde, maxIter, adaptive, luh_upd, 0, none);
   } else {

@@ -241,7 +241,7 @@ class Context:
         return self.B ** (self.dim - 1)
 
     def set_predictor_variant(self, variant):
-        """0: fastest kernel for the shape (default), 1: generic node-column kernel."""
+        """0: fastest kernel for the shape (default), 1: generic column kernel."""
         _check(_lib.exa_ctx_set_predictor_variant(self.h, variant))
 
     def set_dialect(self, dialect, vect_size=1):

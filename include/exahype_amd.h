@@ -99,7 +99,7 @@ int exa_ctx_set_advection(exa_ctx* ctx, const double* a);
 int exa_ctx_set_pde_params(exa_ctx* ctx, const double* prm, int n);
 
 /* Predictor kernel selection: 0 (default) picks the fastest kernel compiled
- * for the shape, 1 forces the generic node-column kernel (every shape); for
+ * for the shape, 1 forces the generic column kernel (every shape); for
  * 3D Euler order 5 also 2 = x-line kernel (VALU), 3 = x-line kernel on 4x4x1
  * matrix-core steps (FP32), 4 = space-time tile kernel on 16x16x4 matrix-core
  * steps (FP32).  Meshes copy the context's settings when they are created. */
@@ -134,7 +134,7 @@ int exa_ctx_set_predictor_variant(exa_ctx* ctx, int variant);
  * vect_size (1, 2, 4 or 8 doubles: the generator's noarch, wsm, snb/hsw,
  * knl/skx widths) sets nVarPad and nDataPad of the exa_opt_* and
  * exa_converter_* entry points.  The optimised Picard dialects run on the
- * node-column predictor kernel.  Meshes copy the context's settings when
+ * column predictor kernel.  Meshes copy the context's settings when
  * created. */
 enum exa_dialect {
   EXA_DIALECT_GENERIC = 0,
@@ -150,7 +150,7 @@ int exa_ctx_set_dialect(exa_ctx* ctx, int dialect, int vect_size);
  * kernels' Continuous Extension Runge-Kutta guess,
  * fusedSPTVI_nonlinear_cpp.template:121-173).  exa_ctx_set_dialect sets it
  * too (CERK for EXA_DIALECT_OPTIMISED_CERK); a later call overrides.  With the
- * generic rule the CERK guess runs on the node-column kernel, and for 3D Euler
+ * generic rule the CERK guess runs on the column kernel, and for 3D Euler
  * order 5 in FP32 with a fixed Picard count on the x-line matrix-core kernel. */
 enum exa_guess { EXA_GUESS_TRIVIAL = 0, EXA_GUESS_CERK = 1 };
 int exa_ctx_set_initial_guess(exa_ctx* ctx, int guess);
@@ -317,9 +317,9 @@ int exa_stableTimeStepSize(exa_ctx* ctx, const double* luh, const double* dx, do
 /* Cell extents of the batched entry points: per_direction = 0 (default): d_h
  * holds one edge length per cell [ncells]; 1: d_h holds the reference's dx
  * vector per cell [ncells][dim] (ADERDGSolver.h:2542-2553 passes dx[D]), used
- * per direction by the predictor (node-column kernel), the face integrals and
+ * per direction by the predictor (column kernel), the face integrals and
  * the stable dt.  The FP32 line and BF16 tile kernels take cubic cells: with 1
- * an FP32 context runs the FP32 node-column kernel and BF16 is refused. */
+ * an FP32 context runs the FP32 column kernel and BF16 is refused. */
 int exa_ctx_set_cell_dx(exa_ctx* ctx, int per_direction);
 
 /* Predictor + volume integral for ncells cells (reference row: a4 + a5).
