@@ -45,8 +45,17 @@ struct Shape {
   static constexpr int NF = cpow(B, D - 1);  // nodes per face
   static constexpr int NL = D * NF;          // lines per cell
   // The smallest workgroup whose lanes own nodes for at least 93 %: one
-  // wavefront needs no barrier waits (orders 1, 2 and 3 in 2D, 1 and 3 in 3D).
+  // wavefront needs no barrier waits (orders 2 and 3 in 2D, 3 in 3D).  Two
+  // exceptions, predictor alone, Euler:
+  // - order 1, bound by HBM alone and in FP32 slower in 64 lanes than with the
+  //   node-column form before it: 256 (375,000 3D cells, three FP32 iterations,
+  //   237 -> 211 us; node-column 218).
+  // - 3D order 2 in FP64: 54 of 64 lanes, because the barriers of 243 of 256
+  //   weigh more than the idle lanes (8,000 cells 33.5 -> 29.4 us, 64 cells 13.1
+  //   -> 9.5, node-column 12.3; 111,111 cells equal).
   static constexpr int threads() {
+    if (B == 2) return 256;
+    if (D == 3 && B == 3 && sizeof(R) == 8) return 64;
     for (int t : {64, 128, 256})
       if (t / NS * NS * 100 >= 93 * t) return t;
     return 256;
@@ -61,9 +70,14 @@ struct Shape {
   // the LDS of a second slice would cost (batched 3D order 4: equal).
   static constexpr int TS = D == 3 && B <= 5 ? 1 : 2;
   static constexpr int NROW = NS / B;
-  // order 3 exchanges its lines between lanes and needs the buffer at the end only
-  static constexpr bool LANES = B == 4;
-  static constexpr int LINE_BYTES = LANES ? 0 : TS * SLICE * int(sizeof(R));
+  // orders 1 and 3 exchange their lines between lanes and need the buffer at the end only
+  static constexpr bool LANES = B == 2 || B == 4;
+  // 3D order 2 in FP32: a node reads the three lines through itself (three values
+  // each, as many LDS accesses as a line task's four, and one phase less), from two
+  // slices in turn; 64 cells, three iterations 12.2 -> 9.9 us (node-column 11.3),
+  // 111,111 cells 264 -> 223 (233)
+  static constexpr bool NODES = D == 3 && B == 3 && sizeof(R) == 4;
+  static constexpr int LINE_BYTES = LANES ? 0 : (NODES ? 2 : TS) * SLICE * int(sizeof(R));
   static constexpr int END_BYTES = (SLICE + CPB * NS * ND) * 8;
   static constexpr int BUF_BYTES = LINE_BYTES > END_BYTES ? LINE_BYTES : END_BYTES;
   static constexpr int RED = CPB * (NS + NROW);
@@ -182,6 +196,8 @@ struct EvenOdd {
   }
 };
 
+// Lines of two nodes (order 1) lie in eight consecutive lanes, the bits of a lane
+// its x, y and z: a partner's value comes by one exchange (x, y) or two (z).
 // Four-node lines (order 3) stay in one wavefront: 16 consecutive lanes hold a
 // plane (x fastest) and, in 3D, the wave's four rows the planes.  The other
 // values of a line come by lane exchange instead of LDS: rotations of the quad
@@ -205,6 +221,8 @@ __device__ __forceinline__ R dpp(R v) {
 constexpr int quad_rotate(int k) {  // lane i of a quad takes lane (i + k) % 4
   return (k & 3) | ((1 + k) & 3) << 2 | ((2 + k) & 3) << 4 | ((3 + k) & 3) << 6;
 }
+// lane i of a quad takes lane i ^ 1, i ^ 2, i ^ 3; lane i of eight takes lane i ^ 7
+constexpr int kQuadXor1 = 0xb1, kQuadXor2 = 0x4e, kQuadXor3 = 0x1b, kHalfRowXor7 = 0x141;
 constexpr int row_take(int n) { return 0x120 + 16 - n; }  // lane i of a row takes lane (i + n) % 16
 
 // The values of the four rows at this lane's place in its row, in every row.
@@ -293,7 +311,12 @@ struct Tile {
   // average in the loop, 481 this way; 2D at 243^2 0.220, 0.249 and 0.200 ms).
   static constexpr bool FHL = sizeof(R) == 8 && B >= 6;
 
-  static constexpr bool LANES = S::LANES;
+  static constexpr bool LANES = S::LANES, NODES = S::NODES;
+
+  // The node's solution stays in registers where the column leaves them (orders 1
+  // and 2, bound by HBM: a second read of luh per iteration misses the L1; 375,000
+  // 3D cells of order 1, three FP32 iterations in 64 lanes 266 -> 237 us)
+  static constexpr bool HOLD = B <= 3;
 
   static __device__ __forceinline__ bool keep(int d, int v) { return !EU || euler_canonical(D, d, v); }
 
@@ -344,12 +367,18 @@ struct Tile {
     for (int d = 0; d < D; d++)
       cd[d] = static_cast<R>(dt / (valid ? hcell[hdim ? cell * hdim + d : cell] : 1.0));
 
-    // the node's solution, read again where it is needed instead of being held
-    auto solution = [&](R(&u)[ND]) {
+    // the node's solution: held, or read again where it is needed
+    R held[ND];
+    auto solution = [&](R(&u)[ND], bool first = false) {
 #pragma unroll
-      for (int v = 0; v < ND; v++)
-        u[v] = valid ? static_cast<R>(luh[(cell * NS + s) * ND + v]) : (v == 0 ? R(1) : R(0));
+      for (int v = 0; v < ND; v++) {
+        if (HOLD && !first)
+          u[v] = held[v];
+        else
+          u[v] = valid ? static_cast<R>(luh[(cell * NS + s) * ND + v]) : (v == 0 ? R(1) : R(0));
+      }
     };
+    if constexpr (HOLD) solution(held, true);
 
     auto publish = [&](int slice, const R(&F)[D][V]) {
 #pragma unroll
@@ -366,38 +395,68 @@ struct Tile {
         g[v] = a;
       }
     };
-    // LANES: row c_d of dt / dx_d dudx; x and y from the node's own entry on round
-    // the line, z from plane 0
-    R cl[LANES ? D : 1][4];
-    if constexpr (LANES) {
+    // LANES, NODES: row c_d of dt / dx_d dudx; LANES: from the node's own entry on
+    // round the line (order 3 along z: from plane 0)
+    R cl[LANES || NODES ? D : 1][B];
+    if constexpr (LANES || NODES) {
 #pragma unroll
       for (int d = 0; d < D; d++) {
         const int c = d == 0 ? x : (d == 1 ? y : z);
 #pragma unroll
-        for (int k = 0; k < 4; k++)
-          cl[d][k] = cd[d] * (sizeof(R) == 8 ? static_cast<R>(T->dudx[c * B + (d == 2 ? k : (c + k) % B)])
-                                             : static_cast<R>(T->dudxf[c * B + (d == 2 ? k : (c + k) % B)]));
+        for (int k = 0; k < B; k++) {
+          const int n = NODES || (B == 4 && d == 2) ? k : (c + k) % B;
+          cl[d][k] = cd[d] * (sizeof(R) == 8 ? static_cast<R>(T->dudx[c * B + n]) : static_cast<R>(T->dudxf[c * B + n]));
+        }
       }
     }
     // dt times the divergence of the flux F by lane exchange
     auto exchange = [&](const R(&F)[D][V], R(&g)[V]) __attribute__((always_inline)) {
+      if constexpr (B == 2) {
+#pragma unroll
+        for (int v = 0; v < V; v++) {
+          R a = cl[0][0] * F[0][v];
+          a += cl[0][1] * dpp<kQuadXor1>(F[0][v]);
+          a += cl[1][0] * F[1][v];
+          a += cl[1][1] * dpp<kQuadXor2>(F[1][v]);
+          if constexpr (D == 3) {
+            a += cl[D - 1][0] * F[D - 1][v];
+            a += cl[D - 1][1] * dpp<kQuadXor3>(dpp<kHalfRowXor7>(F[D - 1][v]));
+          }
+          asm volatile("" : "+v"(a));  // as below
+          g[v] = a;
+        }
+      }
+      if constexpr (B == 4) {
+#pragma unroll
+        for (int v = 0; v < V; v++) {
+          R a = cl[0][0] * F[0][v];
+          a += cl[0][1] * dpp<quad_rotate(1)>(F[0][v]);
+          a += cl[0][2] * dpp<quad_rotate(2)>(F[0][v]);
+          a += cl[0][3] * dpp<quad_rotate(3)>(F[0][v]);
+          a += cl[1][0] * F[1][v];
+          a += cl[1][1] * dpp<row_take(4)>(F[1][v]);
+          a += cl[1][2] * dpp<row_take(8)>(F[1][v]);
+          a += cl[1][3] * dpp<row_take(12)>(F[1][v]);
+          if constexpr (D == 3) {
+            R r[4];
+            all_rows(F[D - 1][v], r);
+#pragma unroll
+            for (int k = 0; k < 4; k++) a += cl[D - 1][k] * r[k];
+          }
+          asm volatile("" : "+v"(a));  // formed here: sunk to its use, it would keep the exchanged values alive
+          g[v] = a;
+        }
+      }
+    };
+    // NODES: the same from the lines of a published slice
+    auto through = [&](int slice, R(&g)[V]) __attribute__((always_inline)) {
 #pragma unroll
       for (int v = 0; v < V; v++) {
-        R a = cl[0][0] * F[0][v];
-        a += cl[0][1] * dpp<quad_rotate(1)>(F[0][v]);
-        a += cl[0][2] * dpp<quad_rotate(2)>(F[0][v]);
-        a += cl[0][3] * dpp<quad_rotate(3)>(F[0][v]);
-        a += cl[1][0] * F[1][v];
-        a += cl[1][1] * dpp<row_take(4)>(F[1][v]);
-        a += cl[1][2] * dpp<row_take(8)>(F[1][v]);
-        a += cl[1][3] * dpp<row_take(12)>(F[1][v]);
-        if constexpr (D == 3) {
-          R r[4];
-          all_rows(F[D - 1][v], r);
+        R a = R(0);
 #pragma unroll
-          for (int k = 0; k < 4; k++) a += cl[D - 1][k] * r[k];
-        }
-        asm volatile("" : "+v"(a));  // formed here: sunk to its use, it would keep the exchanged values alive
+        for (int d = 0; d < D; d++)
+#pragma unroll
+          for (int n = 0; n < B; n++) a += cl[d][n] * slab[slice * SLICE + line[d] * B + n + v * VS];
         g[v] = a;
       }
     };
@@ -415,9 +474,14 @@ struct Tile {
         publish(0, F);
       }
       __syncthreads();
-      lines(slab, 1, T);
-      __syncthreads();
-      if (valid) gather(0, g);
+      if constexpr (NODES) {
+        if (valid) through(0, g);
+        __syncthreads();  // read before the slice is written again
+      } else {
+        lines(slab, 1, T);
+        __syncthreads();
+        if (valid) gather(0, g);
+      }
     };
 
     // FHL: the time-averaged flux of the running iteration accumulates in
@@ -454,7 +518,7 @@ struct Tile {
         res = sq;  // 0 on lanes past the cell
 #pragma unroll
         for (int m = W / 2; m >= 1; m >>= 1) res += __shfl_xor(res, m, 64);
-        if constexpr (THREADS > 64) {
+        if constexpr (NS > 64) {
           if ((tid & 63) == 0) red[tid >> 6] = res;
           __syncthreads();
           res = 0.0;
@@ -554,6 +618,18 @@ struct Tile {
             __builtin_amdgcn_sched_barrier(0);  // slices one after the other: interleaved, they spill
           }
         }
+      } else if constexpr (NODES) {
+#pragma unroll
+        for (int t = 0; t < B; t++) {
+          if (active) {
+            R F[D][V];
+            flux<D, V, R, EU>(P, q[t], F);
+            publish(t & 1, F);
+          }
+          __syncthreads();
+          if (active) through(t & 1, g[t]);
+        }
+        __syncthreads();  // the last slice is read before the next iteration writes it
       } else {
 #pragma unroll
         for (int t0 = 0; t0 < B; t0 += TS) {
@@ -743,6 +819,7 @@ struct Tile {
 // registers, 24 -> 30 ms at 81^3; order 3 at three: 27, 0.375 -> 0.390 ms at 35^3).
 template <int D, int B, int V, int NP, typename R>
 constexpr int min_waves() {
+  if (D == 3 && B <= 3) return 3;  // as many as LDS takes
   return sizeof(R) == 8 ? (B == 4 || B >= 6 ? 2 : 3) : 4;
 }
 
