@@ -817,15 +817,20 @@ struct Tile {
 // Waves per SIMD the register allocation aims at: the two columns (2 B V values)
 // and a line's working set; one wave more spills (FP64 order 5 at three: 52
 // registers, 24 -> 30 ms at 81^3; order 3 at three: 27, 0.375 -> 0.390 ms at 35^3).
-template <int D, int B, int V, int NP, typename R>
+// Order 4 spills at three, 10 to 16 registers for Euler and 41 to 44 for the other
+// equations, and still gains, but for the latter's one-iteration CERK form in 3D
+// (advection, 1,000 cells: 24.0 at three, 18.9 us at two; 24,000 cells 390, 340 us;
+// with the trivial guess 607, 672 us, in 2D 228, 265 us).
+template <int D, int B, int V, int NP, typename R, bool CG, bool EU>
 constexpr int min_waves() {
   if (D == 3 && B <= 3) return 3;  // as many as LDS takes
-  return sizeof(R) == 8 ? (B == 4 || B >= 6 ? 2 : 3) : 4;
+  if (sizeof(R) == 4) return 4;
+  return B == 4 || B >= 6 || (D == 3 && B == 5 && CG && !EU) ? 2 : 3;
 }
 
 // One workgroup per tile of CPB cells, or a smaller grid that loops over the tiles.
 template <int D, int B, int V, int NP, typename R, bool CG, bool EU>
-__global__ __launch_bounds__((Shape<D, B, V, NP, R>::THREADS), (min_waves<D, B, V, NP, R>())) void
+__global__ __launch_bounds__((Shape<D, B, V, NP, R>::THREADS), (min_waves<D, B, V, NP, R, CG, EU>())) void
 column_predictor_kernel(long ncells, long ntiles, const double* luh, const double* __restrict__ hcell,
                         const double* __restrict__ dtp, const int* __restrict__ cinst, double* __restrict__ lduh,
                         double* __restrict__ lQhbnd, double* __restrict__ lFhbnd, int* __restrict__ picard,
