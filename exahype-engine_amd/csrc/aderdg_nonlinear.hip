@@ -671,10 +671,13 @@ __device__ __forceinline__ void atomic_min_pos_double(double* addr, double v) {
 
 // *addr = min(*addr, v) where many workgroups share the address: atomics on one
 // line are served one after the other (~10 ns each across the XCDs), so a value
-// that the address already undercuts is not sent.  The value only falls during a
-// launch, so a load that is late costs an atomic and loses nothing.
+// that the address already undercuts is not sent (bit patterns compared, as the
+// atomic does).  The value only falls during a launch, so a load that is late costs
+// an atomic and loses nothing.
 __device__ __forceinline__ void merge_min(double* addr, double v) {
-  if (v < __hip_atomic_load(addr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomic_min_pos_double(addr, v);
+  auto* p = reinterpret_cast<unsigned long long*>(addr);
+  const auto bits = static_cast<unsigned long long>(__double_as_longlong(v));
+  if (bits < __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(p, bits);
 }
 
 // A node's stable dt is CFL*PNPM / den with den = sum_d max_v |lambda_v(Q, d)| / dx

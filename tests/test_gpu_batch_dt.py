@@ -1,0 +1,48 @@
+"""GPU: the stable dt that the batched corrector merges into dt_next.
+
+The result is a minimum of per-cell values, so it is the smallest cell's own value
+bit for bit, wherever that cell lies in the batch.  dt_next is compared by its bit
+pattern, as the device's integer minimum does: +inf and NaN are above every dt.
+"""
+import numpy as np
+import pytest
+import torch
+
+import exahype_amd as E
+
+pytestmark = pytest.mark.gpu
+
+
+def corrected_dt(ctx, luh, start):
+    n, dim, B = len(luh), ctx.dim, ctx.B
+    t = dict(luh=luh.clone(), lduh=torch.zeros(n, B ** dim, 5, dtype=torch.float64, device="cuda"),
+             fb=torch.zeros(n, 2 * dim, B ** (dim - 1), 5, dtype=torch.float64, device="cuda"),
+             h=torch.full((n,), 0.1, dtype=torch.float64, device="cuda"),
+             dt=torch.full((1,), 1e-3, dtype=torch.float64, device="cuda"),
+             next=torch.full((1,), start, dtype=torch.float64, device="cuda"))
+    p = {k: v.data_ptr() for k, v in t.items()}
+    ctx.batch_corrector(torch.cuda.current_stream().cuda_stream, n, p["luh"], p["lduh"], p["fb"], p["h"], p["dt"],
+                        p["next"])
+    torch.cuda.synchronize()
+    return t["next"].item()
+
+
+# (dim, order, cells per workgroup)
+@pytest.mark.parametrize("dim,order,cpb", [(2, 3, 16), (3, 2, 9), (3, 3, 4)])
+def test_minimum_of_the_batch(dim, order, cpb):
+    ctx = E.Context(dim, order)
+    rng = np.random.default_rng(dim * 10 + order)
+    for groups in (1, 2500):
+        n = groups * cpb - 1
+        print(f"[batch dt] dim={dim} order={order} workgroups={groups}", flush=True)
+        luh = torch.zeros(n, (order + 1) ** dim, 5, dtype=torch.float64)
+        luh[..., 0] = 1.0
+        luh[..., 4] = torch.as_tensor(rng.uniform(2.0, 3.0, n))[:, None]
+        fastest = luh[:1].clone()
+        fastest[..., 4] = 4.0
+        want = corrected_dt(ctx, fastest.cuda(), np.finfo(np.float64).max)
+        for at, start in ((0, np.finfo(np.float64).max), (n // 2, np.inf), (n - 1, np.nan)):
+            batch = luh.clone()
+            batch[at] = fastest[0]
+            assert corrected_dt(ctx, batch.cuda(), start) == want, (groups, at)
+    ctx.close()
