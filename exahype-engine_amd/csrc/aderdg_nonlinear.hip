@@ -669,14 +669,32 @@ __device__ __forceinline__ void atomic_min_pos_double(double* addr, double v) {
   atomicMin(reinterpret_cast<unsigned long long*>(addr), static_cast<unsigned long long>(__double_as_longlong(v)));
 }
 
+// Waves per SIMD the corrector's registers aim at.  Left alone the compiler takes
+// eight (60 registers) for the 3D orders 2, 4 and 5 and puts the node's loads one
+// behind the other; with seven (72) they are in flight together: 32,000 cells of
+// order 4, update and dt, 172 -> 157 us, 64 cells 5.2 -> 4.7.
+template <int D, int B>
+constexpr int kCorrectorWaves = D == 3 && (B == 3 || B >= 5) ? 7 : 8;
+
 // *addr = min(*addr, v) where many workgroups share the address: atomics on one
-// line are served one after the other (~10 ns each across the XCDs), so a value
+// line are served one after the other (~14 ns each across the XCDs), so a value
 // that the address already undercuts is not sent (bit patterns compared, as the
 // atomic does).  The value only falls during a launch, so a load that is late costs
 // an atomic and loses nothing.
-__device__ __forceinline__ void merge_min(double* addr, double v) {
+//
+// From some 800 workgroups (in 3D 1,200 with seven waves and 1,700 with eight: their
+// cells end less at once) the first ones to be resident would all load before one
+// atomic has landed and then send theirs: all but 64 of them wait 1.7 us first.
+// New dt and corrector, atomics alone / load / this: 2D order 3, 800 workgroups 17.4
+// / 22.1 / 13.1, 1,200 21.7 / 30.8 / 16.1, 6,000 80.6 / 56.7 / 42.5 us; 3D order 4,
+// 1,200 24.8 / 22.3 / 18.3, 2,100 38.9 / 45.9 / 24.2.  Below the line the wait
+// costs: 2D 700 11.1 -> 11.7, 3D order 3 1,000 14.2 -> 19.3.
+template <int D, int B>
+__device__ __forceinline__ void merge_min(double* addr, double v, long blk) {
+  constexpr unsigned kBurst = D == 2 ? 750 : (kCorrectorWaves<D, B> == 7 ? 1100 : 1600);
   auto* p = reinterpret_cast<unsigned long long*>(addr);
   const auto bits = static_cast<unsigned long long>(__double_as_longlong(v));
+  if (gridDim.x > kBurst && blk >= 64 && blk < 2048) __builtin_amdgcn_s_sleep(64);
   if (bits < __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(p, bits);
 }
 
@@ -806,7 +824,7 @@ __device__ __forceinline__ void corrector_tile(
     if (slots)
       atomic_min_pos_double(slots + (long(i) * nslots + blk % nslots) * kDtSlotStride, v);
     else
-      merge_min(dt_next + i, v);
+      merge_min<D, B>(dt_next + i, v, blk);
   };
   const bool uniform = !cinst || cinst[first] == cinst[last];
   if (uniform) {
@@ -823,7 +841,8 @@ __device__ __forceinline__ void corrector_tile(
 }
 
 template <int D, int B, int V, int NP>
-__global__ __launch_bounds__((Shape<D, B, V, NP>::THREADS)) void corrector_kernel(
+__global__ __launch_bounds__((Shape<D, B, V, NP>::THREADS))
+__attribute__((amdgpu_waves_per_eu(4, kCorrectorWaves<D, B>))) void corrector_kernel(
     long ncells, long ntiles, double* __restrict__ luh, const double* __restrict__ lduh,
     const double* __restrict__ lFhbnd, const double* __restrict__ hcell, const double* __restrict__ dtp,
     const int* __restrict__ cinst, double* __restrict__ dt_next, const DevTables* __restrict__ T, PdeParams P,

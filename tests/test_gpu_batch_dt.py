@@ -1,4 +1,5 @@
-"""GPU: the stable dt that the batched corrector merges into dt_next.
+"""GPU: the stable dt that the batched corrector merges into dt_next, on both sides
+of the workgroup counts at which its merge changes form.
 
 The result is a minimum of per-cell values, so it is the smallest cell's own value
 bit for bit, wherever that cell lies in the batch.  dt_next is compared by its bit
@@ -27,12 +28,12 @@ def corrected_dt(ctx, luh, start):
     return t["next"].item()
 
 
-# (dim, order, cells per workgroup)
-@pytest.mark.parametrize("dim,order,cpb", [(2, 3, 16), (3, 2, 9), (3, 3, 4)])
-def test_minimum_of_the_batch(dim, order, cpb):
+# (dim, order, cells per workgroup, workgroups at the line)
+@pytest.mark.parametrize("dim,order,cpb,line", [(2, 3, 16, 750), (3, 2, 9, 1100), (3, 3, 4, 1600)])
+def test_minimum_of_the_batch(dim, order, cpb, line):
     ctx = E.Context(dim, order)
     rng = np.random.default_rng(dim * 10 + order)
-    for groups in (1, 2500):
+    for groups in (1, line, line + 1, 2500):
         n = groups * cpb - 1
         print(f"[batch dt] dim={dim} order={order} workgroups={groups}", flush=True)
         luh = torch.zeros(n, (order + 1) ** dim, 5, dtype=torch.float64)
