@@ -569,10 +569,14 @@ __global__ __launch_bounds__((Shape<D, B, V, NP>::THREADS), 1) void predictor_ke
 // Lanes per face: the face nodes rounded up to a power of two, so that a
 // wavefront takes 64 / kFaceLanes faces (2D order 3: sixteen of four nodes
 // where one wavefront per face leaves 60 lanes idle; 3D order 4: two).  25,000
-// cells of 2D order 4: 66 -> 23 us; 12,167 shuffled cells of 3D order 4, bound
-// by their 220 MB: 66 us either way.
+// cells of 2D order 4: 66 -> 23 us.
 template <int NF>
 constexpr int kFaceLanes = NF >= 64 ? 64 : next_pow2(NF);
+// 3D order 4 (25 nodes): two faces a wavefront while the faces are few, one when they
+// are many, then bound by HBM, where half as many wavefronts keep less in flight (one
+// -> two faces: 3,000 9.4 -> 8.5, 7,500 17.2 -> 14.9, 12,000 23.2 -> 23.6, 36,000 58 ->
+// 60 to 67 us).
+constexpr long kWaveFaces = 10000;
 
 // Sum over a group of G lanes (every lane of the group ends with the same bits).
 template <int G>
@@ -585,14 +589,14 @@ __device__ __forceinline__ double group_sum(double v) {
 // Face entry (x, y, d, w): left cell x (its face 2d+1), right cell y (its
 // face 2d); with ghost faces given, w & 2 (w & 1): the left (right) side is
 // ghost face x (y) instead.
-template <int D, int B, int V, int NP>
+template <int D, int B, int V, int NP, int G>
 __global__ __launch_bounds__(256) void riemann_kernel(long nfaces, const int4* __restrict__ faces,
                                                       const double* __restrict__ lQhbnd,
                                                       double* __restrict__ lFhbnd, const double* __restrict__ gq,
                                                       double* __restrict__ gf, const DevTables* __restrict__ T,
                                                       PdeParams P) {
   using S = Shape<D, B, V, NP>;
-  constexpr int ND = S::ND, NF = S::NF, G = kFaceLanes<NF>;
+  constexpr int ND = S::ND, NF = S::NF;
   const int lane = threadIdx.x & (G - 1);
   const long f = (long)blockIdx.x * (blockDim.x / G) + threadIdx.x / G;
   if (f >= nfaces) return;  // uniform per group of G lanes; the sums stay in the group, no block barriers below
@@ -1279,14 +1283,22 @@ struct Launch {
     return D == 3 ? launch_predictor_columns_3d(k, st, n, luh, h, dt, lduh, qb, fb, pic, o)
                   : launch_predictor_columns_2d(k, st, n, luh, h, dt, lduh, qb, fb, pic, o);
   }
+  template <int G>
+  static void riemann_groups(const KernelCfg& k, hipStream_t st, long nf, const int* faces, const double* qb, double* fb,
+                             const LaunchOpts& o, int waves) {
+    const long per = waves * (64 / G);  // faces per workgroup
+    hipLaunchKernelGGL((riemann_kernel<D, B, V, NP, G>), dim3(unsigned((nf + per - 1) / per)), dim3(64 * waves), 0, st, nf,
+                       reinterpret_cast<const int4*>(faces), qb, fb, o.ghost_q, o.ghost_f, k.tab, k.pde);
+  }
   static int riemann(const KernelCfg& k, hipStream_t st, long nf, const int* faces, const double* qb,
                      double* fb, const LaunchOpts& o) {
     // riemann_kernel is compiled for at most 256 threads (4 waves) per workgroup
     const int waves = (o.riemann_waves >= 1 && o.riemann_waves <= 4) ? o.riemann_waves : 4;
-    const long per = waves * (64 / kFaceLanes<S::NF>);  // faces per workgroup
-    const long blocks = (nf + per - 1) / per;
-    hipLaunchKernelGGL((riemann_kernel<D, B, V, NP>), dim3(blocks), dim3(64 * waves), 0, st, nf,
-                       reinterpret_cast<const int4*>(faces), qb, fb, o.ghost_q, o.ghost_f, k.tab, k.pde);
+    constexpr int G = kFaceLanes<S::NF>;
+    if (G == 32 && nf > kWaveFaces)
+      riemann_groups<64>(k, st, nf, faces, qb, fb, o, waves);
+    else
+      riemann_groups<G>(k, st, nf, faces, qb, fb, o, waves);
     return static_cast<int>(hipGetLastError());
   }
   static int corrector(const KernelCfg& k, hipStream_t st, long n, double* luh, double* lduh, const double* fb,

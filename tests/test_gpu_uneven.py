@@ -7,11 +7,15 @@
   their stable-dt minima are merged cell by cell; again after the autotuner,
   whose trials must leave no minima behind.
 
+* a list of more 3D order 4 faces than two share a wavefront, against the same
+  faces in two lists that are shorter, bit for bit (a face's sums are the same).
+
 <= 1e-12 relative L2 (the FP64 parity bar); dt to 1e-13, as a minimum of values
 that differ by rounding.
 """
 import numpy as np
 import pytest
+import torch
 
 import exahype_amd as E
 from exahype_amd import problems as P
@@ -71,3 +75,23 @@ def test_ensemble_workgroups_with_several_instances(dim, order):
         for i, (ref, dt) in enumerate(refs):
             assert rel_l2(ens.get_solution(i), ref) <= 1e-12, (tuned, i)
             assert abs(ens.time(i)[1] - dt) <= 1e-13 * dt, (tuned, i)
+
+
+def test_long_and_short_face_lists():
+    print("[uneven] face lists", flush=True)
+    ctx = E.Context(3, 4)
+    n, s = 3334, torch.cuda.current_stream().cuda_stream
+    i = torch.arange(n, dtype=torch.int32)
+    faces = torch.cat([torch.stack([i, (i + 7) % n, torch.full_like(i, d), torch.zeros_like(i)], 1)
+                       for d in range(3)]).contiguous().cuda()  # 10,002
+    g = torch.Generator().manual_seed(3)
+    qb = 1.0 + torch.rand(n, 6, 25, 5, generator=g, dtype=torch.float64)
+    qb[..., 4] += 8.0
+    fb = torch.rand(n, 6, 25, 5, generator=g, dtype=torch.float64)
+    qb, long, short = qb.cuda(), fb.cuda(), fb.cuda()
+    ctx.batch_riemann(s, len(faces), faces.data_ptr(), qb.data_ptr(), long.data_ptr())
+    for part in (faces[:5001], faces[5001:]):
+        ctx.batch_riemann(s, len(part), part.data_ptr(), qb.data_ptr(), short.data_ptr())
+    torch.cuda.synchronize()
+    assert torch.equal(long, short) and not torch.equal(long, fb.cuda())
+    ctx.close()
