@@ -288,7 +288,10 @@ __device__ __forceinline__ void line_derivatives(const double* __restrict__ Dm, 
 // registers.  The corrected p of a cell with receivers goes to rec_p.  Bound by
 // HBM (u in and out, own faces in, neighbours' from the caches, faces out: 2.8 GB
 // at 54^3 of order 4 where predictor and corrector move 4.0) and the LDS reads of the levels: 0.95 ms a step
-// there instead of 0.64 + 0.40.
+// there instead of 0.64 + 0.40.  Order 5 steps in two kernels: with the corrected
+// state beside the levels 50 registers spill (27^3, ten steps: 3.20 ms fused, 2.53
+// in two kernels).
+constexpr int kAcFusedOrder = 4;
 template <int B, bool UPDATE, bool SPLIT, bool CORR = false>
 __global__ void __launch_bounds__((AcLineShape<B>::THREADS), 2) ac_predict_lines_kernel(AcousticArgs a) {
   using S = AcLineShape<B>;
@@ -882,12 +885,15 @@ int launch_all(int which, const AcousticArgs& a, hipStream_t s) {
         ac_predict_kernel<B, true><<<blocks, kAcThreads, 0, s>>>(a);
       break;
     case kAcStep:
-      if (a.pred_variant != 0) return -1;  // the x-line form
-      if (a.split_ck)
-        ac_predict_lines_kernel<B, true, true, true><<<lblocks, AcLineShape<B>::THREADS, 0, s>>>(a);
-      else
-        ac_predict_lines_kernel<B, true, false, true><<<lblocks, AcLineShape<B>::THREADS, 0, s>>>(a);
-      break;
+      if constexpr (B - 1 <= kAcFusedOrder) {
+        if (a.pred_variant != 0) return -1;  // the x-line form
+        if (a.split_ck)
+          ac_predict_lines_kernel<B, true, true, true><<<lblocks, AcLineShape<B>::THREADS, 0, s>>>(a);
+        else
+          ac_predict_lines_kernel<B, true, false, true><<<lblocks, AcLineShape<B>::THREADS, 0, s>>>(a);
+        break;
+      }
+      return -1;
     case kAcPredictFaces:
       if (a.split_ck) return -1;  // the adjoint sweeps transpose the generic predictor only
       if (a.pred_variant == 0)
@@ -917,6 +923,7 @@ int launch_all(int which, const AcousticArgs& a, hipStream_t s) {
 
 }  // namespace
 
+bool acoustic_steps_fused(int order) { return order <= kAcFusedOrder; }
 bool acoustic_order_supported(int order) { return order >= 1 && order <= 5; }
 
 int launch_acoustic(int which, int order, const AcousticArgs& a, hipStream_t s) {

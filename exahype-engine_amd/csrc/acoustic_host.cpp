@@ -290,9 +290,10 @@ int enqueue_forward(exa_acoustic* ac, double* u, double* u_out, int step, double
 }
 
 // nsteps forward steps on d_u from step s0, receivers as enqueue_forward: the
-// corrector of a step and the predictor of the next run as one kernel.
+// corrector of a step and the predictor of the next run as one kernel where the
+// order has one.
 int enqueue_forward_steps(exa_acoustic* ac, int s0, int nsteps, double* rec) {
-  if (nsteps < 2 || ac->pred_variant != 0) {
+  if (nsteps < 2 || ac->pred_variant != 0 || !exa::acoustic_steps_fused(ac->k.order)) {
     for (int i = 0; i < nsteps; i++) RC_OK(enqueue_forward(ac, ac->d_u, ac->d_u, s0 + i, rec));
     return EXA_OK;
   }

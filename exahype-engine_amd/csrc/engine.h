@@ -296,6 +296,7 @@ struct AcousticArgs {
 // kAcStep: corrector of a step and predictor of the next (step_override) in one kernel
 enum { kAcPredictUpdate = 0, kAcStep, kAcPredictFaces, kAcCorrector, kAcFbar, kAcAdjoint, kAcReceivers };
 bool acoustic_order_supported(int order);
+bool acoustic_steps_fused(int order);  // kAcStep is compiled for the order
 int launch_acoustic(int which, int order, const AcousticArgs& a, hipStream_t s);
 int launch_acoustic_receivers_adj(int order, const AcousticArgs& a, const double* res, hipStream_t s);
 int launch_acoustic_advance(int* step, hipStream_t s);
