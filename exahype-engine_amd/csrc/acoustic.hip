@@ -209,7 +209,7 @@ __global__ void __launch_bounds__(kAcThreads) ac_predict_kernel(AcousticArgs a) 
 // derivative sums are scaled by 1/h after summation (rounding differs from
 // the node form at the 1e-16 level).
 // ---------------------------------------------------------------------------
-template <int B>
+template <int B, int T = (B <= 4 ? 64 : 128)>
 struct AcLineShape {
   static constexpr int N = B * B * B;
   static constexpr int F = B * B;    // lines per cell
@@ -219,7 +219,7 @@ struct AcLineShape {
   // small workgroups: more of them fit beside each other on a CU, so that one
   // computes while another waits at a barrier or for HBM (order 4 at 54^3: 256
   // lanes 0.709, 128 lanes 0.639, 64 lanes, of which 50 have a line, 0.691 ms)
-  static constexpr int THREADS = B <= 4 ? 64 : 128;
+  static constexpr int THREADS = T;
   static constexpr int CPB_T = THREADS / F;
   static constexpr int CPB_L = (60 * 1024) / (LDS * 8);
   static constexpr int CPB = CPB_T < CPB_L ? CPB_T : CPB_L;    // cells per block
@@ -292,9 +292,9 @@ __device__ __forceinline__ void line_derivatives(const double* __restrict__ Dm, 
 // state beside the levels 50 registers spill (27^3, ten steps: 3.20 ms fused, 2.53
 // in two kernels).
 constexpr int kAcFusedOrder = 4;
-template <int B, bool UPDATE, bool SPLIT, bool CORR = false>
-__global__ void __launch_bounds__((AcLineShape<B>::THREADS), 2) ac_predict_lines_kernel(AcousticArgs a) {
-  using S = AcLineShape<B>;
+template <int B, bool UPDATE, bool SPLIT, bool CORR = false, int T = AcLineShape<B>::THREADS>
+__global__ void __launch_bounds__(T, 2) ac_predict_lines_kernel(AcousticArgs a) {
+  using S = AcLineShape<B, T>;
   constexpr int N = S::N, F = S::F, CPB = S::CPB;
   __shared__ double smem[CPB * S::LDS];
   const int t = threadIdx.x;
@@ -869,6 +869,39 @@ __global__ void __launch_bounds__((AcAdjShape<B>::THREADS)) ac_adjoint_kernel(Ac
   }
 }
 
+// Whether the line predictor runs in workgroups of 256 lanes instead of 64 or 128
+// (one step's predictor, smaller -> larger):
+// - Orders 2 and 3, once the faces that the step writes exceed some 200 MB and so no
+//   longer stay in the 256 MB last-level cache: HBM is served better by fewer, longer
+//   streams (order 2 48^3 89 / 90, 50^3 113 -> 108, 60^3 199 -> 175; order 3 40^3 126 /
+//   136, 45^3 188 -> 186, 54^3 324 -> 313 us).
+// - Order 4, where the smaller workgroups run a few at a time on each of the 256 CUs
+//   and a CU has as much to do with them as with the larger ones: 13^3 27.2 -> 25.3,
+//   17^3 31.6 -> 31.2 us.  Elsewhere the larger ones leave CUs idle (14^3 28.3 -> 29.6,
+//   18^3 34.6 -> 41.3) or lose the smaller ones' overlap (27^3 86 -> 97).
+template <int B>
+bool large_line_groups(long ncells) {
+  if constexpr (B == 3 || B == 4) return ncells * (6 * B * B * 32) > 200000000L;
+  if constexpr (B == 5) {
+    auto rounds = [&](int cells) { return ((ncells + cells - 1) / cells + 255) / 256; };
+    const long small = rounds(AcLineShape<B>::CPB), large = rounds(AcLineShape<B, 256>::CPB);
+    return small > 1 && small <= 4 && 2 * large <= small;
+  }
+  return false;
+}
+
+template <int B, bool UPDATE, bool SPLIT, int T>
+void predict_lines(const AcousticArgs& a, hipStream_t s) {
+  constexpr int CPB = AcLineShape<B, T>::CPB;
+  ac_predict_lines_kernel<B, UPDATE, SPLIT, false, T><<<unsigned((a.ncells + CPB - 1) / CPB), T, 0, s>>>(a);
+}
+template <int B, bool UPDATE, bool SPLIT>
+void predict_lines(const AcousticArgs& a, hipStream_t s) {
+  if constexpr (B >= 3 && B <= 5)
+    if (large_line_groups<B>(a.ncells)) return predict_lines<B, UPDATE, SPLIT, 256>(a, s);
+  predict_lines<B, UPDATE, SPLIT, AcLineShape<B>::THREADS>(a, s);
+}
+
 template <int B>
 int launch_all(int which, const AcousticArgs& a, hipStream_t s) {
   using S = AcShape<B>;
@@ -878,9 +911,9 @@ int launch_all(int which, const AcousticArgs& a, hipStream_t s) {
     case kAcPredictUpdate:
       if (a.split_ck && a.pred_variant != 0) return -1;  // the split predictor has the x-line form only
       if (a.split_ck)
-        ac_predict_lines_kernel<B, true, true><<<lblocks, AcLineShape<B>::THREADS, 0, s>>>(a);
+        predict_lines<B, true, true>(a, s);
       else if (a.pred_variant == 0)
-        ac_predict_lines_kernel<B, true, false><<<lblocks, AcLineShape<B>::THREADS, 0, s>>>(a);
+        predict_lines<B, true, false>(a, s);
       else
         ac_predict_kernel<B, true><<<blocks, kAcThreads, 0, s>>>(a);
       break;
@@ -897,7 +930,7 @@ int launch_all(int which, const AcousticArgs& a, hipStream_t s) {
     case kAcPredictFaces:
       if (a.split_ck) return -1;  // the adjoint sweeps transpose the generic predictor only
       if (a.pred_variant == 0)
-        ac_predict_lines_kernel<B, false, false><<<lblocks, AcLineShape<B>::THREADS, 0, s>>>(a);
+        predict_lines<B, false, false>(a, s);
       else
         ac_predict_kernel<B, false><<<blocks, kAcThreads, 0, s>>>(a);
       break;

@@ -74,3 +74,32 @@ def test_fused_steps_on_the_smallest_meshes(order, n):
     want, _ = O.LinearOracle(3, order).run(ref, n, h, dt, steps, src, rec)
     assert rel_l2(got, want) <= 1e-12
     assert rel_l2(ac.get_solution(), ref) <= 1e-12
+
+
+@pytest.mark.parametrize("order,n", [(2, 49), (3, 41), (4, 13)])
+def test_line_predictor_in_large_workgroups(order, n):
+    """Sizes at which the line predictor takes 256 lanes, the last workgroup partly empty, against the node
+    form: single steps (predictor and corrector apart), the faces of a gradient, and a captured run."""
+    print(f"[large workgroups] order={order} n={n}", flush=True)
+    rng = np.random.default_rng(order)
+    c, rho = 1.0 + 0.2 * rng.uniform(-1, 1, n ** 3), 1.0 + 0.1 * rng.uniform(-1, 1, n ** 3)
+    luh = P.acoustic_state(n, order, c, rho, 0.1 * rng.normal(size=(n ** 3, (order + 1) ** 3, 4)))
+    ac = E.Acoustic(E.Context(3, order, 4, 2, E.PDE_ACOUSTIC), n, 1.0 / n)
+    ac.set_dt(0.0)
+    ac.set_source((0.4, 0.6, 0.3), 1.0, 5.0, 0.05)
+    ac.set_receivers(rng.uniform(0.05, 0.95, size=(6, 3)))
+    obs = rng.normal(0.0, 0.1, (2, 6))
+    got = []
+    for variant in (0, 1):
+        ac.set_predictor(variant)
+        ac.set_solution(luh)
+        ac.set_step(0)
+        ac.run(1)
+        ac.run(1)
+        u = ac.get_solution()
+        J, g = ac.misfit_gradient(2, obs, checkpoint_every=1)
+        ac.run(2, use_graph=True)
+        got.append((u, g, ac.get_solution()))
+    ac.close()
+    for line, node, tol in zip(*got, (1e-12, 1e-10, 1e-12)):
+        assert rel_l2(line, node) <= tol
