@@ -79,6 +79,7 @@ struct exa_acoustic {
 namespace {
 
 int fail(hipError_t e, const char* what) {
+  (void)hipGetLastError();  // reported here: not by the next launch
   exa::set_error(std::string(what) + ": " + hipGetErrorString(e));
   return EXA_ERR_HIP;
 }

@@ -31,6 +31,7 @@ const KernelCfg& ctx_cfg(const exa_ctx* c);
 namespace {
 
 int fail(hipError_t e, const char* what) {
+  (void)hipGetLastError();  // reported here: not by the next launch
   exa::set_error(std::string(what) + ": " + hipGetErrorString(e));
   return EXA_ERR_HIP;
 }

@@ -55,6 +55,7 @@ struct exa_ctx {
 namespace {
 
 int hip_fail(hipError_t e, const char* what) {
+  (void)hipGetLastError();  // reported here: not by the next launch
   set_error(std::string(what) + ": " + hipGetErrorString(e));
   return EXA_ERR_HIP;
 }

@@ -1,0 +1,248 @@
+// Host logic of the acoustic mesh on a device made of host memory: the source file
+// itself, with the HIP calls it makes and the kernel launches replaced below.
+//
+// Memory is counted and can run out.  A launch checks that every array it gets is
+// live and large enough and writes in its first value what it then holds (the state
+// before step k: 10 k, with the volume update of step k: 10 k + 5, the faces and
+// the cotangents of step k: k), so that each kernel can check that its inputs are
+// those of its step.
+//
+// usage: acoustic_host_check <scenario>; prints what is wrong and exits 1.
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+
+#include "../../exahype-engine_amd/csrc/acoustic_host.cpp"
+
+namespace {
+std::map<char*, size_t> live;
+size_t used = 0, limit = size_t(1) << 40;
+int fail_at = 0, mallocs = 0, steps_fused = 0, face_launches = 0;
+hipError_t last_error = hipSuccess;
+
+#define CHECK(cond)                                             \
+  do {                                                          \
+    if (!(cond)) {                                              \
+      std::printf("line %d: %s\n", __LINE__, #cond);            \
+      std::exit(1);                                             \
+    }                                                           \
+  } while (0)
+
+// the bytes from p to the end of its allocation
+size_t room(const void* p) {
+  auto it = live.upper_bound(static_cast<char*>(const_cast<void*>(p)));
+  if (!p || it == live.begin()) return 0;
+  --it;
+  const size_t off = static_cast<const char*>(p) - it->first;
+  return off < it->second ? it->second - off : 0;
+}
+bool holds(const void* p, size_t doubles) { return room(p) >= doubles * sizeof(double); }
+}  // namespace
+
+extern "C" {
+hipError_t hipMalloc(void** p, size_t n) {
+  if (++mallocs == fail_at || used + n > limit) return last_error = hipErrorOutOfMemory;
+  *p = std::calloc(1, n);
+  live[static_cast<char*>(*p)] = n;
+  used += n;
+  return hipSuccess;
+}
+hipError_t hipFree(void* p) {
+  auto it = live.find(static_cast<char*>(p));
+  CHECK(!p || it != live.end());
+  if (!p) return hipSuccess;
+  used -= it->second;
+  live.erase(it);
+  std::free(p);
+  return hipSuccess;
+}
+hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind kind) {
+  if (kind != hipMemcpyDeviceToHost) CHECK(room(d) >= n);
+  if (kind != hipMemcpyHostToDevice) CHECK(room(s) >= n);
+  std::memcpy(d, s, n);
+  return hipSuccess;
+}
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind kind, hipStream_t) {
+  return hipMemcpy(d, s, n, kind);
+}
+hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t) {
+  CHECK(room(d) >= n);
+  std::memset(d, v, n);
+  return hipSuccess;
+}
+hipError_t hipMemGetInfo(size_t* free, size_t* total) {
+  *free = used > limit ? 0 : limit - used;
+  *total = limit;
+  return hipSuccess;
+}
+hipError_t hipGetLastError() {
+  const hipError_t e = last_error;
+  last_error = hipSuccess;
+  return e;
+}
+hipError_t hipGetDevice(int* d) { return *d = 0, hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t* e) { return *e = reinterpret_cast<hipEvent_t>(1), hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { return *ms = 0, hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+const char* hipGetErrorString(hipError_t) { return "out of memory"; }
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { return *s = reinterpret_cast<hipStream_t>(1), hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipErrorUnknown; }
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t*) { return hipErrorUnknown; }
+hipError_t hipGraphInstantiate(hipGraphExec_t*, hipGraph_t, hipGraphNode_t*, char*, size_t) { return hipErrorUnknown; }
+hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipErrorUnknown; }
+hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
+hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
+int roctxRangePushA(const char*) { return 0; }
+int roctxRangePop() { return 0; }
+}
+
+namespace exa {
+static KernelCfg cfg;
+const KernelCfg& ctx_cfg(const exa_ctx*) { return cfg; }
+void set_error(const std::string&) {}
+bool acoustic_order_supported(int order) { return order >= 1 && order <= 5; }
+bool acoustic_steps_fused(int order) { return order <= 4; }
+
+int launch_acoustic(int which, int order, const AcousticArgs& a, hipStream_t) {
+  const int B = order + 1, k = a.step_override;
+  const size_t su = size_t(a.ncells) * B * B * B * 4, sq = size_t(a.ncells) * 6 * B * B * 4;
+  CHECK(holds(a.mat, 2 * a.ncells) && holds(a.u, su));
+  switch (which) {
+    case kAcPredictUpdate:
+      CHECK(holds(a.u_out, su) && holds(a.qb, sq) && a.qb == a.qb_out && a.u[0] == 10 * k);
+      a.u_out[0] = 10 * k + 5;
+      a.qb_out[0] = k;
+      break;
+    case kAcStep:
+      CHECK(acoustic_steps_fused(order) && a.u == a.u_out && holds(a.qb, sq) && holds(a.qb_out, sq) && a.qb != a.qb_out);
+      CHECK(a.u[0] == 10 * (k - 1) + 5 && a.qb[0] == k - 1);
+      if (a.rec_p) {
+        CHECK(holds(a.rec_p, size_t(a.nrec) * B * B * B) && room(a.rstart) >= sizeof(int) * (a.ncells + 1));
+        a.rec_p[0] = 10 * k;
+      }
+      a.u[0] = 10 * k + 5;
+      a.qb_out[0] = k;
+      steps_fused++;
+      break;
+    case kAcCorrector:
+      CHECK(holds(a.qb, sq) && a.u[0] == 10 * k + 5 && a.qb[0] == k);
+      a.u[0] = 10 * (k + 1);
+      break;
+    case kAcPredictFaces:
+      CHECK(holds(a.qb_out, sq) && a.u[0] == 10 * k);
+      a.qb_out[0] = k;
+      face_launches++;
+      break;
+    case kAcReceivers:
+      CHECK(holds(a.rec + long(k) * a.nrec, a.nrec) && (a.rec_p ? a.rec_p[0] : a.u[0]) == 10 * (k + 1));
+      for (int r = 0; r < a.nrec; r++) a.rec[long(k) * a.nrec + r] = k;
+      break;
+    case kAcFbar:
+      CHECK(holds(a.ubar, su) && holds(a.fbar, sq) && a.ubar[0] == k + 1);
+      a.fbar[0] = k + 1;
+      break;
+    case kAcAdjoint:
+      CHECK(holds(a.ubar, su) && holds(a.fbar, sq) && holds(a.fbar_out, sq) && a.fbar != a.fbar_out &&
+            holds(a.gc, a.ncells) && holds(a.qb, sq));
+      CHECK(a.u[0] == 10 * k && a.qb[0] == k && a.ubar[0] == k + 1 && a.fbar[0] == k + 1);
+      a.ubar[0] = k;
+      if (a.res_prev) {
+        CHECK(holds(a.res_prev, a.nrec) && a.res_prev[0] == k - 1 && room(a.rorder) >= sizeof(int) * a.nrec);
+        a.fbar_out[0] = k;
+      }
+      a.gc[0] += 1;
+      break;
+  }
+  return static_cast<int>(hipGetLastError());
+}
+int launch_acoustic_receivers_adj(int, const AcousticArgs& a, const double* res, hipStream_t) {
+  CHECK(holds(res, a.nrec));
+  a.ubar[0] = res[0] + 1;  // the residual of step k is k
+  return static_cast<int>(hipGetLastError());
+}
+int launch_acoustic_advance(int* step, hipStream_t) { return ++*step, 0; }
+}  // namespace exa
+
+namespace {
+exa_acoustic* mesh(int order, int n = 2) {
+  exa::cfg.pde.id = EXA_PDE_ACOUSTIC;
+  exa::cfg.dim = 3, exa::cfg.order = order, exa::cfg.nvar = 4, exa::cfg.npar = 2;
+  exa::cfg.precision = EXA_PREC_FP64, exa::cfg.cfl = 0.9, exa::cfg.pnpm = 0.1;
+  exa_acoustic* ac = nullptr;
+  return exa_acoustic_create(&ac, reinterpret_cast<exa_ctx*>(&exa::cfg), n, 1.0 / n) ? nullptr : ac;
+}
+int receivers(exa_acoustic* ac, int nrec) {
+  std::vector<double> x(3 * nrec, 0.3);
+  return exa_acoustic_set_receivers(ac, nrec, x.data());
+}
+void rewind(exa_acoustic* ac) {
+  ac->d_u[0] = 0;
+  CHECK(exa_acoustic_set_step(ac, 0) == EXA_OK);
+}
+int run(exa_acoustic* ac, int steps) {
+  rewind(ac);
+  std::vector<double> rec(size_t(steps) * (ac->nrec ? ac->nrec : 1), -1);
+  const int rc = exa_acoustic_run(ac, steps, 0, rec.data());
+  if (rc) return rc;
+  CHECK(ac->d_u[0] == 10 * steps);
+  for (int k = 0; k < steps && ac->nrec; k++) CHECK(rec[size_t(k) * ac->nrec] == k);
+  return EXA_OK;
+}
+int gradient(exa_acoustic* ac, int steps, int every) {
+  rewind(ac);
+  std::vector<double> obs(size_t(steps) * ac->nrec, 0), g(ac->nc);
+  double J = 0;
+  const int rc = exa_acoustic_misfit_gradient(ac, steps, every, obs.data(), &J, g.data());
+  if (rc) return rc;
+  CHECK(g[0] == steps && ac->d_u[0] == 10 * steps);
+  return EXA_OK;
+}
+size_t su(const exa_acoustic* ac) { return sizeof(double) * ac->nc * ac->N * 4; }
+size_t sq(const exa_acoustic* ac) { return sizeof(double) * ac->nc * 6 * ac->F * 4; }
+
+// every path of run and gradient, one object after other calls and fresh ones
+void dataflow() {
+  for (int order : {1, 4, 5}) {
+    exa_acoustic* ac = mesh(order);
+    for (int nrec : {3, 1, 5})
+      for (int variant : {0, 1})
+        for (int steps : {1, 2, 7, 12})
+          for (int every : {1, 3, 5, 12, 50, 2}) {
+            CHECK(!receivers(ac, nrec) && !exa_acoustic_set_predictor(ac, variant));
+            CHECK(!run(ac, steps) && !gradient(ac, steps, every));
+          }
+    CHECK(!receivers(ac, 0) && !run(ac, 3));
+    CHECK(order == 5 || steps_fused > 0);
+    CHECK(exa_acoustic_destroy(ac) == EXA_OK && used == 0);
+  }
+}
+
+// a failed call has reported its error: the next one's launches do not
+void stale_error() {
+  for (int at = 1; at <= 5; at++) {
+    mallocs = 0, fail_at = at;
+    CHECK(!mesh(4) && used == 0);
+    fail_at = 0;
+    exa_acoustic* ac = mesh(4);
+    CHECK(ac && !run(ac, 3));
+    exa_acoustic_destroy(ac);
+  }
+}
+}  // namespace
+
+int main(int argc, char** argv) {
+  const std::map<std::string, void (*)()> scenarios = {
+      {"dataflow", dataflow},
+      {"stale_error", stale_error},
+  };
+  const auto it = scenarios.find(argc > 1 ? argv[1] : "");
+  if (it == scenarios.end()) return 2;
+  it->second();
+  std::puts("ok");
+  return 0;
+}
