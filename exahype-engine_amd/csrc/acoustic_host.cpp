@@ -675,12 +675,12 @@ int exa_acoustic_misfit_gradient(exa_acoustic* ac, int nsteps, int every, const 
   RC_OK(ensure_source_table(ac, s0 + K));
   RC_OK(grow(&ac->d_rec, &ac->rec_cap, long(K) * R));
   RC_OK(grow(&ac->d_res, &ac->res_cap, long(K) * R));
-  if (!ac->d_ubar) {
-    HIP_OK(hipMalloc(&ac->d_ubar, sizeof(double) * su), "hipMalloc(adjoint)");
-    HIP_OK(hipMalloc(&ac->d_fbar, sizeof(double) * sq), "hipMalloc(adjoint)");
-    HIP_OK(hipMalloc(&ac->d_fbar2, sizeof(double) * sq), "hipMalloc(adjoint)");
-    HIP_OK(hipMalloc(&ac->d_gc, sizeof(double) * ac->nc), "hipMalloc(adjoint)");
-  }
+  struct {
+    double** p;
+    size_t n;
+  } const adjoint[] = {{&ac->d_ubar, su}, {&ac->d_fbar, sq}, {&ac->d_fbar2, sq}, {&ac->d_gc, size_t(ac->nc)}};
+  for (const auto& b : adjoint)  // each by itself: an earlier call may have got only some of them
+    if (!*b.p) HIP_OK(hipMalloc(b.p, sizeof(double) * b.n), "hipMalloc(adjoint)");
   {
     const int rb = gradient_buffers(ac, su, sq, nck, seg);
     if (rb) {

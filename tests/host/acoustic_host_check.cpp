@@ -233,12 +233,27 @@ void stale_error() {
     exa_acoustic_destroy(ac);
   }
 }
+// an allocation that fails leaves an object that can be used again
+void failed_allocation() {
+  for (int at = 1; at < 16; at++) {
+    exa_acoustic* ac = mesh(4);
+    CHECK(!receivers(ac, 2));
+    mallocs = 0, fail_at = at;
+    (void)gradient(ac, 5, 2);
+    fail_at = 0;
+    CHECK(!gradient(ac, 5, 2) && !run(ac, 4));
+    exa_acoustic_destroy(ac);
+    CHECK(used == 0);
+  }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::map<std::string, void (*)()> scenarios = {
       {"dataflow", dataflow},
       {"stale_error", stale_error},
+      {"failed_allocation", failed_allocation},
   };
   const auto it = scenarios.find(argc > 1 ? argv[1] : "");
   if (it == scenarios.end()) return 2;

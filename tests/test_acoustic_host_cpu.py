@@ -8,7 +8,7 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
-SCENARIOS = ["dataflow", "stale_error"]
+SCENARIOS = ["dataflow", "stale_error", "failed_allocation"]
 
 
 @pytest.fixture(scope="module")
