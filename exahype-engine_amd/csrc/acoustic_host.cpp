@@ -290,17 +290,32 @@ int enqueue_forward(exa_acoustic* ac, double* u, double* u_out, int step, double
   return EXA_OK;
 }
 
+// The buffers of the fused steps; false: not enough memory for them, steps in two kernels.
+bool fused_buffers(exa_acoustic* ac, bool receive) {
+  struct {
+    double** p;
+    long n;
+  } const need[] = {{&ac->d_qb2, ac->nc * 6 * ac->F * 4}, {&ac->d_rec_p, receive ? long(ac->nrec) * ac->N : 0}};
+  for (const auto& b : need) {
+    if (*b.p || b.n == 0) continue;
+    if (hipMalloc(b.p, sizeof(double) * b.n) != hipSuccess) {
+      *b.p = nullptr;
+      (void)hipGetLastError();
+      return false;
+    }
+  }
+  return true;
+}
+
 // nsteps forward steps on d_u from step s0, receivers as enqueue_forward: the
 // corrector of a step and the predictor of the next run as one kernel where the
-// order has one.
+// order has one and there is memory for its second face buffer.
 int enqueue_forward_steps(exa_acoustic* ac, int s0, int nsteps, double* rec) {
-  if (nsteps < 2 || ac->pred_variant != 0 || !exa::acoustic_steps_fused(ac->k.order)) {
+  const bool receive = rec && ac->nrec > 0;
+  if (nsteps < 2 || ac->pred_variant != 0 || !exa::acoustic_steps_fused(ac->k.order) || !fused_buffers(ac, receive)) {
     for (int i = 0; i < nsteps; i++) RC_OK(enqueue_forward(ac, ac->d_u, ac->d_u, s0 + i, rec));
     return EXA_OK;
   }
-  if (!ac->d_qb2) HIP_OK(hipMalloc(&ac->d_qb2, sizeof(double) * ac->nc * 6 * ac->F * 4), "hipMalloc(faces)");
-  const bool receive = rec && ac->nrec > 0;
-  if (receive && !ac->d_rec_p) HIP_OK(hipMalloc(&ac->d_rec_p, sizeof(double) * ac->nrec * ac->N), "hipMalloc(receivers)");
   exa::TraceRange tr("exa.acoustic.steps");
   const int o = ac->k.order;
   exa::AcousticArgs a = args(ac, ac->d_u);

@@ -247,6 +247,23 @@ void failed_allocation() {
   }
 }
 
+
+// a mesh that leaves no room for the second face buffer, or for the receivers' p, steps without
+void no_second_faces() {
+  for (int nrec : {0, 2}) {
+    exa_acoustic* ac = mesh(4);
+    CHECK(!receivers(ac, nrec));
+    steps_fused = 0;
+    limit = used + sq(ac) - 1;  // the steps' records fit
+    CHECK(!run(ac, 5) && !run(ac, 5) && steps_fused == 0);
+    limit = used + sq(ac) + 1;
+    CHECK(!run(ac, 5) && (steps_fused > 0) == (nrec == 0));
+    limit = size_t(1) << 40;
+    CHECK(!run(ac, 5) && steps_fused > 0);
+    exa_acoustic_destroy(ac);
+    CHECK(used == 0);
+  }
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -254,6 +271,7 @@ int main(int argc, char** argv) {
       {"dataflow", dataflow},
       {"stale_error", stale_error},
       {"failed_allocation", failed_allocation},
+      {"no_second_faces", no_second_faces},
   };
   const auto it = scenarios.find(argc > 1 ? argv[1] : "");
   if (it == scenarios.end()) return 2;
