@@ -134,14 +134,51 @@ long locate(const exa_acoustic* ac, const double* p, double* xi) {
   return (long(ic[2]) * ac->n + ic[1]) * ac->n + ic[0];
 }
 
-int grow(double** p, long* cap, long need) {
+// Frees what a mesh holds only to save time: the fused steps' and the gradient's buffers.
+void free_optional(exa_acoustic* ac) {
+  for (double** p : {&ac->d_qb2, &ac->d_rec_p, &ac->d_ck, &ac->d_seg, &ac->d_segq}) {
+    if (*p) (void)hipFree(*p);
+    *p = nullptr;
+  }
+  ac->ck_cap = ac->seg_cap = ac->segq_cap = 0;
+}
+
+// hipMalloc of what a call cannot do without; before it uses an optional buffer
+template <typename T>
+hipError_t allocate(exa_acoustic* ac, T** p, size_t n) {
+  hipError_t e = hipMalloc(p, sizeof(T) * n);
+  if (e == hipSuccess) return e;
+  (void)hipGetLastError();
+  free_optional(ac);
+  e = hipMalloc(p, sizeof(T) * n);
+  if (e != hipSuccess) *p = nullptr;
+  return e;
+}
+// of what it can: false (and no error left) without memory for it
+bool try_allocate(double** p, size_t n) {
+  if (hipMalloc(p, sizeof(double) * n) == hipSuccess) return true;
+  (void)hipGetLastError();
+  *p = nullptr;
+  return false;
+}
+
+int grow(exa_acoustic* ac, double** p, long* cap, long need) {
   if (*cap >= need) return EXA_OK;
   if (*p) (void)hipFree(*p);
   *p = nullptr;
   *cap = 0;
-  HIP_OK(hipMalloc(p, sizeof(double) * need), "hipMalloc");
+  HIP_OK(allocate(ac, p, need), "hipMalloc");
   *cap = need;
   return EXA_OK;
+}
+bool try_grow(double** p, long* cap, long need) {
+  if (*cap >= need) return true;
+  if (*p) (void)hipFree(*p);
+  *p = nullptr;
+  *cap = 0;
+  if (!try_allocate(p, need)) return false;
+  *cap = need;
+  return true;
 }
 
 // Time factors of the source for steps [0, steps).
@@ -203,7 +240,7 @@ int ensure_source_table(exa_acoustic* ac, int steps) {
   if (ac->d_src_tab) (void)hipFree(ac->d_src_tab);
   ac->d_src_tab = nullptr;
   ac->src_tab_steps = 0;
-  HIP_OK(hipMalloc(&ac->d_src_tab, sizeof(double) * tabh.size()), "hipMalloc(source table)");
+  HIP_OK(allocate(ac, &ac->d_src_tab, tabh.size()), "hipMalloc(source table)");
   HIP_OK(hipMemcpy(ac->d_src_tab, tabh.data(), sizeof(double) * tabh.size(), hipMemcpyHostToDevice),
          "upload source table");
   ac->src_tab_steps = cap;
@@ -240,30 +277,34 @@ exa::AcousticArgs args(exa_acoustic* ac, double* u) {
 }
 
 // Buffers of one gradient: grown on demand and kept for the next unless they take
-// more than an eighth of the GPU's memory.  The faces of a segment's steps are
-// kept (and not formed a second time) when they fit a quarter of what is free.
+// more than an eighth of the GPU's memory.  Where they do not fit beside what earlier
+// calls left, that goes first.  The faces of a segment's steps are kept (and not
+// formed a second time) when they fit a quarter of what is free.
 int gradient_buffers(exa_acoustic* ac, size_t su, size_t sq, int nck, int seg) {
-  RC_OK(grow(&ac->d_ck, &ac->ck_cap, long(su) * nck));
-  if (seg > 0) RC_OK(grow(&ac->d_seg, &ac->seg_cap, long(su) * seg));
+  auto states = [&] {
+    return try_grow(&ac->d_ck, &ac->ck_cap, long(su) * nck) && try_grow(&ac->d_seg, &ac->seg_cap, long(su) * seg);
+  };
+  if (!states()) {
+    free_optional(ac);
+    if (!states()) {
+      free_optional(ac);
+      return fail(hipErrorOutOfMemory, "hipMalloc(checkpoints)");
+    }
+  }
   const long faces = long(sq) * (seg + 1);
   if (ac->segq_cap < faces) {
     size_t free = 0, total = 0;
     HIP_OK(hipMemGetInfo(&free, &total), "memory");
-    if (sizeof(double) * size_t(faces) <= free / 4) RC_OK(grow(&ac->d_segq, &ac->segq_cap, faces));
+    if (sizeof(double) * size_t(faces) <= free / 4) (void)try_grow(&ac->d_segq, &ac->segq_cap, faces);
   }
   return EXA_OK;
 }
 
-void release_gradient_buffers(exa_acoustic* ac, bool all) {
+void release_gradient_buffers(exa_acoustic* ac) {
   size_t free = 0, total = 0;
-  if (!all && hipMemGetInfo(&free, &total) == hipSuccess &&
-      sizeof(double) * size_t(ac->ck_cap + ac->seg_cap + ac->segq_cap) <= total / 8)
-    return;
-  for (double** p : {&ac->d_ck, &ac->d_seg, &ac->d_segq}) {
-    if (*p) (void)hipFree(*p);
-    *p = nullptr;
-  }
-  ac->ck_cap = ac->seg_cap = ac->segq_cap = 0;
+  if (hipMemGetInfo(&free, &total) != hipSuccess ||
+      sizeof(double) * size_t(ac->ck_cap + ac->seg_cap + ac->segq_cap) > total / 8)
+    free_optional(ac);
 }
 
 // one forward step from u to u_out (step index `step`, or the device counter if < 0);
@@ -298,11 +339,7 @@ bool fused_buffers(exa_acoustic* ac, bool receive) {
   } const need[] = {{&ac->d_qb2, ac->nc * 6 * ac->F * 4}, {&ac->d_rec_p, receive ? long(ac->nrec) * ac->N : 0}};
   for (const auto& b : need) {
     if (*b.p || b.n == 0) continue;
-    if (hipMalloc(b.p, sizeof(double) * b.n) != hipSuccess) {
-      *b.p = nullptr;
-      (void)hipGetLastError();
-      return false;
-    }
+    if (!try_allocate(b.p, b.n)) return false;
   }
   return true;
 }
@@ -587,12 +624,12 @@ int exa_acoustic_set_receivers(exa_acoustic* ac, int nrec, const double* xr) {
   for (long c = 0; c < ac->nc; c++) start[c + 1] += start[c];
   std::vector<int> at(start.begin(), start.end() - 1);
   for (int r = 0; r < nrec; r++) order[at[cells[r]]++] = r;
-  HIP_OK(hipMalloc(&ac->d_rstart, sizeof(int) * start.size()), "hipMalloc(receivers)");
-  HIP_OK(hipMalloc(&ac->d_rorder, sizeof(int) * nrec), "hipMalloc(receivers)");
+  HIP_OK(allocate(ac, &ac->d_rstart, start.size()), "hipMalloc(receivers)");
+  HIP_OK(allocate(ac, &ac->d_rorder, nrec), "hipMalloc(receivers)");
   HIP_OK(hipMemcpy(ac->d_rstart, start.data(), sizeof(int) * start.size(), hipMemcpyHostToDevice), "upload receivers");
   HIP_OK(hipMemcpy(ac->d_rorder, order.data(), sizeof(int) * nrec, hipMemcpyHostToDevice), "upload receivers");
-  HIP_OK(hipMalloc(&ac->d_rcell, sizeof(int) * nrec), "hipMalloc(receivers)");
-  HIP_OK(hipMalloc(&ac->d_rw, sizeof(double) * wts.size()), "hipMalloc(receivers)");
+  HIP_OK(allocate(ac, &ac->d_rcell, nrec), "hipMalloc(receivers)");
+  HIP_OK(allocate(ac, &ac->d_rw, wts.size()), "hipMalloc(receivers)");
   HIP_OK(hipMemcpy(ac->d_rcell, cells.data(), sizeof(int) * nrec, hipMemcpyHostToDevice), "upload receivers");
   HIP_OK(hipMemcpy(ac->d_rw, wts.data(), sizeof(double) * wts.size(), hipMemcpyHostToDevice), "upload receivers");
   ac->nrec = nrec;
@@ -604,7 +641,7 @@ int exa_acoustic_run(exa_acoustic* ac, int nsteps, int use_graph, double* rec) {
   if (nsteps == 0) return EXA_OK;
   const int s0 = ac->step;
   RC_OK(ensure_source_table(ac, s0 + nsteps));
-  RC_OK(grow(&ac->d_rec, &ac->rec_cap, long(nsteps) * (ac->nrec > 0 ? ac->nrec : 1)));
+  RC_OK(grow(ac, &ac->d_rec, &ac->rec_cap, long(nsteps) * (ac->nrec > 0 ? ac->nrec : 1)));
   hipEvent_t e0 = nullptr, e1 = nullptr;
   HIP_OK(hipEventCreate(&e0), "event");
   HIP_OK(hipEventCreate(&e1), "event");
@@ -688,21 +725,15 @@ int exa_acoustic_misfit_gradient(exa_acoustic* ac, int nsteps, int every, const 
   const int seg = (every < K ? every : K) - 1;  // states of a segment besides its checkpoint
   const size_t su = size_t(ac->nc) * ac->N * 4, sq = size_t(ac->nc) * 6 * ac->F * 4;
   RC_OK(ensure_source_table(ac, s0 + K));
-  RC_OK(grow(&ac->d_rec, &ac->rec_cap, long(K) * R));
-  RC_OK(grow(&ac->d_res, &ac->res_cap, long(K) * R));
+  RC_OK(grow(ac, &ac->d_rec, &ac->rec_cap, long(K) * R));
+  RC_OK(grow(ac, &ac->d_res, &ac->res_cap, long(K) * R));
   struct {
     double** p;
     size_t n;
   } const adjoint[] = {{&ac->d_ubar, su}, {&ac->d_fbar, sq}, {&ac->d_fbar2, sq}, {&ac->d_gc, size_t(ac->nc)}};
   for (const auto& b : adjoint)  // each by itself: an earlier call may have got only some of them
-    if (!*b.p) HIP_OK(hipMalloc(b.p, sizeof(double) * b.n), "hipMalloc(adjoint)");
-  {
-    const int rb = gradient_buffers(ac, su, sq, nck, seg);
-    if (rb) {
-      release_gradient_buffers(ac, true);
-      return rb;
-    }
-  }
+    if (!*b.p) HIP_OK(allocate(ac, b.p, b.n), "hipMalloc(adjoint)");
+  RC_OK(gradient_buffers(ac, su, sq, nck, seg));
   double *d_ck = ac->d_ck, *d_seg = ac->d_seg;
   double* d_segq = ac->segq_cap >= long(sq) * (seg + 1) ? ac->d_segq : nullptr;
   std::vector<hipEvent_t> ev(2 + 3 * nck, nullptr);
@@ -794,7 +825,7 @@ int exa_acoustic_misfit_gradient(exa_acoustic* ac, int nsteps, int every, const 
   (void)hipStreamSynchronize(ac->stream);
   for (auto& e : ev)
     if (e) (void)hipEventDestroy(e);
-  release_gradient_buffers(ac, false);
+  release_gradient_buffers(ac);
   if (rc) return rc;
   *J = Jv;
   return set_step(ac, s0 + K);

@@ -264,6 +264,44 @@ void no_second_faces() {
     CHECK(used == 0);
   }
 }
+
+// a gradient that fits an object of its own fits one that earlier calls left buffers in
+void gradient_without_room() {
+  for (int faces : {0, 1}) {
+    exa_acoustic* ac = mesh(4);
+    CHECK(!receivers(ac, 2) && !run(ac, 12));
+    free_optional(ac);
+    const size_t before = used;
+    CHECK(!gradient(ac, 12, 2));  // six checkpoints, one state
+    free_optional(ac);
+    const size_t own = used - before;
+    // room for the adjoint arrays (there now), one checkpoint and eleven states
+    limit = used + 12 * su(ac);
+    face_launches = 0;
+    CHECK(!gradient(ac, 12, 12) && face_launches == 12 && own > 0);  // no faces kept
+    limit = size_t(1) << 40;
+    CHECK(!gradient(ac, 12, 2) && !run(ac, 3));  // other shapes, faces kept, second face buffer
+    limit = used - sizeof(double) * (ac->ck_cap + ac->seg_cap + ac->segq_cap) - sq(ac) - sizeof(double) * 2 * ac->N + 12 * su(ac);
+    if (faces) limit += 12 * sq(ac);
+    CHECK(!gradient(ac, 12, 12) && !gradient(ac, 12, 2) && !gradient(ac, 12, 12));
+    limit -= su(ac) + (faces ? 12 * sq(ac) : 0);
+    CHECK(gradient(ac, 12, 12) == EXA_ERR_HIP && !gradient(ac, 12, 3) && !run(ac, 12));
+    limit = size_t(1) << 40;
+    CHECK(!gradient(ac, 12, 12));
+    exa_acoustic_destroy(ac);
+    CHECK(used == 0);
+  }
+  // the optional allocations fail one after the other: never an error
+  for (int at = 1; at <= 12; at++) {
+    exa_acoustic* ac = mesh(4);
+    CHECK(!receivers(ac, 2) && !gradient(ac, 6, 2));
+    mallocs = 0, fail_at = at;
+    CHECK(!gradient(ac, 12, 5) && !run(ac, 9));
+    fail_at = 0;
+    exa_acoustic_destroy(ac);
+    CHECK(used == 0);
+  }
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -272,6 +310,7 @@ int main(int argc, char** argv) {
       {"stale_error", stale_error},
       {"failed_allocation", failed_allocation},
       {"no_second_faces", no_second_faces},
+      {"gradient_without_room", gradient_without_room},
   };
   const auto it = scenarios.find(argc > 1 ? argv[1] : "");
   if (it == scenarios.end()) return 2;

@@ -8,7 +8,7 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
-SCENARIOS = ["dataflow", "stale_error", "failed_allocation", "no_second_faces"]
+SCENARIOS = ["dataflow", "stale_error", "failed_allocation", "no_second_faces", "gradient_without_room"]
 
 
 @pytest.fixture(scope="module")
