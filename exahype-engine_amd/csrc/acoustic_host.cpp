@@ -23,6 +23,7 @@
 
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <utility>
 #include <vector>
@@ -74,6 +75,11 @@ struct exa_acoustic {
   std::vector<hipEvent_t> ev;
   int timed_steps = 0;
   int pred_variant = 0;  // forward predictor: 0 x-line form, 1 node form
+  // optional buffers kept between calls
+  int device = 0;
+  size_t device_bytes = 0;  // its memory
+  bool idle = false;        // in the list of meshes that keep some
+  exa_acoustic* next_idle = nullptr;
 };
 
 namespace {
@@ -143,10 +149,59 @@ void free_optional(exa_acoustic* ac) {
   ac->ck_cap = ac->seg_cap = ac->segq_cap = 0;
 }
 
+size_t optional_bytes(const exa_acoustic* ac) {
+  const long doubles = (ac->d_qb2 ? ac->nc * 6 * ac->F * 4 : 0) + (ac->d_rec_p ? long(ac->nrec) * ac->N : 0) +
+                       ac->ck_cap + ac->seg_cap + ac->segq_cap;
+  return sizeof(double) * size_t(doubles);
+}
+
+// Allocating and freeing its optional buffers costs a gradient 6 % at 27^3 of order 4
+// (40 steps) and 40 % at 13^3, so a mesh keeps them for its next call: all meshes of
+// a device together at most an eighth of its memory, and what idle meshes keep is
+// freed as soon as the library cannot allocate something (device_malloc).
+std::mutex idle_mutex;
+exa_acoustic* idle_meshes = nullptr;  // no call in flight, some buffers kept
+
+void unlink_idle(exa_acoustic* ac) {  // idle_mutex held
+  if (!ac->idle) return;
+  exa_acoustic** p = &idle_meshes;
+  while (*p != ac) p = &(*p)->next_idle;
+  *p = ac->next_idle;
+  ac->idle = false;
+}
+
+// A call that may use or free the optional buffers of its mesh.
+class Call {
+ public:
+  explicit Call(exa_acoustic* ac) : ac_(ac) {
+    std::lock_guard<std::mutex> lock(idle_mutex);
+    unlink_idle(ac);
+  }
+  ~Call() {
+    std::lock_guard<std::mutex> lock(idle_mutex);
+    size_t kept = optional_bytes(ac_);
+    if (kept == 0) return;
+    for (const exa_acoustic* m = idle_meshes; m; m = m->next_idle)
+      if (m->device == ac_->device) kept += optional_bytes(m);
+    if (kept > ac_->device_bytes / 8) {
+      free_optional(ac_);
+      return;
+    }
+    ac_->next_idle = idle_meshes;
+    ac_->idle = true;
+    idle_meshes = ac_;
+  }
+  Call(const Call&) = delete;
+  Call& operator=(const Call&) = delete;
+
+ private:
+  exa_acoustic* ac_;
+};
+
 // hipMalloc of what a call cannot do without; before it uses an optional buffer
 template <typename T>
 hipError_t allocate(exa_acoustic* ac, T** p, size_t n) {
-  hipError_t e = hipMalloc(p, sizeof(T) * n);
+  hipError_t e = exa::device_malloc(p, sizeof(T) * n);
   if (e == hipSuccess) return e;
   (void)hipGetLastError();
   free_optional(ac);
@@ -156,7 +211,7 @@ hipError_t allocate(exa_acoustic* ac, T** p, size_t n) {
 }
 // of what it can: false (and no error left) without memory for it
 bool try_allocate(double** p, size_t n) {
-  if (hipMalloc(p, sizeof(double) * n) == hipSuccess) return true;
+  if (exa::device_malloc(p, sizeof(double) * n) == hipSuccess) return true;
   (void)hipGetLastError();
   *p = nullptr;
   return false;
@@ -276,8 +331,7 @@ exa::AcousticArgs args(exa_acoustic* ac, double* u) {
   return a;
 }
 
-// Buffers of one gradient: grown on demand and kept for the next unless they take
-// more than an eighth of the GPU's memory.  Where they do not fit beside what earlier
+// Buffers of one gradient, grown on demand.  Where they do not fit beside what earlier
 // calls left, that goes first.  The faces of a segment's steps are kept (and not
 // formed a second time) when they fit a quarter of what is free.
 int gradient_buffers(exa_acoustic* ac, size_t su, size_t sq, int nck, int seg) {
@@ -298,13 +352,6 @@ int gradient_buffers(exa_acoustic* ac, size_t su, size_t sq, int nck, int seg) {
     if (sizeof(double) * size_t(faces) <= free / 4) (void)try_grow(&ac->d_segq, &ac->segq_cap, faces);
   }
   return EXA_OK;
-}
-
-void release_gradient_buffers(exa_acoustic* ac) {
-  size_t free = 0, total = 0;
-  if (hipMemGetInfo(&free, &total) != hipSuccess ||
-      sizeof(double) * size_t(ac->ck_cap + ac->seg_cap + ac->segq_cap) > total / 8)
-    free_optional(ac);
 }
 
 // one forward step from u to u_out (step index `step`, or the device counter if < 0);
@@ -331,8 +378,11 @@ int enqueue_forward(exa_acoustic* ac, double* u, double* u_out, int step, double
   return EXA_OK;
 }
 
-// The buffers of the fused steps; false: not enough memory for them, steps in two kernels.
-bool fused_buffers(exa_acoustic* ac, bool receive) {
+// The buffers of the fused steps; false: steps in two kernels, for want of memory or
+// because a face buffer too large to keep takes as long to allocate as some six
+// steps gain by it.
+bool fused_buffers(exa_acoustic* ac, bool receive, int nsteps) {
+  if (!ac->d_qb2 && nsteps < 16 && sizeof(double) * ac->nc * 6 * ac->F * 4 > ac->device_bytes / 8) return false;
   struct {
     double** p;
     long n;
@@ -349,7 +399,7 @@ bool fused_buffers(exa_acoustic* ac, bool receive) {
 // order has one and there is memory for its second face buffer.
 int enqueue_forward_steps(exa_acoustic* ac, int s0, int nsteps, double* rec) {
   const bool receive = rec && ac->nrec > 0;
-  if (nsteps < 2 || ac->pred_variant != 0 || !exa::acoustic_steps_fused(ac->k.order) || !fused_buffers(ac, receive)) {
+  if (nsteps < 2 || ac->pred_variant != 0 || !exa::acoustic_steps_fused(ac->k.order) || !fused_buffers(ac, receive, nsteps)) {
     for (int i = 0; i < nsteps; i++) RC_OK(enqueue_forward(ac, ac->d_u, ac->d_u, s0 + i, rec));
     return EXA_OK;
   }
@@ -382,6 +432,10 @@ int enqueue_forward_steps(exa_acoustic* ac, int s0, int nsteps, double* rec) {
 }
 
 void free_acoustic(exa_acoustic* ac) {
+  {
+    std::lock_guard<std::mutex> lock(idle_mutex);
+    unlink_idle(ac);
+  }
   double* bufs[] = {ac->d_ck,    ac->d_seg,   ac->d_segq,  ac->d_qb2,   ac->d_rec_p, ac->d_u,     ac->d_mat,   ac->d_qb,     ac->d_ubar,  ac->d_fbar, ac->d_fbar2,
                     ac->d_gc,    ac->d_src_g, ac->d_src_tab, ac->d_rw,   ac->d_rec,  ac->d_res};
   for (double* b : bufs)
@@ -411,6 +465,29 @@ int set_step(exa_acoustic* ac, int step) {
 
 }  // namespace
 
+namespace exa {
+hipError_t device_malloc(void** p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e == hipSuccess) return e;
+  int device = 0;
+  if (hipGetDevice(&device) != hipSuccess) return e;
+  bool freed = false;
+  {
+    std::lock_guard<std::mutex> lock(idle_mutex);
+    for (exa_acoustic *m = idle_meshes, *next; m; m = next) {
+      next = m->next_idle;
+      if (m->device != device) continue;
+      free_optional(m);
+      unlink_idle(m);
+      freed = true;
+    }
+  }
+  if (!freed) return e;
+  (void)hipGetLastError();  // the one above
+  return hipMalloc(p, bytes);
+}
+}  // namespace exa
+
 extern "C" {
 
 int exa_acoustic_create(exa_acoustic** out, exa_ctx* ctx, int n, double h) {
@@ -436,12 +513,15 @@ int exa_acoustic_create(exa_acoustic** out, exa_ctx* ctx, int n, double h) {
   ac->nc = long(n) * n * n;
   ac->mat.assign(size_t(2) * ac->nc, 1.0);
   const size_t su = size_t(ac->nc) * ac->N * 4, sq = size_t(ac->nc) * 6 * ac->F * 4;
-  hipError_t e = hipStreamCreateWithFlags(&ac->stream, hipStreamNonBlocking);
-  if (e == hipSuccess) e = hipMalloc(&ac->d_u, sizeof(double) * su);
-  if (e == hipSuccess) e = hipMalloc(&ac->d_mat, sizeof(double) * 2 * ac->nc);
-  if (e == hipSuccess) e = hipMalloc(&ac->d_qb, sizeof(double) * sq);
-  if (e == hipSuccess) e = hipMalloc(&ac->d_step, sizeof(int));
-  if (e == hipSuccess) e = hipMalloc(&ac->d_src_g, sizeof(double) * ac->N);
+  size_t free = 0;
+  hipError_t e = hipGetDevice(&ac->device);
+  if (e == hipSuccess) e = hipMemGetInfo(&free, &ac->device_bytes);
+  if (e == hipSuccess) e = hipStreamCreateWithFlags(&ac->stream, hipStreamNonBlocking);
+  if (e == hipSuccess) e = exa::device_malloc(&ac->d_u, sizeof(double) * su);
+  if (e == hipSuccess) e = exa::device_malloc(&ac->d_mat, sizeof(double) * 2 * ac->nc);
+  if (e == hipSuccess) e = exa::device_malloc(&ac->d_qb, sizeof(double) * sq);
+  if (e == hipSuccess) e = exa::device_malloc(&ac->d_step, sizeof(int));
+  if (e == hipSuccess) e = exa::device_malloc(&ac->d_src_g, sizeof(double) * ac->N);
   if (e == hipSuccess) e = hipMemsetAsync(ac->d_u, 0, sizeof(double) * su, ac->stream);
   if (e != hipSuccess) {
     free_acoustic(ac);
@@ -596,6 +676,7 @@ int exa_acoustic_set_source(exa_acoustic* ac, const double* x, double amp, doubl
 
 int exa_acoustic_set_receivers(exa_acoustic* ac, int nrec, const double* xr) {
   if (!ac || nrec < 0 || (nrec > 0 && !xr)) return argerr("exa_acoustic_set_receivers: invalid argument");
+  const Call call(ac);
   for (int* p : {ac->d_rcell, ac->d_rstart, ac->d_rorder})
     if (p) (void)hipFree(p);
   if (ac->d_rw) (void)hipFree(ac->d_rw);
@@ -639,6 +720,7 @@ int exa_acoustic_set_receivers(exa_acoustic* ac, int nrec, const double* xr) {
 int exa_acoustic_run(exa_acoustic* ac, int nsteps, int use_graph, double* rec) {
   if (!ac || nsteps < 0) return argerr("exa_acoustic_run: invalid argument");
   if (nsteps == 0) return EXA_OK;
+  const Call call(ac);
   const int s0 = ac->step;
   RC_OK(ensure_source_table(ac, s0 + nsteps));
   RC_OK(grow(ac, &ac->d_rec, &ac->rec_cap, long(nsteps) * (ac->nrec > 0 ? ac->nrec : 1)));
@@ -720,6 +802,7 @@ int exa_acoustic_misfit_gradient(exa_acoustic* ac, int nsteps, int every, const 
                    "EXA_DIALECT_SPLIT_CK)");
     return EXA_ERR_UNSUPPORTED;
   }
+  const Call call(ac);
   const int s0 = ac->step, K = nsteps, R = ac->nrec, o = ac->k.order;
   const int nck = (K + every - 1) / every;
   const int seg = (every < K ? every : K) - 1;  // states of a segment besides its checkpoint
@@ -825,7 +908,6 @@ int exa_acoustic_misfit_gradient(exa_acoustic* ac, int nsteps, int every, const 
   (void)hipStreamSynchronize(ac->stream);
   for (auto& e : ev)
     if (e) (void)hipEventDestroy(e);
-  release_gradient_buffers(ac);
   if (rc) return rc;
   *J = Jv;
   return set_step(ac, s0 + K);

@@ -65,7 +65,7 @@ int status(int rc, const char* what) {
 template <typename T>
 int upload(T** dst, const std::vector<T>& v, const char* what) {
   if (v.empty()) return EXA_OK;
-  HIP_OK(hipMalloc(dst, sizeof(T) * v.size()), what);
+  HIP_OK(exa::device_malloc(dst, sizeof(T) * v.size()), what);
   HIP_OK(hipMemcpy(*dst, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice), what);
   return EXA_OK;
 }
@@ -172,18 +172,18 @@ struct CellSet {
     V = k.nvar;
     ND = k.nvar + k.npar;
     HIP_OK(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking), "stream");
-    HIP_OK(hipMalloc(&d_luh, sizeof(double) * ncells * NS * ND), "hipMalloc(luh)");
-    HIP_OK(hipMalloc(&d_lduh, sizeof(double) * ncells * NS * V), "hipMalloc(lduh)");
-    HIP_OK(hipMalloc(&d_qb, sizeof(double) * nslots * 2 * D * NF * ND), "hipMalloc(lQhbnd)");
-    HIP_OK(hipMalloc(&d_fb, sizeof(double) * nslots * 2 * D * NF * V), "hipMalloc(lFhbnd)");
-    HIP_OK(hipMalloc(&d_state, sizeof(double) * 3 * ninst), "hipMalloc(state)");
-    HIP_OK(hipMalloc(&d_picard, sizeof(int) * ncells), "hipMalloc(picard)");
+    HIP_OK(exa::device_malloc(&d_luh, sizeof(double) * ncells * NS * ND), "hipMalloc(luh)");
+    HIP_OK(exa::device_malloc(&d_lduh, sizeof(double) * ncells * NS * V), "hipMalloc(lduh)");
+    HIP_OK(exa::device_malloc(&d_qb, sizeof(double) * nslots * 2 * D * NF * ND), "hipMalloc(lQhbnd)");
+    HIP_OK(exa::device_malloc(&d_fb, sizeof(double) * nslots * 2 * D * NF * V), "hipMalloc(lFhbnd)");
+    HIP_OK(exa::device_malloc(&d_state, sizeof(double) * 3 * ninst), "hipMalloc(state)");
+    HIP_OK(exa::device_malloc(&d_picard, sizeof(int) * ncells), "hipMalloc(picard)");
     HIP_OK(hipMemset(d_picard, 0, sizeof(int) * ncells), "clear");
     std::vector<double> st(3 * ninst, 0.0);
     for (int i = ninst; i < 3 * ninst; i++) st[i] = DBL_MAX;
     HIP_OK(hipMemcpy(d_state, st.data(), sizeof(double) * st.size(), hipMemcpyHostToDevice), "state");
     dt_nslots = exa::kDtSlots / ninst > 8 ? exa::kDtSlots / ninst : 8;
-    HIP_OK(hipMalloc(&d_slots, sizeof(double) * ninst * dt_nslots * exa::kDtSlotStride), "hipMalloc(slots)");
+    HIP_OK(exa::device_malloc(&d_slots, sizeof(double) * ninst * dt_nslots * exa::kDtSlotStride), "hipMalloc(slots)");
     RC_OK(reset_slots());
     HIP_OK(hipMemset(d_qb, 0, sizeof(double) * nslots * 2 * D * NF * ND), "clear");
     HIP_OK(hipMemset(d_fb, 0, sizeof(double) * nslots * 2 * D * NF * V), "clear");
@@ -272,8 +272,8 @@ struct CellSet {
     // the corrector updates luh and dt_next: keep copies to restore
     double* save_luh = nullptr;
     double* save_state = nullptr;
-    HIP_OK(hipMalloc(&save_luh, sizeof(double) * ncells * NS * ND), "hipMalloc(autotune)");
-    hipError_t e = hipMalloc(&save_state, sizeof(double) * 3 * ninst);
+    HIP_OK(exa::device_malloc(&save_luh, sizeof(double) * ncells * NS * ND), "hipMalloc(autotune)");
+    hipError_t e = exa::device_malloc(&save_state, sizeof(double) * 3 * ninst);
     if (e == hipSuccess)
       e = hipMemcpyAsync(save_luh, d_luh, sizeof(double) * ncells * NS * ND, hipMemcpyDeviceToDevice, stream);
     if (e == hipSuccess)

@@ -81,7 +81,7 @@ int ensure_scratch(exa_ctx* c, size_t bytes) {
   if (c->h_scratch) (void)hipHostFree(c->h_scratch);
   c->d_scratch = c->h_scratch = nullptr;
   c->scratch_bytes = 0;
-  HIP_OK(hipMalloc(&c->d_scratch, bytes), "hipMalloc(scratch)");
+  HIP_OK(exa::device_malloc(&c->d_scratch, bytes), "hipMalloc(scratch)");
   HIP_OK(hipHostMalloc(reinterpret_cast<void**>(&c->h_scratch), bytes, hipHostMallocDefault), "hipHostMalloc(scratch)");
   c->scratch_bytes = bytes;
   return EXA_OK;
@@ -154,7 +154,7 @@ int ensure_guard(exa_ctx* c, long ncells) {
   if (c->d_guard) (void)hipFree(c->d_guard);
   c->d_guard = nullptr;
   c->guard_cap = 0;
-  HIP_OK(hipMalloc(&c->d_guard, sizeof(int) * (2 + ncells)), "hipMalloc(guard)");
+  HIP_OK(exa::device_malloc(&c->d_guard, sizeof(int) * (2 + ncells)), "hipMalloc(guard)");
   HIP_OK(hipMemset(c->d_guard, 0, 2 * sizeof(int)), "clear guard");
   c->guard_cap = ncells;
   return EXA_OK;
@@ -394,7 +394,7 @@ int exa_ctx_create(exa_ctx** out, int dim, int order, int nvar, int npar, int pd
   fill_even_odd(c->tab.dudx, B, h.dudx_eo);
   fill_even_odd(c->tab.Kxi, B, h.Kxi_eo);
   for (int i = 0; i < exa::kEvenOdd; i++) h.dudx_eof[i] = static_cast<float>(h.dudx_eo[i]);
-  hipError_t e = hipMalloc(&c->d_tab, sizeof(exa::DevTables));
+  hipError_t e = exa::device_malloc(&c->d_tab, sizeof(exa::DevTables));
   if (e == hipSuccess) e = hipMemcpy(c->d_tab, &h, sizeof(h), hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
   if (e != hipSuccess) {

@@ -301,6 +301,14 @@ int launch_acoustic(int which, int order, const AcousticArgs& a, hipStream_t s);
 int launch_acoustic_receivers_adj(int order, const AcousticArgs& a, const double* res, hipStream_t s);
 int launch_acoustic_advance(int* step, hipStream_t s);
 
+// hipMalloc of the library's objects: out of memory it tries again without the
+// buffers that idle acoustic meshes keep for their next call (acoustic_host.cpp).
+hipError_t device_malloc(void** p, size_t bytes);
+template <typename T>
+hipError_t device_malloc(T** p, size_t bytes) {
+  return device_malloc(reinterpret_cast<void**>(p), bytes);
+}
+
 void set_error(const std::string& msg);
 
 }  // namespace exa

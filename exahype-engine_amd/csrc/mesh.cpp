@@ -350,17 +350,17 @@ int exa_mesh_create_uniform(exa_mesh** out, exa_ctx* ctx, int n, double h) {
   m->ND = m->k.nvar + m->k.npar;
   const int V = m->k.nvar;
   hipError_t e = hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking);
-  if (e == hipSuccess) e = hipMalloc(&m->d_luh, sizeof(double) * m->ncells * m->NS * m->ND);
-  if (e == hipSuccess) e = hipMalloc(&m->d_lduh, sizeof(double) * m->ncells * m->NS * V);
-  if (e == hipSuccess) e = hipMalloc(&m->d_qb, sizeof(double) * m->ncells * 2 * D * m->NF * m->ND);
-  if (e == hipSuccess) e = hipMalloc(&m->d_fb, sizeof(double) * m->ncells * 2 * D * m->NF * V);
-  if (e == hipSuccess) e = hipMalloc(&m->d_h, sizeof(double) * m->ncells);
-  if (e == hipSuccess) e = hipMalloc(&m->d_state, sizeof(double) * 4);
+  if (e == hipSuccess) e = exa::device_malloc(&m->d_luh, sizeof(double) * m->ncells * m->NS * m->ND);
+  if (e == hipSuccess) e = exa::device_malloc(&m->d_lduh, sizeof(double) * m->ncells * m->NS * V);
+  if (e == hipSuccess) e = exa::device_malloc(&m->d_qb, sizeof(double) * m->ncells * 2 * D * m->NF * m->ND);
+  if (e == hipSuccess) e = exa::device_malloc(&m->d_fb, sizeof(double) * m->ncells * 2 * D * m->NF * V);
+  if (e == hipSuccess) e = exa::device_malloc(&m->d_h, sizeof(double) * m->ncells);
+  if (e == hipSuccess) e = exa::device_malloc(&m->d_state, sizeof(double) * 4);
   // room for the face list of any boundary choice: (n + 1) n^(D-1) entries per direction
-  if (e == hipSuccess) e = hipMalloc(&m->d_faces, sizeof(int) * 4 * D * (n + 1) * (m->ncells / n));
-  if (e == hipSuccess) e = hipMalloc(&m->d_picard, sizeof(int) * m->ncells);
-  if (e == hipSuccess) e = hipMalloc(&m->d_slots, sizeof(double) * exa::kDtSlots * exa::kDtSlotStride);
-  if (e == hipSuccess) e = hipMalloc(&m->d_guard, sizeof(int) * (2 + m->ncells));
+  if (e == hipSuccess) e = exa::device_malloc(&m->d_faces, sizeof(int) * 4 * D * (n + 1) * (m->ncells / n));
+  if (e == hipSuccess) e = exa::device_malloc(&m->d_picard, sizeof(int) * m->ncells);
+  if (e == hipSuccess) e = exa::device_malloc(&m->d_slots, sizeof(double) * exa::kDtSlots * exa::kDtSlotStride);
+  if (e == hipSuccess) e = exa::device_malloc(&m->d_guard, sizeof(int) * (2 + m->ncells));
   if (e != hipSuccess) {
     free_mesh(m);
     return fail(e, "exa_mesh_create_uniform");
@@ -448,7 +448,7 @@ int exa_mesh_adjust_solution(exa_mesh* m, int ic, const double* params, int npar
     return EXA_ERR_ARG;
   }
   double* d_prm = nullptr;
-  HIP_OK(hipMalloc(&d_prm, sizeof(double) * nparams), "hipMalloc(params)");
+  HIP_OK(exa::device_malloc(&d_prm, sizeof(double) * nparams), "hipMalloc(params)");
   hipError_t e = hipMemcpyAsync(d_prm, params, sizeof(double) * nparams, hipMemcpyHostToDevice, m->stream);
   int rc = EXA_OK;
   if (e == hipSuccess) {
@@ -627,8 +627,8 @@ int exa_mesh_set_boundary(exa_mesh* m, const int* kinds) {
   HIP_OK(hipStreamSynchronize(m->stream), "sync");
   if (mask && !m->d_gq) {
     const size_t nghost = size_t(2 * D) * (m->ncells / m->n) * m->NF;
-    HIP_OK(hipMalloc(&m->d_gq, sizeof(double) * nghost * m->ND), "hipMalloc(ghost faces)");
-    HIP_OK(hipMalloc(&m->d_gf, sizeof(double) * nghost * m->k.nvar), "hipMalloc(ghost fluxes)");
+    HIP_OK(exa::device_malloc(&m->d_gq, sizeof(double) * nghost * m->ND), "hipMalloc(ghost faces)");
+    HIP_OK(exa::device_malloc(&m->d_gf, sizeof(double) * nghost * m->k.nvar), "hipMalloc(ghost fluxes)");
   }
   m->bc = bc;
   m->bcmask = mask;
@@ -647,8 +647,8 @@ int exa_mesh_global_observables(exa_mesh* m, double* out, int nout) {
   }
   const int nobs = 2 + 3 * m->ND;
   double *d_part = nullptr, *d_out = nullptr;
-  hipError_t e = hipMalloc(&d_part, sizeof(double) * exa::observables_blocks(m->ncells) * 3 * m->ND);
-  if (e == hipSuccess) e = hipMalloc(&d_out, sizeof(double) * nobs);
+  hipError_t e = exa::device_malloc(&d_part, sizeof(double) * exa::observables_blocks(m->ncells) * 3 * m->ND);
+  if (e == hipSuccess) e = exa::device_malloc(&d_out, sizeof(double) * nobs);
   int rc = EXA_OK;
   if (e == hipSuccess) {
     rc = status(exa::launch_observables(m->k, m->stream, m->ncells, m->h, m->d_luh, d_part, d_out),
@@ -678,8 +678,8 @@ int exa_mesh_probe(exa_mesh* m, int npoints, const double* points, double* value
     }
   double *d_pts = nullptr, *d_out = nullptr;
   const size_t npb = sizeof(double) * npoints * D, nob = sizeof(double) * npoints * m->ND;
-  hipError_t e = hipMalloc(&d_pts, npb);
-  if (e == hipSuccess) e = hipMalloc(&d_out, nob);
+  hipError_t e = exa::device_malloc(&d_pts, npb);
+  if (e == hipSuccess) e = exa::device_malloc(&d_out, nob);
   if (e == hipSuccess) e = hipMemcpyAsync(d_pts, points, npb, hipMemcpyHostToDevice, m->stream);
   int rc = EXA_OK;
   if (e == hipSuccess) {
@@ -754,7 +754,7 @@ int exa_mesh_halo_pack_host(exa_mesh* m, int face, double* msg_q, double* msg_f)
   if (!m || !msg_q || !msg_f) return EXA_ERR_ARG;
   long nq = 0, nf = 0;
   exa_mesh_halo_size(m, &nq, &nf);
-  if (!m->d_halo) HIP_OK(hipMalloc(&m->d_halo, sizeof(double) * (nq + nf)), "hipMalloc(halo staging)");
+  if (!m->d_halo) HIP_OK(exa::device_malloc(&m->d_halo, sizeof(double) * (nq + nf)), "hipMalloc(halo staging)");
   const int rc = exa_mesh_halo_pack(m, face, m->d_halo, m->d_halo + nq);
   if (rc) return rc;
   HIP_OK(hipMemcpyAsync(msg_q, m->d_halo, sizeof(double) * nq, hipMemcpyDeviceToHost, m->stream), "halo copy");
@@ -767,7 +767,7 @@ int exa_mesh_halo_unpack_host(exa_mesh* m, int face, const double* msg_q, const 
   if (!m || !msg_q || !msg_f) return EXA_ERR_ARG;
   long nq = 0, nf = 0;
   exa_mesh_halo_size(m, &nq, &nf);
-  if (!m->d_halo) HIP_OK(hipMalloc(&m->d_halo, sizeof(double) * (nq + nf)), "hipMalloc(halo staging)");
+  if (!m->d_halo) HIP_OK(exa::device_malloc(&m->d_halo, sizeof(double) * (nq + nf)), "hipMalloc(halo staging)");
   // the previous use of the staging buffer has completed: every halo call synchronises
   HIP_OK(hipMemcpyAsync(m->d_halo, msg_q, sizeof(double) * nq, hipMemcpyHostToDevice, m->stream), "halo copy");
   HIP_OK(hipMemcpyAsync(m->d_halo + nq, msg_f, sizeof(double) * nf, hipMemcpyHostToDevice, m->stream), "halo copy");

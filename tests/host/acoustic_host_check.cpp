@@ -10,16 +10,21 @@
 // usage: acoustic_host_check <scenario>; prints what is wrong and exits 1.
 #include <cstdio>
 #include <cstdlib>
+#include <atomic>
 #include <cstring>
 #include <map>
+#include <mutex>
+#include <thread>
 
 #include "../../exahype-engine_amd/csrc/acoustic_host.cpp"
 
 namespace {
+std::recursive_mutex device;  // of the memory's books
 std::map<char*, size_t> live;
 size_t used = 0, limit = size_t(1) << 40;
-int fail_at = 0, mallocs = 0, steps_fused = 0, face_launches = 0;
-hipError_t last_error = hipSuccess;
+int fail_at = 0, mallocs = 0;
+std::atomic<int> steps_fused{0}, face_launches{0};
+thread_local hipError_t last_error = hipSuccess;
 
 #define CHECK(cond)                                             \
   do {                                                          \
@@ -31,6 +36,7 @@ hipError_t last_error = hipSuccess;
 
 // the bytes from p to the end of its allocation
 size_t room(const void* p) {
+  std::lock_guard<std::recursive_mutex> lock(device);
   auto it = live.upper_bound(static_cast<char*>(const_cast<void*>(p)));
   if (!p || it == live.begin()) return 0;
   --it;
@@ -42,6 +48,7 @@ bool holds(const void* p, size_t doubles) { return room(p) >= doubles * sizeof(d
 
 extern "C" {
 hipError_t hipMalloc(void** p, size_t n) {
+  std::lock_guard<std::recursive_mutex> lock(device);
   if (++mallocs == fail_at || used + n > limit) return last_error = hipErrorOutOfMemory;
   *p = std::calloc(1, n);
   live[static_cast<char*>(*p)] = n;
@@ -49,6 +56,7 @@ hipError_t hipMalloc(void** p, size_t n) {
   return hipSuccess;
 }
 hipError_t hipFree(void* p) {
+  std::lock_guard<std::recursive_mutex> lock(device);
   auto it = live.find(static_cast<char*>(p));
   CHECK(!p || it != live.end());
   if (!p) return hipSuccess;
@@ -72,6 +80,7 @@ hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t) {
   return hipSuccess;
 }
 hipError_t hipMemGetInfo(size_t* free, size_t* total) {
+  std::lock_guard<std::recursive_mutex> lock(device);
   *free = used > limit ? 0 : limit - used;
   *total = limit;
   return hipSuccess;
@@ -285,6 +294,7 @@ void gradient_without_room() {
     if (faces) limit += 12 * sq(ac);
     CHECK(!gradient(ac, 12, 12) && !gradient(ac, 12, 2) && !gradient(ac, 12, 12));
     limit -= su(ac) + (faces ? 12 * sq(ac) : 0);
+    free_optional(ac);
     CHECK(gradient(ac, 12, 12) == EXA_ERR_HIP && !gradient(ac, 12, 3) && !run(ac, 12));
     limit = size_t(1) << 40;
     CHECK(!gradient(ac, 12, 12));
@@ -302,6 +312,80 @@ void gradient_without_room() {
     CHECK(used == 0);
   }
 }
+
+// what a mesh cannot do without after its first gradient
+size_t required(const exa_acoustic* ac) {
+  size_t n = 0;
+  for (const void* p : {(void*)ac->d_u, (void*)ac->d_mat, (void*)ac->d_qb, (void*)ac->d_step, (void*)ac->d_src_g,
+                        (void*)ac->d_ubar, (void*)ac->d_fbar, (void*)ac->d_fbar2, (void*)ac->d_gc, (void*)ac->d_rcell,
+                        (void*)ac->d_rstart, (void*)ac->d_rorder, (void*)ac->d_rw, (void*)ac->d_rec, (void*)ac->d_res})
+    n += room(p);
+  return n;
+}
+
+// what meshes keep is bounded for all of them together, and goes when memory is short
+void many_meshes() {
+  exa_acoustic* first = mesh(4);
+  CHECK(!receivers(first, 2) && !gradient(first, 8, 4));
+  const size_t need = required(first), kept = used - need;
+  exa_acoustic_destroy(first);
+  CHECK(used == 0);
+  limit = 10 * need + 40 * kept;  // an eighth: some five meshes' buffers
+  std::vector<exa_acoustic*> all;
+  for (int i = 0; i < 10; i++) {
+    all.push_back(mesh(4));
+    CHECK(all.back() && !receivers(all.back(), 2) && !gradient(all.back(), 8, 4));
+    size_t n = 0;
+    for (const exa_acoustic* ac : all) n += required(ac);
+    CHECK(used - n <= limit / 8 && used - n >= kept);
+  }
+  limit = used + su(all[0]);  // only what idle meshes keep is left for a mesh more
+  exa_acoustic* more = mesh(4);
+  CHECK(more && !run(more, 3) && more->d_u);
+  exa_acoustic_destroy(more);
+  void* other = nullptr;  // and for the library's other objects
+  CHECK(!gradient(all[3], 2, 2));
+  limit = used;
+  CHECK(exa::device_malloc(&other, kept / 8) == hipSuccess && hipGetLastError() == hipSuccess);
+  (void)hipFree(other);
+  CHECK(exa::device_malloc(&other, limit) == hipErrorOutOfMemory && hipGetLastError() != hipSuccess);
+  limit = size_t(1) << 40;
+  for (exa_acoustic* ac : all) {
+    CHECK(!gradient(ac, 8, 4) && !run(ac, 5));
+    exa_acoustic_destroy(ac);
+  }
+  CHECK(used == 0 && !idle_meshes);
+}
+
+// a face buffer that cannot be kept is allocated for long runs only
+void large_mesh() {
+  limit = 120000;
+  exa_acoustic* ac = mesh(4);
+  CHECK(ac && sq(ac) > limit / 8);
+  steps_fused = 0;
+  CHECK(!run(ac, 15) && steps_fused == 0 && !ac->d_qb2);
+  CHECK(!run(ac, 16) && steps_fused == 15 && !ac->d_qb2);
+  exa_acoustic_destroy(ac);
+}
+
+// meshes of several threads, in turn taking memory from each other's
+void threads() {
+  exa_acoustic* one = mesh(4);
+  CHECK(!receivers(one, 2) && !gradient(one, 8, 4));
+  limit = 4 * used;
+  exa_acoustic_destroy(one);
+  exa::cfg.order = 4;
+  std::vector<std::thread> pool;
+  for (int t = 0; t < 3; t++)
+    pool.emplace_back([t] {
+      exa_acoustic* ac = nullptr;
+      CHECK(!exa_acoustic_create(&ac, reinterpret_cast<exa_ctx*>(&exa::cfg), 2, 0.5));
+      for (int i = 0; i < 300; i++) CHECK(!receivers(ac, 1 + (i + t) % 2) && !run(ac, 1 + i % 5) && !gradient(ac, 8, 1 + (i + t) % 4));
+      exa_acoustic_destroy(ac);
+    });
+  for (std::thread& t : pool) t.join();
+  CHECK(used == 0 && !idle_meshes);
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -311,6 +395,9 @@ int main(int argc, char** argv) {
       {"failed_allocation", failed_allocation},
       {"no_second_faces", no_second_faces},
       {"gradient_without_room", gradient_without_room},
+      {"many_meshes", many_meshes},
+      {"large_mesh", large_mesh},
+      {"threads", threads},
   };
   const auto it = scenarios.find(argc > 1 ? argv[1] : "");
   if (it == scenarios.end()) return 2;

@@ -8,7 +8,8 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
-SCENARIOS = ["dataflow", "stale_error", "failed_allocation", "no_second_faces", "gradient_without_room"]
+SCENARIOS = ["dataflow", "stale_error", "failed_allocation", "no_second_faces", "gradient_without_room", "many_meshes",
+             "large_mesh", "threads"]
 
 
 @pytest.fixture(scope="module")
