@@ -9,6 +9,7 @@ the other gradient tests; J and the forward state 1e-12.
 """
 import numpy as np
 import pytest
+import torch
 
 import exahype_amd as E
 import oracle as O
@@ -103,3 +104,70 @@ def test_line_predictor_in_large_workgroups(order, n):
     ac.close()
     for line, node, tol in zip(*got, (1e-12, 1e-10, 1e-12)):
         assert rel_l2(line, node) <= tol
+
+
+def shot(order=4, n=5, receivers=3, seed=0):
+    rng = np.random.default_rng(seed)
+    c, rho = 1.0 + 0.2 * rng.uniform(-1, 1, n ** 3), 1.0 + 0.1 * rng.uniform(-1, 1, n ** 3)
+    luh = P.acoustic_state(n, order, c, rho, 0.1 * rng.normal(size=(n ** 3, (order + 1) ** 3, 4)))
+    ac = E.Acoustic(E.Context(3, order, 4, 2, E.PDE_ACOUSTIC), n, 1.0 / n)
+    ac.set_solution(luh)
+    ac.set_dt(0.0)
+    ac.set_source((0.4, 0.6, 0.3), 1.0, 5.0, 0.05)
+    place(ac, receivers)
+    return ac, luh
+
+
+def place(ac, receivers):
+    ac.set_receivers(np.random.default_rng(receivers).uniform(0.05, 0.95, size=(receivers, 3)))
+
+
+def one_gradient(ac, luh, steps, receivers, every):
+    ac.set_solution(luh)
+    ac.set_step(0)
+    obs = np.random.default_rng(steps + receivers).normal(0.0, 0.1, (steps, receivers))
+    J, g = ac.misfit_gradient(steps, obs, checkpoint_every=every)
+    return J, g, ac.get_solution()
+
+
+def test_gradients_on_buffers_of_earlier_calls():
+    """One object through other intervals, step counts and receivers, runs in between, against fresh
+    objects: bit for bit."""
+    ac, luh = shot()
+    for steps, receivers, every in ((9, 3, 1), (9, 3, 50), (7, 5, 3), (12, 2, 4), (3, 5, 2), (12, 2, 12)):
+        print(f"[kept buffers] steps={steps} receivers={receivers} every={every}", flush=True)
+        place(ac, receivers)
+        got = one_gradient(ac, luh, steps, receivers, every)
+        ac.run(3)
+        fresh, _ = shot(receivers=receivers)
+        want = one_gradient(fresh, luh, steps, receivers, every)
+        fresh.close()
+        assert got[0] == want[0]
+        np.testing.assert_array_equal(got[1], want[1])
+        np.testing.assert_array_equal(got[2], want[2])
+    ac.close()
+
+
+def test_gradient_without_memory_for_the_faces():
+    """A segment's faces larger than a quarter of what is free (most of the memory is held by a tensor):
+    they are formed step by step, and the gradient is the one with the faces kept, bit for bit."""
+    n, order, every, steps = 13, 4, 130, 131
+    faces = n ** 3 * 6 * (order + 1) ** 2 * 4 * 8 * every
+    ac, luh = shot(order, n)
+    want = one_gradient(ac, luh, steps, 3, every)
+    ac.close()
+    torch.cuda.empty_cache()
+    hold = torch.cuda.mem_get_info()[0] - (4 << 30)
+    print(f"[no faces] holding {hold >> 20} MiB", flush=True)
+    held = torch.empty(hold, dtype=torch.uint8, device="cuda")
+    try:
+        ac, luh = shot(order, n)
+        assert faces > torch.cuda.mem_get_info()[0] // 4
+        got = one_gradient(ac, luh, steps, 3, every)
+        ac.close()
+    finally:
+        del held
+        torch.cuda.empty_cache()
+    assert got[0] == want[0]
+    np.testing.assert_array_equal(got[1], want[1])
+    np.testing.assert_array_equal(got[2], want[2])
