@@ -307,8 +307,9 @@ void drop_graph(exa_mesh* m) {
 
 // Steps of the larger graph of exa_mesh_run.  Between two graph launches the GPU
 // waits about 4 us (27^2 order 3: 22 us a step with one-step graphs, 18 with
-// eight); the first run captures one step only, so that a single short run does not
-// pay for the larger graph.
+// eight).  A mesh's first captured run takes one-step graphs only, however long it
+// is: what capturing and instantiating the larger one costs is left to programs that
+// run again.
 constexpr int kGraphSteps = 8;
 
 int capture_steps(exa_mesh* m, int steps, hipGraph_t* graph, hipGraphExec_t* exec) {
@@ -322,8 +323,13 @@ int capture_steps(exa_mesh* m, int steps, hipGraph_t* graph, hipGraphExec_t* exe
     return rc;
   }
   if (e != hipSuccess) return fail(e, "end capture");
+  const hipError_t ei = hipGraphInstantiate(exec, g, nullptr, nullptr, 0);
+  if (ei != hipSuccess) {
+    (void)hipGraphDestroy(g);
+    *exec = nullptr;
+    return fail(ei, "instantiate");
+  }
   *graph = g;
-  HIP_OK(hipGraphInstantiate(exec, g, nullptr, nullptr, 0), "instantiate");
   return EXA_OK;
 }
 
@@ -508,10 +514,8 @@ int exa_mesh_run(exa_mesh* m, int nsteps, int use_graph) {
       const int rc = capture_steps(m, 1, &m->graph, &m->graph_exec);
       if (rc) return rc;
     }
-    if (again && nsteps >= kGraphSteps && !m->graph_many_exec) {
-      const int rc = capture_steps(m, kGraphSteps, &m->graph_many, &m->graph_many_exec);
-      if (rc) return rc;
-    }
+    if (again && nsteps >= kGraphSteps && !m->graph_many_exec)  // where it cannot be had, steps one by one
+      (void)capture_steps(m, kGraphSteps, &m->graph_many, &m->graph_many_exec);
     int left = nsteps;
     for (; m->graph_many_exec && left >= kGraphSteps; left -= kGraphSteps)
       HIP_OK(hipGraphLaunch(m->graph_many_exec, m->stream), "graph launch");
