@@ -218,7 +218,9 @@ struct AcLineShape {
   static constexpr int LDS = 2 * BUF > 24 * F ? 2 * BUF : 24 * F;
   // small workgroups: more of them fit beside each other on a CU, so that one
   // computes while another waits at a barrier or for HBM (order 4 at 54^3: 256
-  // lanes 0.709, 128 lanes 0.639, 64 lanes, of which 50 have a line, 0.691 ms)
+  // lanes 0.709, 128 lanes 0.639, 64 lanes, of which 50 have a line, 0.691 ms; order 3
+  // at 9^3 128 lanes 12.9, 64 lanes 10.7 us, at 40^3 127 and 126; larger ones where
+  // large_line_groups says)
   static constexpr int THREADS = T;
   static constexpr int CPB_T = THREADS / F;
   static constexpr int CPB_L = (60 * 1024) / (LDS * 8);

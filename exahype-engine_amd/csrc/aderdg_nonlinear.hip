@@ -56,11 +56,6 @@ struct Shape {
   static constexpr int NSP = next_pow2(NS);
 };
 
-template <typename R>
-__device__ __forceinline__ R tabI(const DevTables* T, int i) { return T->iK1[i]; }
-template <typename R>
-__device__ __forceinline__ R tabD(const DevTables* T, int i) { return T->dudx[i]; }
-
 // Coordinates (z, y, x) of spatial node s; z = 0 in 2D.
 template <int D, int B>
 __device__ __forceinline__ void node_zyx(int s, int& z, int& y, int& x) {
@@ -475,7 +470,7 @@ __device__ __forceinline__ void predictor_tile(
 #pragma unroll
               for (int n = 0; n < B; n++)
                 g += static_cast<R>(invDx[d]) * qs[(base[d] + n * stride_of<D, B>(d)) * V + v] *
-                     tabD<R>(T, cc[d] * B + n);
+                     T->dudx[cc[d] * B + n];
               gq[d][v] = g;
             }
           R Sv[V];
@@ -494,9 +489,9 @@ __device__ __forceinline__ void predictor_tile(
 #pragma unroll
           for (int v = 0; v < V; v++) {
             if (t == 0)
-              acc[tp][v] = r[v] * tabI<R>(T, tp * B + t);
+              acc[tp][v] = r[v] * T->iK1[tp * B + t];
             else
-              acc[tp][v] += r[v] * tabI<R>(T, tp * B + t);
+              acc[tp][v] += r[v] * T->iK1[tp * B + t];
           }
       }
     }

@@ -32,9 +32,11 @@ struct exa_ctx {
   exa::Tables tab{};
   exa::DevTables* d_tab = nullptr;
   hipStream_t stream = nullptr;
-  // scratch for the per-cell compatibility entry points
-  // and its host image in pinned memory: a call lays out its inputs there, copies
-  // them in one piece, and reads its outputs back in one
+  // Scratch for the per-cell compatibility entry points, and its host image in
+  // pinned memory: the nonlinear predictor, Riemann solver, surface integral, update
+  // and stable dt lay out their inputs there, copy them in one piece and read their
+  // outputs back in one.  The other entry points (single faces, boundary
+  // conditions, the linear path, projections) copy array by array.
   double* d_scratch = nullptr;
   double* h_scratch = nullptr;
   size_t scratch_bytes = 0;
@@ -375,7 +377,6 @@ int exa_ctx_create(exa_ctx** out, int dim, int order, int nvar, int npar, int pd
     h.iK1[i] = c->tab.iK1[i];
     h.dudx[i] = c->tab.dudx[i];
     h.Kxif[i] = static_cast<float>(c->tab.Kxi[i]);
-    h.iK1f[i] = static_cast<float>(c->tab.iK1[i]);
     h.dudxf[i] = static_cast<float>(c->tab.dudx[i]);
     h.Pt[i] = c->tab.iK1[i] * c->tab.w[i % B];
     h.Ptf[i] = static_cast<float>(h.Pt[i]);

@@ -27,7 +27,6 @@ struct DevTables {
   float F0f[kMaxBasis];
   float F1f[kMaxBasis];
   float Kxif[kMaxBasis * kMaxBasis];
-  float iK1f[kMaxBasis * kMaxBasis];
   // derived operators of the line-decomposed predictor
   float dudxf[kMaxBasis * kMaxBasis];
   double Pt[kMaxBasis * kMaxBasis];  // Pt[i][j] = iK1[i][j] * w[j]

@@ -305,7 +305,8 @@ struct Tile {
                        SLICE = S::SLICE, TS = S::TS, VS = CPB * NL * B;
 
   // Two waves per SIMD leave the registers for the average in the loop (CERK at
-  // 40^3, order 5: 2.02 -> 1.86 ms); the other shapes run at three or four, order
+  // 40^3, order 5: 2.02 -> 1.86 ms); order 3, in FP64 at two waves too, needs them for
+  // the rows of its exchange.  The other shapes run at three or four (min_waves), order
   // 4 with a few spilled registers, and gain more from the third wave (batched 3D
   // order 4 at 23^3, whole step: 518 us at two waves, 539 at three with the
   // average in the loop, 481 this way; 2D at 243^2 0.220, 0.249 and 0.200 ms).

@@ -2,7 +2,7 @@
 
 The reference passes dx[D] to the predictor and the time-step size
 (ExaHyPE/exahype/solvers/ADERDGSolver.h:2542-2553; stableTimeStepSize.cpph:14-62
-sums max |lambda_d| / dx_d).  A cell with unequal edges runs the node-column
+sums max |lambda_d| / dx_d).  A cell with unequal edges runs the column
 predictor with 1/dx per direction (stiffness, CERK divergences, volume
 integral) and the stable dt with dx per direction.  FP64 bar 1e-12 relative L2
 with equal Picard counts; the FP32 form within 1e-4 of the oracle (lduh of a

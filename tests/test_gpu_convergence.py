@@ -15,7 +15,7 @@ every pair (the coarsest meshes are pre-asymptotic).
   iteration stops that far from its fixed point), so 27^3 would measure the
   stopping rule, not the discretisation.
 * The headline FP32 form (CERK guess, one collapsed Picard iteration with the
-  Picard guard; N = 5 on the x-line kernel, N = 3, 4 on the node-column
+  Picard guard; N = 5 on the x-line kernel, N = 3, 4 on the column
   kernel) until its FP32 error floor near 1.3e-7: N = 5 on 3^3, 4^3, 5^3
   cells, N = 4 on 4^3, 6^3, 9^3, N = 3 on 3^3, 6^3, 9^3.
 """

@@ -181,7 +181,7 @@ def test_dialect_error_paths():
 
 @pytest.mark.parametrize("D,order,n,steps", [(3, 5, 3, 3), (2, 4, 9, 4)])
 def test_mesh_with_cerk_guess_and_generic_rule_vs_oracle(D, order, n, steps):
-    """FP64 node-column kernel: CERK initial guess with the generic adaptive rule."""
+    """FP64 column kernel: CERK initial guess with the generic adaptive rule."""
     print(f"[cerk generic] D={D} order={order} n={n}", flush=True)
     luh0 = P.density_wave_3d(n, order) if D == 3 else P.density_wave_2d(n, order)
     ref = luh0.copy()
@@ -207,7 +207,7 @@ def test_mesh_with_cerk_guess_and_generic_rule_vs_oracle(D, order, n, steps):
 @pytest.mark.parametrize("picard", [1, 2, 3])
 def test_fp32_line_kernel_with_cerk_guess(picard):
     """The FP32 matrix-core line kernel with the CERK guess and a fixed count
-    agrees with the FP32 node-column kernel with the same guess and count, and
+    agrees with the FP32 column kernel with the same guess and count, and
     stays within 1e-6 of the FP64 generic adaptive oracle."""
     n, order, steps = 3, 5, 3
     luh = P.density_wave_3d(n, order)
@@ -237,7 +237,7 @@ def test_fp32_line_kernel_with_cerk_guess(picard):
 
 @pytest.mark.parametrize("D,order,n,steps,bc", [(3, 4, 3, 2, [1, 1, 0, 0, 2, 2]), (2, 3, 6, 4, [2, 2, 1, 1])])
 def test_mesh_with_boundaries_and_cerk_guess_vs_oracle(D, order, n, steps, bc):
-    """CERK guess (generic rule, FP64 node-column kernel) on a mesh with wall and
+    """CERK guess (generic rule, FP64 column kernel) on a mesh with wall and
     Dirichlet faces: the boundary path and the guess together."""
     print(f"[cerk boundary] D={D} order={order} n={n} bc={bc}", flush=True)
     o = O.Oracle(D, order, dialect="cerk")
@@ -275,7 +275,7 @@ def test_mesh_with_boundaries_and_cerk_guess_vs_oracle(D, order, n, steps, bc):
 def test_fp32_cerk_line_kernel_with_walls_agrees_with_node_kernel():
     """FP32, CERK guess, one fixed iteration (the one-iteration line kernel with
     FP64 faces, since walls rule out the FP32-face step) against the FP32
-    node-column kernel with the same guess and count."""
+    column kernel with the same guess and count."""
     n, order, steps = 3, 5, 2
     bc = [1, 1, 0, 0, 0, 0]
     o = O.Oracle(3, order)

@@ -6,11 +6,12 @@ linear advection (F_d = a_d Q, any number of variables) for 1 variable in 2D
 and 3D at order 3 and 3 variables in 3D at order 2, and a user PDE for its
 declared kNVar.  Checked at the FP64 bar 1e-12 relative L2 with identical
 Picard counts: the per-cell fused predictor + volume integral, the per-face
-Rusanov solve, uniform periodic meshes in both step forms; the FP32 node-column
-form within 1e-6; 3D order 5 with five advected variables (the node-column
-kernel's general flux slab, which Euler no longer uses), both initial guesses;
-and the host refuses Euler or the user PDE with another variable count.  The oracle's advection path is pinned to the exact space-time
-solution (tests/test_oracle_dialect.py, CERK exactness for quadratic data).
+Rusanov solve, uniform periodic meshes in both step forms; the FP32 column
+form within 1e-6; 3D order 5 with five advected variables (the column kernel's
+general flux, which Euler does not use), both initial guesses; and the host refuses
+Euler or the user PDE with another variable count.  The oracle's advection path is
+pinned to the exact space-time solution (tests/test_oracle_dialect.py, CERK exactness
+for quadratic data).
 """
 import numpy as np
 import pytest
@@ -114,8 +115,8 @@ def test_fp32_node_column_form():
 @pytest.mark.parametrize("guess", ["trivial", "cerk"])
 def test_order5_advection_five_variables_vs_oracle(guess):
     """3D order 5 with five variables and a PDE other than Euler: the FP64
-    node-column kernel with its general flux slab (Euler runs the 12-slot
-    form), both initial guesses, per-cell and on a periodic mesh."""
+    column kernel with its general flux (Euler has an instantiation of its own),
+    both initial guesses, per-cell and on a periodic mesh."""
     D, order, V, n, steps = 3, 5, 5, 3, 2
     print(f"[order5 advection] guess={guess}", flush=True)
     dial = "cerk" if guess == "cerk" else None

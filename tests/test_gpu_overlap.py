@@ -123,7 +123,7 @@ def test_overlap_arguments():
         mesh.set_overlap(3)
     mesh.close()
     ctx.close()
-    ctx64 = E.Context(3, ORDER)  # FP64 node-column predictor: whole-mesh launches only
+    ctx64 = E.Context(3, ORDER)  # FP64 column predictor: whole-mesh launches only
     mesh = E.Mesh(ctx64, 4, 0.25)
     with pytest.raises(E.ExaError):
         mesh.set_overlap(3)

@@ -354,7 +354,7 @@ def test_device_initial_condition_matches_host(dim, n, order):
                                                    (E.PREC_FP32, 0, 2e-6)])
 def test_predictor_variants_agree(precision, variant, tol):
     """The line-decomposed 3D order-5 predictor (VALU and matrix-core forms)
-    and the FP32 space-time tile predictor agree with the generic node-column
+    and the FP32 space-time tile predictor agree with the generic column
     kernel."""
     n, order, steps = 4, 5, 2
     luh = P.density_wave_3d(n, order)
@@ -379,7 +379,7 @@ def test_predictor_variants_agree(precision, variant, tol):
 def test_fp32_fixed_picard_counts_agree(picard):
     """The FP32 matrix-core line predictor with a fixed Picard count (time
     averages formed by the time lanes: fluxes of iteration picard - 2's output,
-    or of the initial guess for one iteration) against the FP32 node-column
+    or of the initial guess for one iteration) against the FP32 column
     kernel with the same count."""
     n, order, steps = 3, 5, 2
     luh = P.density_wave_3d(n, order)
