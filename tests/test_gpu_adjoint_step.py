@@ -7,9 +7,10 @@ and the checkpoint intervals cover a segment of one step, a shorter last segment
 and one segment for the whole run.  Bar: 1e-10 relative L2 of the gradient, as of
 the other gradient tests; J and the forward state 1e-12.
 """
+import ctypes
+
 import numpy as np
 import pytest
-import torch
 
 import exahype_amd as E
 import oracle as O
@@ -149,25 +150,31 @@ def test_gradients_on_buffers_of_earlier_calls():
 
 
 def test_gradient_without_memory_for_the_faces():
-    """A segment's faces larger than a quarter of what is free (most of the memory is held by a tensor):
+    """A segment's faces larger than a quarter of what is free (most of the memory is held by the test):
     they are formed step by step, and the gradient is the one with the faces kept, bit for bit."""
     n, order, every, steps = 13, 4, 130, 131
     faces = n ** 3 * 6 * (order + 1) ** 2 * 4 * 8 * every
     ac, luh = shot(order, n)
     want = one_gradient(ac, luh, steps, 3, every)
     ac.close()
-    torch.cuda.empty_cache()
-    hold = torch.cuda.mem_get_info()[0] - (4 << 30)
+    hip = ctypes.CDLL(next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line))
+    held = ctypes.c_void_p()
+
+    def free():
+        f, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(f), ctypes.byref(total)) == 0
+        return f.value
+
+    hold = free() - (4 << 30)
     print(f"[no faces] holding {hold >> 20} MiB", flush=True)
-    held = torch.empty(hold, dtype=torch.uint8, device="cuda")
+    assert hip.hipMalloc(ctypes.byref(held), ctypes.c_size_t(hold)) == 0
     try:
         ac, luh = shot(order, n)
-        assert faces > torch.cuda.mem_get_info()[0] // 4
+        assert faces > free() // 4
         got = one_gradient(ac, luh, steps, 3, every)
         ac.close()
     finally:
-        del held
-        torch.cuda.empty_cache()
+        assert hip.hipFree(held) == 0
     assert got[0] == want[0]
     np.testing.assert_array_equal(got[1], want[1])
     np.testing.assert_array_equal(got[2], want[2])
