@@ -819,19 +819,24 @@ struct Tile {
 // and a line's working set; one wave more spills (FP64 order 5 at three: 52
 // registers, 24 -> 30 ms at 81^3; order 3 at three: 27, 0.375 -> 0.390 ms at 35^3).
 // Order 4 spills at three, 10 to 16 registers for Euler and 41 to 44 for the other
-// equations, and still gains, but for the latter's one-iteration CERK form in 3D
-// (advection, 1,000 cells: 24.0 at three, 18.9 us at two; 24,000 cells 390, 340 us;
-// with the trivial guess 607, 672 us, in 2D 228, 265 us).
-template <int D, int B, int V, int NP, typename R, bool CG, bool EU>
+// equations, and still gains from the third wave once the cells fill it.
+template <int D, int B, int V, int NP, typename R>
 constexpr int min_waves() {
   if (D == 3 && B <= 3) return 3;  // as many as LDS takes
   if (sizeof(R) == 4) return 4;
-  return B == 4 || B >= 6 || (D == 3 && B == 5 && CG && !EU) ? 2 : 3;
+  return B == 4 || B >= 6 ? 2 : 3;
 }
+// The CERK forms of the other equations in 3D at order 4 exist at two waves as well,
+// for one iteration and for meshes that two waves per SIMD hold at once (advection,
+// two iterations, node form before / three / two waves: 1,000 cells 31.8 / 31.8 / 26.9,
+// 1,500 50.1 / 39.9 / 46.9, 24,000 640 / 489 / 514 us; one iteration: 1,000 cells 20.7 /
+// 23.8 / 18.9, 24,000 389 / 389 / 338; the trivial guess: 24,000 945 / 607 / 672).
+template <int D, int B, typename R, bool CG, bool EU>
+constexpr bool kTwoWaves = D == 3 && B == 5 && sizeof(R) == 8 && CG && !EU;
 
 // One workgroup per tile of CPB cells, or a smaller grid that loops over the tiles.
-template <int D, int B, int V, int NP, typename R, bool CG, bool EU>
-__global__ __launch_bounds__((Shape<D, B, V, NP, R>::THREADS), (min_waves<D, B, V, NP, R, CG, EU>())) void
+template <int D, int B, int V, int NP, typename R, bool CG, bool EU, int WAVES = min_waves<D, B, V, NP, R>()>
+__global__ __launch_bounds__((Shape<D, B, V, NP, R>::THREADS), WAVES) void
 column_predictor_kernel(long ncells, long ntiles, const double* luh, const double* __restrict__ hcell,
                         const double* __restrict__ dtp, const int* __restrict__ cinst, double* __restrict__ lduh,
                         double* __restrict__ lQhbnd, double* __restrict__ lFhbnd, int* __restrict__ picard,
@@ -857,9 +862,15 @@ struct Launch {
     using S = Shape<D, B, V, NP, R>;
     const long tiles = (n + S::CPB - 1) / S::CPB;
     const long grid = (o.grid > 0 && o.grid < tiles) ? o.grid : tiles;
-    hipLaunchKernelGGL((column_predictor_kernel<D, B, V, NP, R, CG, EU>), dim3(unsigned(grid)), dim3(S::THREADS), 0, st,
-                       n, tiles, luh, h, dt, o.cinst, lduh, qb, fb, pic, k.tab, k.pde, maxIter, adaptive, o.luh_update,
-                       k.dialect, o.hdim);
+    auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(unsigned(grid)), dim3(S::THREADS), 0, st, n, tiles, luh, h, dt, o.cinst, lduh, qb, fb,
+                         pic, k.tab, k.pde, maxIter, adaptive, o.luh_update, k.dialect, o.hdim);
+    };
+    if constexpr (kTwoWaves<D, B, R, CG, EU>) {
+      if (maxIter == 1 || grid * (S::THREADS / 64) <= 2048)  // 1,024 SIMDs
+        return launch(column_predictor_kernel<D, B, V, NP, R, CG, EU, 2>);
+    }
+    launch(column_predictor_kernel<D, B, V, NP, R, CG, EU>);
   }
   template <typename R, bool CG>
   static void pde(const KernelCfg& k, hipStream_t st, long n, const double* luh, const double* h, const double* dt,
