@@ -826,13 +826,13 @@ constexpr int min_waves() {
   if (sizeof(R) == 4) return 4;
   return B == 4 || B >= 6 ? 2 : 3;
 }
-// The CERK forms of the other equations in 3D at order 4 exist at two waves as well,
-// for one iteration and for meshes that two waves per SIMD hold at once (advection,
-// two iterations, node form before / three / two waves: 1,000 cells 31.8 / 31.8 / 26.9,
-// 1,500 50.1 / 39.9 / 46.9, 24,000 640 / 489 / 514 us; one iteration: 1,000 cells 20.7 /
-// 23.8 / 18.9, 24,000 389 / 389 / 338; the trivial guess: 24,000 945 / 607 / 672).
-template <int D, int B, typename R, bool CG, bool EU>
-constexpr bool kTwoWaves = D == 3 && B == 5 && sizeof(R) == 8 && CG && !EU;
+// 3D order 4 in FP64 exists at two waves as well, for meshes that two waves per SIMD
+// hold at once (node form before / three / two waves: Euler, one CERK iteration, 500
+// cells 15.4 / 16.5 / 15.5 us; advection, three iterations, 1,000 cells 30.8 / 30.5 /
+// 24.8; 1,500 cells 50.0 / 38.5 / 42.8) and for one CERK iteration of the other
+// equations (24,000 cells 389 / 389 / 338; two iterations 602 / 488 / 495).
+template <int D, int B, typename R>
+constexpr bool kTwoWaves = D == 3 && B == 5 && sizeof(R) == 8;
 
 // One workgroup per tile of CPB cells, or a smaller grid that loops over the tiles.
 template <int D, int B, int V, int NP, typename R, bool CG, bool EU, int WAVES = min_waves<D, B, V, NP, R>()>
@@ -866,8 +866,8 @@ struct Launch {
       hipLaunchKernelGGL(kernel, dim3(unsigned(grid)), dim3(S::THREADS), 0, st, n, tiles, luh, h, dt, o.cinst, lduh, qb, fb,
                          pic, k.tab, k.pde, maxIter, adaptive, o.luh_update, k.dialect, o.hdim);
     };
-    if constexpr (kTwoWaves<D, B, R, CG, EU>) {
-      if (maxIter == 1 || grid * (S::THREADS / 64) <= 2048)  // 1,024 SIMDs
+    if constexpr (kTwoWaves<D, B, R>) {
+      if (grid * (S::THREADS / 64) <= 2048 || (CG && !EU && maxIter == 1))  // 1,024 SIMDs
         return launch(column_predictor_kernel<D, B, V, NP, R, CG, EU, 2>);
     }
     launch(column_predictor_kernel<D, B, V, NP, R, CG, EU>);

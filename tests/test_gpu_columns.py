@@ -112,20 +112,25 @@ def test_batches_around_a_workgroup(dim, order, form):
     ctx.close()
 
 
-@pytest.mark.parametrize("iterations", [1, 2])
-def test_two_and_three_waves_of_the_order4_cerk_form(iterations):
-    """Equations other than Euler's, 3D order 4, CERK guess: one batch beyond the cells that two waves per
-    SIMD hold against its halves within, cell by cell the same operations: bit for bit."""
-    print(f"[columns] waves iterations={iterations}", flush=True)
-    ctx = E.Context(3, 4, 5, 0, E.PDE_ADVECTION, picard_max=iterations)
-    ctx.set_advection(np.array([1.0, 0.5, 0.25]))
-    ctx.set_initial_guess(E.GUESS_CERK)
-    luh = np.random.default_rng(iterations).normal(1.0, 0.2, (1301, 125, 5))
+@pytest.mark.parametrize("pde,form", [("euler", "trivial"), ("euler", "cerk"), ("advection", "trivial"),
+                                      ("advection", "cerk")])
+def test_two_and_three_waves_of_order4(pde, form):
+    """3D order 4 in FP64: one batch beyond the cells that two waves per SIMD hold against its halves
+    within, cell by cell the same operations: bit for bit."""
+    print(f"[columns] waves pde={pde} form={form}", flush=True)
+    adv = [1.0, 0.5, 0.25]
+    ctx = E.Context(3, 4, 5, 0, E.PDE_EULER if pde == "euler" else E.PDE_ADVECTION, picard_max=2)
+    if pde != "euler":
+        ctx.set_advection(np.array(adv))
+    if form == "cerk":
+        ctx.set_initial_guess(E.GUESS_CERK)
+    luh = np.tile(states(3, 4, 50, 11), (27, 1, 1))[:1301]
     whole = batch(ctx, luh, 0.1, 1e-3, 3, 4)
     halves = [batch(ctx, part, 0.1, 1e-3, 3, 4) for part in (luh[:651], luh[651:])]
     for key in ("lduh", "qb", "fb"):
         np.testing.assert_array_equal(whole[key], np.concatenate([h[key] for h in halves]))
-    orc = O.Oracle(3, 4, nvar=5, pde=O.PDE_ADVECTION, adv=[1.0, 0.5, 0.25], dialect="cerk", max_picard=iterations)
+    orc = O.Oracle(3, 4, pde=O.PDE_EULER if pde == "euler" else O.PDE_ADVECTION, adv=adv, max_picard=2,
+                   dialect="cerk" if form == "cerk" else None)
     for c in (0, 1300):
         want = orc.fused(luh[c].ravel().copy(), [0.1] * 3, 1e-3)
         for key, ref in (("lduh", "lduh"), ("qb", "lQhbnd"), ("fb", "lFhbnd")):
