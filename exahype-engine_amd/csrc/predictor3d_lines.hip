@@ -387,13 +387,12 @@ __device__ __forceinline__ void finish_cell(R (&q)[B][LShape<B>::V], R* tl, unsi
 // wave-rounds of 60 lanes; the nine rounds go round the waves, so a round's
 // direction is wave-uniform and its strides are immediate offsets.  A line's B
 // values are read and written once (the node form before it read the three lines
-// through its node, 15 B values, and its operator rows).  The rows of dudx sum to
-// zero, so it acts on the differences to the line's first value: 35 operations and
-// rounding of the order of the line's variation.  By the mirrored halves of dudx and
-// Kxi, 30 operations, the predictor took 4.58 against 4.75 ms at 81^3, but the state
-// was further from FP64 than with the products (3.8e-8 against 3.5e-8).  Nine rounds on four
-// waves give one of them three: turn moves that one from phase to phase (1 % of the
-// one-iteration kernel at 81^3).
+// through its node, 15 B values, and its operator rows).  All B products of a row:
+// with the differences to the line's first value (the rows of dudx sum to zero) or the
+// mirrored halves of dudx and Kxi the state was further from FP64 (27^3, one step:
+// products, as the node form, 2.62e-8; differences 2.66e-8 in the same time; halves
+// 4.58 against 4.75 ms at 81^3).  Nine rounds on four waves give one of them three:
+// turn moves that one from phase to phase (1 % of the one-iteration kernel at 81^3).
 template <int B>
 __device__ __forceinline__ void contract_lines(float* f, int l, const DevTables* __restrict__ T, int turn) {
   constexpr int V = 5, NS = B * B * B, LINES = B * B * V, LANES = LINES / 3;
@@ -407,12 +406,10 @@ __device__ __forceinline__ void contract_lines(float* f, int l, const DevTables*
 #pragma unroll
     for (int n = 0; n < B; n++) a[n] = p[n * S];
 #pragma unroll
-    for (int n = 1; n < B; n++) a[n] -= a[0];
-#pragma unroll
     for (int i = 0; i < B; i++) {
-      o[i] = D[i * B + 1] * a[1];
+      o[i] = D[i * B] * a[0];
 #pragma unroll
-      for (int n = 2; n < B; n++) o[i] += D[i * B + n] * a[n];
+      for (int n = 1; n < B; n++) o[i] += D[i * B + n] * a[n];
     }
 #pragma unroll
     for (int n = 0; n < B; n++) p[n * S] = o[n];
