@@ -197,7 +197,7 @@ def run_form(E, P, n, order, steps, warmup, precision, picard, seed, modes, vari
 
 def cpu_threads():
     """(threads used, CPUs visible): the threads are the host's CPU share of one
-    GPU (16 on the GPU box), capped by what this process may run on."""
+    GPU (16), capped by what this process may run on."""
     try:
         visible = len(os.sched_getaffinity(0))
     except AttributeError:

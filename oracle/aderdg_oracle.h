@@ -3,8 +3,8 @@
  * ("generic::c") ADER-DG kernels, used ONLY as test infrastructure.
  *
  * Who may use this: the tests under tests/, __graft_entry__.smoke() and the
- * cpu_baseline leg of bench.py -- and only as the checker or the CPU
- * baseline, never as the product path.  The product (the HIP library behind
+ * cpu_baseline leg of bench.py -- and only as what results are compared
+ * with or the CPU baseline, never as the product path.  The product (the HIP library behind
  * include/exahype_amd.h) never links, loads or calls anything in oracle/.
  *
  * Every function cites the reference file:line it restates.  Paths are

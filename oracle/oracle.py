@@ -1,8 +1,8 @@
 """ctypes front end of the CPU oracle (test infrastructure only).
 
 Only tests/, ``__graft_entry__.smoke()`` and the ``cpu_baseline`` leg of
-bench.py import this module, and only as the checker / CPU baseline.  The
-operator tables come from ``tests/golden/legendre_tables.json`` -- the values
+bench.py import this module, and only as what results are compared with or
+as the CPU baseline.  The operator tables come from ``tests/golden/legendre_tables.json`` -- the values
 the reference generator printed (ExaHyPE/kernels/generated/GaussLegendreBasis.csnippet).
 """
 import ctypes
